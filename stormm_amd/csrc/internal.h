@@ -43,10 +43,11 @@ constexpr int kLdsCrdBits = 24;
 constexpr int kOriginBits = 38;
 constexpr int kMaxPlainGposBits = 38;
 constexpr int kMaxPlainFrcBits = 40;
-// Threads of an evaluation block: the default, and the largest a single-precision launch may
-// use; double-precision launches use at most kMaxEvalBlockDouble threads (their kernels need
+// Threads of an evaluation block: the default, the fewest, and the largest a single-precision
+// launch may use; double-precision launches use at most kMaxEvalBlockDouble threads (their kernels need
 // more than the 128 registers per lane that 16-wavefront blocks allow).
 constexpr int kEvalBlock = 512;
+constexpr int kMinEvalBlock = 256;
 constexpr int kMaxEvalBlock = 1024;
 constexpr int kMaxEvalBlockDouble = 512;
 // Entries of each wavefront's LDS queue of near-field Born-integral pairs.  A wave drains 64
@@ -69,7 +70,7 @@ enum TermMask : int { kTermNonbonded = 1, kTermValence = 2 };
 // Valence term kinds (VTerm.x).
 enum VKind : int { kVBond = 0, kVAngle = 1, kVDihedral = 2 };
 
-// Work-unit descriptor, 8 ints.  The unit's tile tasks are the clean off-diagonal tasks of all of
+// Work-unit descriptor, 12 ints.  The unit's tile tasks are the clean off-diagonal tasks of all of
 // its systems, then their other off-diagonal tasks, then their diagonal tasks (so that most
 // wavefronts hold four tasks of one kind: clean tiles run steps without pair masks, and
 // wavefronts given only diagonal tiles run the short rotation); its valence terms are those of
@@ -83,6 +84,10 @@ struct WuDesc {
   int term_count;    // valence terms of all systems
   int lj_table;      // 1 = systems in this unit read their stored LJ tables
   int rst_count;     // restraints of all systems
+  int clean_count;   // clean off-diagonal tile tasks of all systems
+  int bond_count;    // bonds and angles of all systems (the other terms are dihedrals)
+  int angl_count;
+  int pad;
 };
 
 // One system inside a work unit and the ranges of its topology template: the template's tile
@@ -105,7 +110,14 @@ struct WuSys {
   int lj_nt;
   int rst_first;     // the system's restraints in the synthesis restraint list
   int rst_count;
+  // Running totals over the unit's earlier systems: clean off-diagonal, other off-diagonal and
+  // diagonal tile tasks, and bonds, angles and dihedrals.
+  int clean_pre, offd_pre, diag_pre;
+  int bond_pre, angl_pre, dihe_pre;
+  int bond_par, angl_par, dihe_par;  // the template's first bond, angle and dihedral parameters
+  int pad[3];
 };
+static_assert(sizeof(WuSys) % sizeof(int4) == 0, "work-unit systems are copied 16 bytes at a time");
 
 // One 16 x 16 tile task of a template: x = first atom of the i tile | (first atom of the j tile
 // << 16), relative to the system; y = (diagonal << 8) | (ni << 12) | (nj << 20); z =
@@ -147,8 +159,7 @@ struct MMKit {
   const double2 *ljab14;     // 1:4 A, B per system table
   const double *rho;         // intrinsic radius - offset
   const double *scr;         // screening factor * rho
-  const double *pbr;         // intrinsic radius
-  const double *gb_alpha, *gb_beta, *gb_gamma;
+  double gb_alpha, gb_beta, gb_gamma;  // OBC constants of the solvent model
   long long *xcrd, *ycrd, *zcrd;
   long long *xfrc, *yfrc, *zfrc;
   // Overflow words of 95-bit coordinates (gpos_bits > 38) and forces (stored frc_bits > 40),

@@ -137,12 +137,19 @@ template <typename T> __device__ __forceinline__ void settle(T &x) {
   asm volatile("" : "+v"(x));
 }
 
-// Sum of a 64-bit integer over the 16 lanes of a row.
+// Sum of a 64-bit integer over the 16 lanes of a row, on every lane of the row (all 16 lanes must
+// be active): rotations, whose moves fold into the additions, where a shuffle goes through the
+// LDS crossbar.
+template <int K> __device__ __forceinline__ long long row_ror(long long v) {
+  const int lo = row_ror<K>(static_cast<int>(v & 0xffffffffLL));
+  const int hi = row_ror<K>(static_cast<int>(v >> 32));
+  return (static_cast<long long>(hi) << 32) | (static_cast<long long>(lo) & 0xffffffffLL);
+}
 __device__ __forceinline__ long long row_sum(long long v) {
-  v += __shfl_xor(v, 8, 16);
-  v += __shfl_xor(v, 4, 16);
-  v += __shfl_xor(v, 2, 16);
-  v += __shfl_xor(v, 1, 16);
+  v += row_ror<8>(v);
+  v += row_ror<4>(v);
+  v += row_ror<2>(v);
+  v += row_ror<1>(v);
   return v;
 }
 
@@ -260,20 +267,37 @@ template <> struct EvalBlockLimit<double> {
 };
 
 // ------------------------------------------------------------------------------------------
-// Work-unit LDS layout.
+// Work-unit LDS layout.  What the pair loops read of one atom lies together, so that a lane
+// fetches it with one address and one or two wide reads: with one array per quantity the tile
+// set-up and the near-pair passes spent a third of their vector instructions on addresses.
 // ------------------------------------------------------------------------------------------
+template <typename T> struct alignas(16) AtomPos {
+  typename Prec<T>::crd_t x, y, z;
+  T scr;                    // screened radius
+};
+template <typename T> struct alignas(2 * sizeof(T)) AtomRad {
+  T rho, irho;              // offset radius and its inverse
+};
+template <typename T> struct alignas(16) AtomNb {
+  T q, p1, p2;              // charge and Lennard-Jones parameters
+  T rad;                    // effective Born radius
+};
+struct AtomFrc {
+  long long x, y, z;        // 24 bytes: consecutive atoms' components fall in different banks
+};
+
 template <typename T> struct WuLds {
   using crd_t = typename Prec<T>::crd_t;
   int4 *tasks;              // the unit's tile tasks, placed at their systems' LDS bases
-  long long *psi, *dedr, *fx, *fy, *fz, *nrg, *org;
+  AtomPos<T> *pos;
+  AtomNb<T> *nb;
+  AtomRad<T> *rr;
+  AtomFrc *frc;
+  long long *psi, *dedr, *nrg, *org;
   double *move;             // per system: pending line move (coordinate units per direction unit)
-  T *q, *p1, *p2, *rho, *irho, *scr, *rad, *irad, *sd;
-  crd_t *cx, *cy, *cz;
+  T *irad;                  // inverse Born radius; after the pair stage the chain-rule factor
   int *gidx, *slot;
   WuSys *sys;
-  int *cpre, *opre, *dpre;  // per slot: first clean off-diagonal task, first other off-diagonal
-                            // task (counted among those), first diagonal task
-  int *vpre;                // per kind (bonds, angles, dihedrals): each slot's first term
   int *work;                // per-stage work-item counters (kStageCounters)
   T *clash_d, *clash_r;     // per-system clash distance and sigma ratio of this evaluation
   int *clash_on;            // per-system flag: damped potentials apply
@@ -282,15 +306,16 @@ template <typename T> struct WuLds {
   static __host__ __device__ size_t bytes(int maxa, int waves) {
     const size_t m = static_cast<size_t>(maxa);
     return (kMaxWuTasks * sizeof(int4)) +
-           (5 * m * sizeof(long long)) + (kMaxWuSystems * 16 * sizeof(long long)) +
-           (3 * kMaxWuSystems * sizeof(long long)) + (kMaxWuSystems * sizeof(double)) +
-           (9 * m * sizeof(T)) +
-           (3 * m * sizeof(crd_t)) + (2 * m * sizeof(int)) + (kMaxWuSystems * sizeof(WuSys)) +
-           (6 * (kMaxWuSystems + 1) * sizeof(int)) + (kStageCounters * sizeof(int)) +
-           (2 * kMaxWuSystems * sizeof(T)) + (kMaxWuSystems * sizeof(int)) +
+           (m * (sizeof(AtomPos<T>) + sizeof(AtomNb<T>) + sizeof(AtomRad<T>) + sizeof(AtomFrc))) +
+           (kMaxWuSystems * sizeof(WuSys)) + (2 * m * sizeof(long long)) +
+           (kMaxWuSystems * 16 * sizeof(long long)) + (3 * kMaxWuSystems * sizeof(long long)) +
+           (kMaxWuSystems * sizeof(double)) + (m * sizeof(T)) + (2 * kMaxWuSystems * sizeof(T)) +
+           (2 * m * sizeof(int)) + (kStageCounters * sizeof(int)) +
+           (kMaxWuSystems * sizeof(int)) +
            (static_cast<size_t>(waves) * kNearQueueStride * sizeof(unsigned));
   }
 
+  // maxa is a multiple of 16 (kTile), so every array below starts on the alignment of its type.
   __device__ WuLds(unsigned char *base, int maxa, int waves) {
     unsigned char *p = base;
     auto take = [&](size_t nbytes) {
@@ -300,35 +325,21 @@ template <typename T> struct WuLds {
     };
     const size_t m = static_cast<size_t>(maxa);
     tasks = reinterpret_cast<int4 *>(take(kMaxWuTasks * sizeof(int4)));
+    pos = reinterpret_cast<AtomPos<T> *>(take(m * sizeof(AtomPos<T>)));
+    nb = reinterpret_cast<AtomNb<T> *>(take(m * sizeof(AtomNb<T>)));
+    rr = reinterpret_cast<AtomRad<T> *>(take(m * sizeof(AtomRad<T>)));
+    frc = reinterpret_cast<AtomFrc *>(take(m * sizeof(AtomFrc)));
+    sys = reinterpret_cast<WuSys *>(take(kMaxWuSystems * sizeof(WuSys)));
     psi = reinterpret_cast<long long *>(take(m * sizeof(long long)));
     dedr = reinterpret_cast<long long *>(take(m * sizeof(long long)));
-    fx = reinterpret_cast<long long *>(take(m * sizeof(long long)));
-    fy = reinterpret_cast<long long *>(take(m * sizeof(long long)));
-    fz = reinterpret_cast<long long *>(take(m * sizeof(long long)));
     nrg = reinterpret_cast<long long *>(take(kMaxWuSystems * 16 * sizeof(long long)));
     org = reinterpret_cast<long long *>(take(3 * kMaxWuSystems * sizeof(long long)));
     move = reinterpret_cast<double *>(take(kMaxWuSystems * sizeof(double)));
-    q = reinterpret_cast<T *>(take(m * sizeof(T)));
-    p1 = reinterpret_cast<T *>(take(m * sizeof(T)));
-    p2 = reinterpret_cast<T *>(take(m * sizeof(T)));
-    rho = reinterpret_cast<T *>(take(m * sizeof(T)));
-    irho = reinterpret_cast<T *>(take(m * sizeof(T)));
-    scr = reinterpret_cast<T *>(take(m * sizeof(T)));
-    rad = reinterpret_cast<T *>(take(m * sizeof(T)));
     irad = reinterpret_cast<T *>(take(m * sizeof(T)));
-    sd = reinterpret_cast<T *>(take(m * sizeof(T)));
     clash_d = reinterpret_cast<T *>(take(kMaxWuSystems * sizeof(T)));
     clash_r = reinterpret_cast<T *>(take(kMaxWuSystems * sizeof(T)));
-    cx = reinterpret_cast<crd_t *>(take(m * sizeof(crd_t)));
-    cy = reinterpret_cast<crd_t *>(take(m * sizeof(crd_t)));
-    cz = reinterpret_cast<crd_t *>(take(m * sizeof(crd_t)));
     gidx = reinterpret_cast<int *>(take(m * sizeof(int)));
     slot = reinterpret_cast<int *>(take(m * sizeof(int)));
-    sys = reinterpret_cast<WuSys *>(take(kMaxWuSystems * sizeof(WuSys)));
-    cpre = reinterpret_cast<int *>(take((kMaxWuSystems + 1) * sizeof(int)));
-    opre = reinterpret_cast<int *>(take((kMaxWuSystems + 1) * sizeof(int)));
-    dpre = reinterpret_cast<int *>(take((kMaxWuSystems + 1) * sizeof(int)));
-    vpre = reinterpret_cast<int *>(take(3 * (kMaxWuSystems + 1) * sizeof(int)));
     work = reinterpret_cast<int *>(take(kStageCounters * sizeof(int)));
     clash_on = reinterpret_cast<int *>(take(kMaxWuSystems * sizeof(int)));
     nearq = reinterpret_cast<unsigned *>(take(static_cast<size_t>(waves) * kNearQueueStride *

@@ -1,6 +1,6 @@
 // Work-unit evaluation stages (device functions).  A work unit is one thread block holding one
 // or more whole systems in LDS.  The stages run in order, separated by block barriers:
-//   stage_load      global coordinates / parameters -> LDS, accumulators zeroed
+//   stage_load      system table, tile tasks, parameters, coordinates -> LDS, accumulators zeroed
 //   stage_psi       Born-radius integrals over 16 x 16 pair tiles (both directions per pair)
 //   stage_radii     effective Born radii, GB self energies, self part of dE/dR (per atom, FP64)
 //   stage_pairs     Coulomb + Lennard-Jones (exclusion masked) and GB pair energy / force / dE/dR
@@ -27,17 +27,18 @@ template <typename T> struct StageCtx {
   int cycle;         // minimization cycle of this evaluation (clash-damping schedule)
   int rst_step;      // restraint step number when the kit gives no per-system cycle counts
   bool gb;
-  bool move_pending = false;  // the coordinate stage adds L.move[slot] x direction first
+  bool move_pending = false;  // stage_load adds L.move[slot] x direction first
   __device__ StageCtx(unsigned char *smem, int maxa, int waves) : L(smem, maxa, waves) {}
 };
 
-// Slot s of the unit's system that holds item t, given ascending per-slot starts pre[0..n]
-// (pre[0] = 0 <= t < pre[n]): the s with pre[s] <= t < pre[s + 1].
-__device__ __forceinline__ int find_slot(const int *pre, int n, int t) {
+// Slot of the unit's system that holds item t, given the running total F of each system's items
+// over the earlier systems: the last system whose total does not exceed t.
+template <int WuSys::*F>
+__device__ __forceinline__ int find_slot(const WuSys *sys, int n, int t) {
   int lo = 0, hi = n;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (pre[mid] <= t) {
+    if (sys[mid].*F <= t) {
       lo = mid;
     }
     else {
@@ -47,152 +48,36 @@ __device__ __forceinline__ int find_slot(const int *pre, int n, int t) {
   return lo;
 }
 
-// ------------------------------------------------------------------------------------------
-// Work-unit set-up: system table, per-atom parameters, and the coordinate origins.
-template <typename T>
-__device__ __forceinline__ void stage_load_params(StageCtx<T> &c, const MMKit &k) {
-  WuLds<T> &L = c.L;
-  const WuDesc &wu = c.wu;
-  if (c.tid < wu.sys_count) {
-    L.sys[c.tid] = k.wu_sys[wu.sys_first + c.tid];
-  }
-  __syncthreads();
-  if (c.tid == 0) {
-    // Valence terms are taken kind by kind (all bonds of the unit, then all angles, then all
-    // dihedrals), so that a chunk of 64 runs one kind's code.
-    constexpr int K1 = kMaxWuSystems + 1;
-    int cl = 0, o = 0, d = 0, vb = 0, va = 0, vd = 0;
-    for (int s = 0; s < wu.sys_count; s++) {
-      const WuSys &ws = L.sys[s];
-      L.cpre[s] = cl;
-      L.opre[s] = o;
-      L.dpre[s] = d;
-      L.vpre[s] = vb;
-      L.vpre[K1 + s] = va;
-      L.vpre[2 * K1 + s] = vd;
-      cl += ws.clean_count;
-      o += ws.offd_count - ws.clean_count;
-      d += ws.diag_count;
-      vb += ws.bond_count;
-      va += ws.angl_count;
-      vd += ws.term_count - ws.bond_count - ws.angl_count;
-    }
-    L.cpre[wu.sys_count] = cl;
-    L.opre[wu.sys_count] = o;
-    L.dpre[wu.sys_count] = d;
-    L.vpre[wu.sys_count] = vb;
-    L.vpre[K1 + wu.sys_count] = va;
-    L.vpre[2 * K1 + wu.sys_count] = vd;
-  }
-  __syncthreads();
-  // The unit's tile tasks, read once per evaluation: the clean off-diagonal tasks of every
-  // system, then their other off-diagonal tasks, then the diagonal ones, each with its system's
-  // LDS base added and its slot in the low bits of y.
-  const int nclean = L.cpre[wu.sys_count];
-  for (int t = c.tid; t < wu.task_count; t += c.nthr) {
-    int s, idx;
-    if (t < nclean) {
-      s = find_slot(L.cpre, wu.sys_count, t);
-      idx = L.sys[s].task_first + (t - L.cpre[s]);
-    }
-    else if (t < wu.offd_count) {
-      const int to = t - nclean;
-      s = find_slot(L.opre, wu.sys_count, to);
-      idx = L.sys[s].task_first + L.sys[s].clean_count + (to - L.opre[s]);
-    }
-    else {
-      const int td = t - wu.offd_count;
-      s = find_slot(L.dpre, wu.sys_count, td);
-      idx = L.sys[s].task_first + L.sys[s].offd_count + (td - L.dpre[s]);
-    }
-    int4 tk = k.tasks[idx];
-    const int base = L.sys[s].lds_base;
-    tk.x += base | (base << 16);
-    tk.y |= s;
-    L.tasks[t] = tk;
-  }
-  for (int a = c.tid; a < wu.lds_atoms; a += c.nthr) {
-    int s = 0;
-    for (int t = 1; t < wu.sys_count; t++) {
-      s = (a >= L.sys[t].lds_base) ? t : s;
-    }
-    const WuSys ws = L.sys[s];
-    const int local = a - ws.lds_base;
-    const bool valid = local < ws.natom;
-    const int g = ws.global_start + local;
-    L.gidx[a] = valid ? g : -1;
-    L.slot[a] = s;
-    if (valid) {
-      L.q[a] = static_cast<T>(k.q[g]);
-      if (c.wu.lj_table) {
-        L.p1[a] = static_cast<T>(k.lj_type[g]);
-        L.p2[a] = T(0);
-      }
-      else {
-        L.p1[a] = static_cast<T>(0.5 * k.ljp1[g]);  // half sigma: sigma_ij = p1_i + p1_j
-        L.p2[a] = static_cast<T>(k.ljp2[g]);
-      }
-      const double rho = k.rho[g];
-      L.rho[a] = static_cast<T>(rho);
-      L.irho[a] = (rho > 0.0) ? static_cast<T>(1.0 / rho) : T(0);
-      L.scr[a] = static_cast<T>(k.scr[g]);
-    }
-    else {
-      L.q[a] = T(0);
-      L.p1[a] = T(0);
-      L.p2[a] = T(0);
-      L.rho[a] = T(1);
-      L.irho[a] = T(1);
-      L.scr[a] = T(0);
-    }
-  }
-  __syncthreads();
-}
-
 template <typename T>
 __device__ __forceinline__ bool clash_params(const MMKit &k, int sys_index, int cycle, T &d,
                                              T &r);
 
-// Coordinates into LDS (relative to a per-system origin) and all accumulators zeroed.
+// A coordinate after the pending line move mf (0: none), x += rint(mf * direction) with the
+// normalized direction in the force arrays (line_movement.cui:343-360).
+__device__ __forceinline__ long long moved(const long long *crd, const long long *dir, int g,
+                                           double mf) {
+  const long long x = crd[g];
+  return (mf != 0.0) ? x + static_cast<long long>(__builtin_rint(mf *
+                                                                 static_cast<double>(dir[g])))
+                     : x;
+}
+
+// Work-unit set-up: system table, tile tasks, per-atom parameters, coordinates relative to a
+// per-system origin (its first atom's position, with the bits below the LDS resolution cleared),
+// and all accumulators zeroed.  Every thread takes its system's origin from the first atom
+// itself, so that after the system table the tasks, parameters and coordinates all arrive in one
+// round trip to memory: the set-up is latency, 4 us of a block's time with a barrier and a round
+// trip for each of them.
 template <typename T, bool CLASH>
-__device__ void stage_load_coords(StageCtx<T> &c, const MMKit &k) {
+__device__ __forceinline__ void stage_load(StageCtx<T> &c, const MMKit &k) {
   WuLds<T> &L = c.L;
   const WuDesc &wu = c.wu;
-  if (c.tid < wu.sys_count) {
-    if (CLASH) {
-      T d, r;
-      const bool on = clash_params<T>(k, L.sys[c.tid].sys_index, c.cycle, d, r);
-      L.clash_d[c.tid] = on ? d : T(0);
-      L.clash_r[c.tid] = on ? r : T(0);
-      L.clash_on[c.tid] = on ? 1 : 0;
-    }
-    const int gs = L.sys[c.tid].global_start;
-    if (k.xcrd_ovrf != nullptr) {
-      // 95-bit coordinates: the first atom's value with the bits below the LDS resolution
-      // cleared, kept in units of 2^-(gpos_bits - org_shift) A.
-      const long long *crd[3] = {k.xcrd, k.ycrd, k.zcrd};
-      const int *ovr[3] = {k.xcrd_ovrf, k.ycrd_ovrf, k.zcrd_ovrf};
-      for (int d = 0; d < 3; d++) {
-        const __int128 v = (i95_value(crd[d][gs], ovr[d][gs]) >> c.crd_shift) << c.crd_shift;
-        L.org[3 * c.tid + d] = static_cast<long long>(v >> c.org_shift);
-      }
-    }
-    else {
-      const long long mask = ~((1LL << c.crd_shift) - 1LL);
-      long long x0 = k.xcrd[gs], y0 = k.ycrd[gs], z0 = k.zcrd[gs];
-      if (c.move_pending) {
-        // The origin comes from the moved first atom, as it would after a separate move.  This
-        // thread wrote the system's move factor itself before the stage began.
-        const double mf = L.move[c.tid];
-        if (mf != 0.0) {
-          x0 += static_cast<long long>(__builtin_rint(mf * static_cast<double>(k.xfrc[gs])));
-          y0 += static_cast<long long>(__builtin_rint(mf * static_cast<double>(k.yfrc[gs])));
-          z0 += static_cast<long long>(__builtin_rint(mf * static_cast<double>(k.zfrc[gs])));
-        }
-      }
-      L.org[3 * c.tid + 0] = x0 & mask;
-      L.org[3 * c.tid + 1] = y0 & mask;
-      L.org[3 * c.tid + 2] = z0 & mask;
+  {
+    constexpr int kWords = sizeof(WuSys) / sizeof(int4);
+    const int4 *src = reinterpret_cast<const int4 *>(k.wu_sys + wu.sys_first);
+    int4 *dst = reinterpret_cast<int4 *>(L.sys);
+    for (int e = c.tid; e < wu.sys_count * kWords; e += c.nthr) {
+      dst[e] = src[e];
     }
   }
   for (int e = c.tid; e < wu.sys_count * 16; e += c.nthr) {
@@ -202,69 +87,146 @@ __device__ void stage_load_coords(StageCtx<T> &c, const MMKit &k) {
     L.work[c.tid] = 0;
   }
   __syncthreads();
-  for (int a = c.tid; a < wu.lds_atoms; a += c.nthr) {
-    const int g = L.gidx[a];
-    const int s = L.slot[a];
+  if (CLASH && c.tid < wu.sys_count) {
+    T d, r;
+    const bool on = clash_params<T>(k, L.sys[c.tid].sys_index, c.cycle, d, r);
+    L.clash_d[c.tid] = on ? d : T(0);
+    L.clash_r[c.tid] = on ? r : T(0);
+    L.clash_on[c.tid] = on ? 1 : 0;
+  }
+  // A thread's atoms (at most two: blocks hold at least 256 threads), their moved coordinates
+  // kept until every thread has read the unmoved ones.
+  constexpr int kPer = kMaxWuAtoms / kMinEvalBlock;
+  long long at[kPer][3];
+  int owned[kPer];
+#pragma unroll
+  for (int it = 0; it < kPer; it++) {
+    const int a = c.tid + (it * c.nthr);
+    owned[it] = -1;
+    if (a >= wu.lds_atoms) {
+      continue;
+    }
+    const int s = find_slot<&WuSys::lds_base>(L.sys, wu.sys_count, a);
+    const int gs = L.sys[s].global_start;
+    const int local = a - L.sys[s].lds_base;
+    const bool valid = local < L.sys[s].natom;
+    const int g = gs + local;
+    L.gidx[a] = valid ? g : -1;
+    L.slot[a] = s;
     L.psi[a] = 0;
     L.dedr[a] = 0;
-    L.fx[a] = 0;
-    L.fy[a] = 0;
-    L.fz[a] = 0;
-    L.rad[a] = T(1);
+    L.frc[a] = {0, 0, 0};
     L.irad[a] = T(1);
-    L.sd[a] = T(0);
-    if (g >= 0 && k.xcrd_ovrf != nullptr) {
-      const __int128 dx = i95_value(k.xcrd[g], k.xcrd_ovrf[g]) -
-                          (static_cast<__int128>(L.org[3 * s]) << c.org_shift);
-      const __int128 dy = i95_value(k.ycrd[g], k.ycrd_ovrf[g]) -
-                          (static_cast<__int128>(L.org[3 * s + 1]) << c.org_shift);
-      const __int128 dz = i95_value(k.zcrd[g], k.zcrd_ovrf[g]) -
-                          (static_cast<__int128>(L.org[3 * s + 2]) << c.org_shift);
-      if (!(CrdConv<T>::in_range_wide(dx, c.crd_shift) &&
-            CrdConv<T>::in_range_wide(dy, c.crd_shift) &&
-            CrdConv<T>::in_range_wide(dz, c.crd_shift))) {
-        atomicOr(k.status, static_cast<int>(kStatusCoordinateRange));
+    AtomPos<T> pos = {0, 0, 0, T(0)};
+    AtomNb<T> nb = {T(0), T(0), T(0), T(1)};
+    AtomRad<T> rr = {T(1), T(1)};
+    if (valid) {
+      nb.q = static_cast<T>(k.q[g]);
+      if (wu.lj_table) {
+        nb.p1 = static_cast<T>(k.lj_type[g]);
       }
-      L.cx[a] = CrdConv<T>::to_lds_wide(dx, c.crd_shift);
-      L.cy[a] = CrdConv<T>::to_lds_wide(dy, c.crd_shift);
-      L.cz[a] = CrdConv<T>::to_lds_wide(dz, c.crd_shift);
-    }
-    else if (g >= 0) {
-      long long gx = k.xcrd[g], gy = k.ycrd[g], gz = k.zcrd[g];
-      if (c.move_pending) {
-        // The pending line move, x += rint(mf * direction) with the normalized direction in the
-        // force arrays (line_movement.cui:343-360), written back as the new coordinates.
-        const double mf = L.move[s];
-        if (mf != 0.0) {
-          gx += static_cast<long long>(__builtin_rint(mf * static_cast<double>(k.xfrc[g])));
-          gy += static_cast<long long>(__builtin_rint(mf * static_cast<double>(k.yfrc[g])));
-          gz += static_cast<long long>(__builtin_rint(mf * static_cast<double>(k.zfrc[g])));
-          k.xcrd[g] = gx;
-          k.ycrd[g] = gy;
-          k.zcrd[g] = gz;
+      else {
+        nb.p1 = static_cast<T>(0.5 * k.ljp1[g]);  // half sigma: sigma_ij = p1_i + p1_j
+        nb.p2 = static_cast<T>(k.ljp2[g]);
+      }
+      const double rho = k.rho[g];
+      rr.rho = static_cast<T>(rho);
+      rr.irho = (rho > 0.0) ? static_cast<T>(Prec<double>::rcp(rho)) : T(0);
+      pos.scr = static_cast<T>(k.scr[g]);
+      bool ok;
+      if (k.xcrd_ovrf != nullptr) {
+        // 95-bit coordinates: origins kept in units of 2^-(gpos_bits - org_shift) A.
+        auto wide = [&](const long long *crd, const int *ovr, int d) {
+          const __int128 v = (i95_value(crd[gs], ovr[gs]) >> c.crd_shift) << c.crd_shift;
+          const long long o = static_cast<long long>(v >> c.org_shift);
+          if (local == 0) {
+            L.org[3 * s + d] = o;
+          }
+          return i95_value(crd[g], ovr[g]) - (static_cast<__int128>(o) << c.org_shift);
+        };
+        const __int128 dx = wide(k.xcrd, k.xcrd_ovrf, 0);
+        const __int128 dy = wide(k.ycrd, k.ycrd_ovrf, 1);
+        const __int128 dz = wide(k.zcrd, k.zcrd_ovrf, 2);
+        ok = CrdConv<T>::in_range_wide(dx, c.crd_shift) &&
+             CrdConv<T>::in_range_wide(dy, c.crd_shift) &&
+             CrdConv<T>::in_range_wide(dz, c.crd_shift);
+        pos.x = CrdConv<T>::to_lds_wide(dx, c.crd_shift);
+        pos.y = CrdConv<T>::to_lds_wide(dy, c.crd_shift);
+        pos.z = CrdConv<T>::to_lds_wide(dz, c.crd_shift);
+      }
+      else {
+        const double mf = c.move_pending ? L.move[s] : 0.0;
+        const long long mask = ~((1LL << c.crd_shift) - 1LL);
+        const long long gx = moved(k.xcrd, k.xfrc, g, mf);
+        const long long gy = moved(k.ycrd, k.yfrc, g, mf);
+        const long long gz = moved(k.zcrd, k.zfrc, g, mf);
+        const long long ox = moved(k.xcrd, k.xfrc, gs, mf) & mask;
+        const long long oy = moved(k.ycrd, k.yfrc, gs, mf) & mask;
+        const long long oz = moved(k.zcrd, k.zfrc, gs, mf) & mask;
+        if (local == 0) {
+          L.org[3 * s + 0] = ox;
+          L.org[3 * s + 1] = oy;
+          L.org[3 * s + 2] = oz;
         }
+        if (mf != 0.0) {
+          owned[it] = g;
+          at[it][0] = gx;
+          at[it][1] = gy;
+          at[it][2] = gz;
+        }
+        ok = CrdConv<T>::in_range(gx, ox, c.crd_shift) &&
+             CrdConv<T>::in_range(gy, oy, c.crd_shift) &&
+             CrdConv<T>::in_range(gz, oz, c.crd_shift);
+        pos.x = CrdConv<T>::to_lds(gx, ox, c.crd_shift);
+        pos.y = CrdConv<T>::to_lds(gy, oy, c.crd_shift);
+        pos.z = CrdConv<T>::to_lds(gz, oz, c.crd_shift);
       }
-      const long long ox = L.org[3 * s], oy = L.org[3 * s + 1], oz = L.org[3 * s + 2];
-      if (!(CrdConv<T>::in_range(gx, ox, c.crd_shift) &&
-            CrdConv<T>::in_range(gy, oy, c.crd_shift) &&
-            CrdConv<T>::in_range(gz, oz, c.crd_shift))) {
+      if (!ok) {
         atomicOr(k.status, static_cast<int>(kStatusCoordinateRange));
       }
-      L.cx[a] = CrdConv<T>::to_lds(gx, ox, c.crd_shift);
-      L.cy[a] = CrdConv<T>::to_lds(gy, oy, c.crd_shift);
-      L.cz[a] = CrdConv<T>::to_lds(gz, oz, c.crd_shift);
+    }
+    L.pos[a] = pos;
+    L.nb[a] = nb;
+    L.rr[a] = rr;
+  }
+  // The unit's tile tasks, read once per evaluation: the clean off-diagonal tasks of every
+  // system, then their other off-diagonal tasks, then the diagonal ones, each with its system's
+  // LDS base added and its slot in the low bits of y.
+  for (int t = c.tid; t < wu.task_count; t += c.nthr) {
+    int s, idx;
+    if (t < wu.clean_count) {
+      s = find_slot<&WuSys::clean_pre>(L.sys, wu.sys_count, t);
+      idx = L.sys[s].task_first + (t - L.sys[s].clean_pre);
+    }
+    else if (t < wu.offd_count) {
+      const int to = t - wu.clean_count;
+      s = find_slot<&WuSys::offd_pre>(L.sys, wu.sys_count, to);
+      idx = L.sys[s].task_first + L.sys[s].clean_count + (to - L.sys[s].offd_pre);
     }
     else {
-      L.cx[a] = 0;
-      L.cy[a] = 0;
-      L.cz[a] = 0;
+      const int td = t - wu.offd_count;
+      s = find_slot<&WuSys::diag_pre>(L.sys, wu.sys_count, td);
+      idx = L.sys[s].task_first + L.sys[s].offd_count + (td - L.sys[s].diag_pre);
     }
+    int4 tk = k.tasks[idx];
+    const int base = L.sys[s].lds_base;
+    tk.x += base | (base << 16);
+    tk.y |= s;
+    L.tasks[t] = tk;
   }
   __syncthreads();
+#pragma unroll
+  for (int it = 0; it < kPer; it++) {
+    if (owned[it] >= 0) {
+      k.xcrd[owned[it]] = at[it][0];
+      k.ycrd[owned[it]] = at[it][1];
+      k.zcrd[owned[it]] = at[it][2];
+    }
+  }
 }
 
 template <typename T>
-__device__ void init_ctx(StageCtx<T> &c, const MMKit &k, int wu_index, int terms) {
+__device__ __forceinline__ void init_ctx(StageCtx<T> &c, const MMKit &k, int wu_index, int terms) {
   c.wu = k.wu[wu_index];
   c.tid = threadIdx.x;
   c.nthr = blockDim.x;
@@ -363,24 +325,27 @@ struct TileTask {
   }
 };
 
-// Coordinates of lane il's i atom and first j atom of a tile, in Angstroms.  The padding slots
-// of a partial tile (lanes past ni on the i side, past nj on the j side) are put far away, so
-// that their pairs are far-field pairs with terms of exactly zero in the Born-integral and
-// derivative loops, which need no pair mask on off-diagonal tiles.
+// Coordinates (Angstroms) and screened radii of lane il's i atom and first j atom of a tile.  The
+// padding slots of a partial tile (lanes past ni on the i side, past nj on the j side) are put far
+// away, so that their pairs are far-field pairs with terms of exactly zero in the Born-integral
+// and derivative loops, which need no pair mask on off-diagonal tiles.
 template <typename T>
 __device__ __forceinline__ void tile_coords(const StageCtx<T> &c, const TileTask &tt, T &xi,
-                                            T &yi, T &zi, T &xj, T &yj, T &zj) {
-  const WuLds<T> &L = c.L;
-  const auto ox = tile_centre(L.cx[tt.ib], L.cx[tt.jb]);
-  const auto oy = tile_centre(L.cy[tt.ib], L.cy[tt.jb]);
-  const auto oz = tile_centre(L.cz[tt.ib], L.cz[tt.jb]);
+                                            T &yi, T &zi, T &xj, T &yj, T &zj, T &si, T &sj) {
+  const AtomPos<T> *pos = c.L.pos;
+  const AtomPos<T> bi = pos[tt.ib], bj = pos[tt.jb], pi = pos[tt.i], pj = pos[tt.j0];
+  const auto ox = tile_centre(bi.x, bj.x);
+  const auto oy = tile_centre(bi.y, bj.y);
+  const auto oz = tile_centre(bi.z, bj.z);
   const bool jvalid = tt.jl0 < tt.nj;
-  xi = tt.ivalid ? tile_crd(L.cx[tt.i], ox, c.crd_scale) : FarAway<T>::kCrd;
-  yi = tt.ivalid ? tile_crd(L.cy[tt.i], oy, c.crd_scale) : FarAway<T>::kCrd;
-  zi = tt.ivalid ? tile_crd(L.cz[tt.i], oz, c.crd_scale) : FarAway<T>::kCrd;
-  xj = jvalid ? tile_crd(L.cx[tt.j0], ox, c.crd_scale) : -FarAway<T>::kCrd;
-  yj = jvalid ? tile_crd(L.cy[tt.j0], oy, c.crd_scale) : -FarAway<T>::kCrd;
-  zj = jvalid ? tile_crd(L.cz[tt.j0], oz, c.crd_scale) : -FarAway<T>::kCrd;
+  xi = tt.ivalid ? tile_crd(pi.x, ox, c.crd_scale) : FarAway<T>::kCrd;
+  yi = tt.ivalid ? tile_crd(pi.y, oy, c.crd_scale) : FarAway<T>::kCrd;
+  zi = tt.ivalid ? tile_crd(pi.z, oz, c.crd_scale) : FarAway<T>::kCrd;
+  xj = jvalid ? tile_crd(pj.x, ox, c.crd_scale) : -FarAway<T>::kCrd;
+  yj = jvalid ? tile_crd(pj.y, oy, c.crd_scale) : -FarAway<T>::kCrd;
+  zj = jvalid ? tile_crd(pj.z, oz, c.crd_scale) : -FarAway<T>::kCrd;
+  si = pi.scr;
+  sj = pj.scr;
 }
 
 // True on every lane when `b` holds on every active lane of the wavefront.
@@ -395,7 +360,7 @@ __device__ __forceinline__ bool step_bit(unsigned mask, int ks) {
 // ------------------------------------------------------------------------------------------
 
 // Tile task t of the work unit, placed at its system's LDS base and tagged with its slot
-// (staged in LDS by stage_load_params).
+// (staged in LDS by stage_load).
 template <typename T>
 __device__ __forceinline__ Task fetch_task(const StageCtx<T> &c, const MMKit &, int t) {
   return c.L.tasks[t];
@@ -439,25 +404,22 @@ __device__ __forceinline__ int stage_item(int i, int quads, int chunks) {
 }
 
 template <typename T, bool FORCES, bool CLASH>
-__device__ void valence_term(StageCtx<T> &c, const MMKit &k, int kind, int t);
+__device__ __forceinline__ void valence_term(StageCtx<T> &c, const MMKit &k, int kind, int t);
 
 // Chunks of 64 valence terms of the unit: its bonds, then its angles, then its dihedrals, each
 // kind starting a chunk of its own.
 template <typename T> __device__ __forceinline__ int valence_chunks(const StageCtx<T> &c) {
-  constexpr int K1 = kMaxWuSystems + 1;
-  const int n = c.wu.sys_count;
-  return ((c.L.vpre[n] + 63) >> 6) + ((c.L.vpre[K1 + n] + 63) >> 6) +
-         ((c.L.vpre[2 * K1 + n] + 63) >> 6);
+  const WuDesc &wu = c.wu;
+  return ((wu.bond_count + 63) >> 6) + ((wu.angl_count + 63) >> 6) +
+         ((wu.term_count - wu.bond_count - wu.angl_count + 63) >> 6);
 }
 
 // Valence chunk `chunk` (wavefront-uniform), one term per lane.
 template <typename T, bool FORCES, bool CLASH>
 __device__ __forceinline__ void valence_chunk(StageCtx<T> &c, const MMKit &k, int chunk,
                                               int lane) {
-  constexpr int K1 = kMaxWuSystems + 1;
-  const int n = c.wu.sys_count;
-  const int cb = (c.L.vpre[n] + 63) >> 6;
-  const int ca = (c.L.vpre[K1 + n] + 63) >> 6;
+  const int cb = (c.wu.bond_count + 63) >> 6;
+  const int ca = (c.wu.angl_count + 63) >> 6;
   const int kind = (chunk < cb) ? kVBond : (chunk < cb + ca) ? kVAngle : kVDihedral;
   const int local = chunk - ((kind == kVBond) ? 0 : (kind == kVAngle) ? cb : cb + ca);
   valence_term<T, FORCES, CLASH>(c, k, kind, (local << 6) + lane);
@@ -510,16 +472,19 @@ static_assert(63 + ((kStepGroup - 1) * 64) + 64 <= kNearQueue,
 template <typename T> struct NearPair {
   int i, j;
   bool near_i, near_j;
-  T dx, dy, dz, r2, invr, r;
+  T dx, dy, dz, r2, invr, r, si, sj;
   __device__ __forceinline__ NearPair(const StageCtx<T> &c, unsigned e) {
     using P = Prec<T>;
     i = static_cast<int>(e & 0x1ffu);
     j = static_cast<int>((e >> 9) & 0x1ffu);
     near_i = (e & kNearI) != 0u;
     near_j = (e & kNearJ) != 0u;
-    dx = crd_delta(c.L.cx[j], c.L.cx[i], c.crd_scale);
-    dy = crd_delta(c.L.cy[j], c.L.cy[i], c.crd_scale);
-    dz = crd_delta(c.L.cz[j], c.L.cz[i], c.crd_scale);
+    const AtomPos<T> pi = c.L.pos[i], pj = c.L.pos[j];
+    dx = crd_delta(pj.x, pi.x, c.crd_scale);
+    dy = crd_delta(pj.y, pi.y, c.crd_scale);
+    dz = crd_delta(pj.z, pi.z, c.crd_scale);
+    si = pi.scr;
+    sj = pj.scr;
     r2 = (dx * dx) + (dy * dy) + (dz * dz);
     invr = P::rsqrt(r2);
     r = r2 * invr;
@@ -533,12 +498,13 @@ __device__ __forceinline__ void psi_drain(StageCtx<T> &c, const unsigned *q, int
   WuLds<T> &L = c.L;
   if (lane < count) {
     const NearPair<T> p(c, q[lane]);
+    const AtomRad<T> ri = L.rr[p.i], rj = L.rr[p.j];
     if (p.near_i) {
-      const T t = psi_near(p.r, p.r2, p.invr, L.rho[p.i], L.irho[p.i], L.scr[p.j]);
+      const T t = psi_near(p.r, p.r2, p.invr, ri.rho, ri.irho, p.sj);
       lds_add(&L.psi[p.i], fixed_contrib(t, kPsiBits));
     }
     if (p.near_j) {
-      const T t = psi_near(p.r, p.r2, p.invr, L.rho[p.j], L.irho[p.j], L.scr[p.i]);
+      const T t = psi_near(p.r, p.r2, p.invr, rj.rho, rj.irho, p.si);
       lds_add(&L.psi[p.j], fixed_contrib(t, kPsiBits));
     }
   }
@@ -553,7 +519,7 @@ __device__ __forceinline__ void psi_drain(StageCtx<T> &c, const unsigned *q, int
 // series in x, and r > 4 s is x < 1/16.
 // Chunks of valence terms (`val_chunks`, possibly 0) are taken as work items alongside the tiles.
 template <typename T, bool FORCES, bool CLASH>
-__device__ void stage_psi(StageCtx<T> &c, const MMKit &k, int val_chunks) {
+__device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int val_chunks) {
   using P = Prec<T>;
   WuLds<T> &L = c.L;
   const int il = c.tid & 15;
@@ -573,12 +539,10 @@ __device__ void stage_psi(StageCtx<T> &c, const MMKit &k, int val_chunks) {
       continue;
     }
     const TileTask tt(wave_task(c, k, ((-1 - it) << 2) + ((c.tid >> 4) & 3)), il);
-    T xi, yi, zi, xj, yj, zj;
-    tile_coords(c, tt, xi, yi, zi, xj, yj, zj);
-    const T si = L.scr[tt.i];
+    T xi, yi, zi, xj, yj, zj, si, sj;
+    tile_coords(c, tt, xi, yi, zi, xj, yj, zj, si, sj);
     const T si2 = si * si;
     const T si3 = si2 * si;
-    const T sj = L.scr[tt.j0];
     T sj2 = sj * sj;
     T sj3 = sj2 * sj;
     // Queue entry bits of the pair: i in bits 0..8, the j atom in bits 9..17.
@@ -660,7 +624,7 @@ __device__ void stage_psi(StageCtx<T> &c, const MMKit &k, int val_chunks) {
 // Effective radii (src/Potential/nonbonded_potential.tpp:731-781), self energies and the self
 // part of the radius derivative accumulator (:784-806), all in double precision.
 template <typename T, bool FORCES>
-__device__ void stage_radii(StageCtx<T> &c, const MMKit &k, double coulomb_inv_scaled) {
+__device__ __forceinline__ void stage_radii(StageCtx<T> &c, const MMKit &k, double coulomb_inv_scaled) {
   WuLds<T> &L = c.L;
   const double nrg_scale = ldexp(1.0, k.nrg_bits);
   const double inv_diel = 1.0 / k.dielectric;
@@ -671,7 +635,6 @@ __device__ void stage_radii(StageCtx<T> &c, const MMKit &k, double coulomb_inv_s
     }
     const double psi = static_cast<double>(L.psi[a]) * ldexp(1.0, -kPsiBits);
     const double rho = k.rho[g];
-    const double pbr = k.pbr[g];
     double R;
     if (k.igb == 1) {
       R = 1.0 / ((1.0 / rho) + psi);
@@ -679,7 +642,8 @@ __device__ void stage_radii(StageCtx<T> &c, const MMKit &k, double coulomb_inv_s
     }
     else {
       const double fipsi = psi * (-rho);
-      const double al = k.gb_alpha[g], be = k.gb_beta[g], ga = k.gb_gamma[g];
+      const double al = k.gb_alpha, be = k.gb_beta, ga = k.gb_gamma;
+      const double pbr = rho + kGbOffset;  // intrinsic radius
       const double thi = tanh((al - (be * fipsi) + (ga * fipsi * fipsi)) * fipsi);
       R = 1.0 / ((1.0 / rho) - thi / pbr);
       if (FORCES) {
@@ -690,7 +654,7 @@ __device__ void stage_radii(StageCtx<T> &c, const MMKit &k, double coulomb_inv_s
         L.psi[a] = __double_as_longlong(dr_dpsi);
       }
     }
-    L.rad[a] = static_cast<T>(R);
+    L.nb[a].rad = static_cast<T>(R);
     L.irad[a] = static_cast<T>(1.0 / R);
     // q holds charge * sqrt(Coulomb), so q^2 = Coulomb * charge^2.
     const double qg = k.q[g];
@@ -773,7 +737,7 @@ __device__ __forceinline__ void clash_pair(T r, T qq, T lja, T ljb, T sigma, T c
 // one lane per step.  The radius-derivative sums hold dE/dR / R and are scaled
 // by the atom's radius at the end.
 template <typename T, bool FORCES, bool LJTABLE, bool GB, bool CLASH>
-__device__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
+__device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
   using P = Prec<T>;
   WuLds<T> &L = c.L;
   const int row = c.tid >> 4;
@@ -791,10 +755,11 @@ __device__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
     const TileTask tt(tk, il);
     const unsigned emask = (tk.z >= 0 && tt.ivalid) ? k.masks[tk.z + il] : 0u;
     const unsigned nbmask = tt.valid & ~step_mask(emask, tt.jl0);
-    T xi, yi, zi, xj, yj, zj;
-    tile_coords(c, tt, xi, yi, zi, xj, yj, zj);
-    const T qi = L.q[tt.i], p1i = L.p1[tt.i], p2i = L.p2[tt.i], Ri = L.rad[tt.i];
-    T qj = L.q[tt.j0], p1j = L.p1[tt.j0], p2j = L.p2[tt.j0], Rj = L.rad[tt.j0];
+    T xi, yi, zi, xj, yj, zj, si, sj;
+    tile_coords(c, tt, xi, yi, zi, xj, yj, zj, si, sj);
+    const AtomNb<T> ni = L.nb[tt.i], nj = L.nb[tt.j0];
+    const T qi = ni.q, p1i = ni.p1, p2i = ni.p2, Ri = ni.rad;
+    T qj = nj.q, p1j = nj.p1, p2j = nj.p2, Rj = nj.rad;
     // exp(-r^2 / (4 Ri Rj)) = GbExp(r^2 * (1 / Rj) * (scale / Ri)).
     T iRj = GB ? L.irad[tt.j0] : T(0);
     const T iRi = GB ? L.irad[tt.i] * GbExp<T>::kScale : T(0);
@@ -972,9 +937,9 @@ __device__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
     }
     if (FORCES) {
       if (tt.ivalid) {
-        lds_add(&L.fx[tt.i], P::fixed(fxi * frc_scale));
-        lds_add(&L.fy[tt.i], P::fixed(fyi * frc_scale));
-        lds_add(&L.fz[tt.i], P::fixed(fzi * frc_scale));
+        lds_add(&L.frc[tt.i].x, P::fixed(fxi * frc_scale));
+        lds_add(&L.frc[tt.i].y, P::fixed(fyi * frc_scale));
+        lds_add(&L.frc[tt.i].z, P::fixed(fzi * frc_scale));
         if (GB) {
           lds_add(&L.dedr[tt.i], P::fixed(Ri * dri * dedr_scale));
         }
@@ -983,11 +948,11 @@ __device__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
       const int jl_home = tt.jl_home();
       if (jl_home < tt.nj) {
         const int j = tt.jb + jl_home;
-        lds_add(&L.fx[j], P::fixed(fxj * frc_scale));
-        lds_add(&L.fy[j], P::fixed(fyj * frc_scale));
-        lds_add(&L.fz[j], P::fixed(fzj * frc_scale));
+        lds_add(&L.frc[j].x, P::fixed(fxj * frc_scale));
+        lds_add(&L.frc[j].y, P::fixed(fyj * frc_scale));
+        lds_add(&L.frc[j].z, P::fixed(fzj * frc_scale));
         if (GB) {
-          lds_add(&L.dedr[j], P::fixed(L.rad[j] * drj * dedr_scale));
+          lds_add(&L.dedr[j], P::fixed(L.nb[j].rad * drj * dedr_scale));
         }
       }
     }
@@ -1007,14 +972,15 @@ __device__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
 
 // ------------------------------------------------------------------------------------------
 // OBC chain rule on the accumulated radius derivatives, src/Potential/nonbonded_potential.tpp:
-// 985-1017.  The HCT model uses the accumulated values as they stand.
+// 985-1017.  The HCT model uses the accumulated values as they stand.  The factors take the place
+// of the inverse radii, which the pair stage was the last to read.
 template <typename T>
-__device__ void stage_chain(StageCtx<T> &c, const MMKit &k) {
+__device__ __forceinline__ void stage_chain(StageCtx<T> &c, const MMKit &k) {
   WuLds<T> &L = c.L;
   for (int a = c.tid; a < c.wu.lds_atoms; a += c.nthr) {
     const int g = L.gidx[a];
     if (g < 0) {
-      L.sd[a] = T(0);
+      L.irad[a] = T(0);
       continue;
     }
     double sdi = static_cast<double>(L.dedr[a]) * ldexp(1.0, -kDedrBits);
@@ -1022,7 +988,7 @@ __device__ void stage_chain(StageCtx<T> &c, const MMKit &k) {
       // The radii stage left dR/dpsi in the psi slot.
       sdi *= __longlong_as_double(L.psi[a]);
     }
-    L.sd[a] = static_cast<T>(sdi);
+    L.irad[a] = static_cast<T>(sdi);
   }
   __syncthreads();
 }
@@ -1035,25 +1001,24 @@ __device__ __forceinline__ void deriv_drain(StageCtx<T> &c, const unsigned *q, i
   WuLds<T> &L = c.L;
   if (lane < count) {
     const NearPair<T> p(c, q[lane]);
+    const AtomRad<T> ri = L.rr[p.i], rj = L.rr[p.j];
     const T invr2 = p.invr * p.invr;
     T fmag = T(0);
     if (p.near_i) {
-      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, L.rho[p.i], L.irho[p.i], L.scr[p.j]) *
-              L.sd[p.i];
+      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, ri.rho, ri.irho, p.sj) * L.irad[p.i];
     }
     if (p.near_j) {
-      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, L.rho[p.j], L.irho[p.j], L.scr[p.i]) *
-              L.sd[p.j];
+      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, rj.rho, rj.irho, p.si) * L.irad[p.j];
     }
     const long long fx = fixed_contrib(fmag * p.dx, frc_bits);
     const long long fy = fixed_contrib(fmag * p.dy, frc_bits);
     const long long fz = fixed_contrib(fmag * p.dz, frc_bits);
-    lds_add(&L.fx[p.i], -fx);
-    lds_add(&L.fy[p.i], -fy);
-    lds_add(&L.fz[p.i], -fz);
-    lds_add(&L.fx[p.j], fx);
-    lds_add(&L.fy[p.j], fy);
-    lds_add(&L.fz[p.j], fz);
+    lds_add(&L.frc[p.i].x, -fx);
+    lds_add(&L.frc[p.i].y, -fy);
+    lds_add(&L.frc[p.i].z, -fz);
+    lds_add(&L.frc[p.j].x, fx);
+    lds_add(&L.frc[p.j].y, fy);
+    lds_add(&L.frc[p.j].z, fz);
   }
 }
 
@@ -1077,15 +1042,14 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
   const int quads = (c.wu.task_count + 3) >> 2;
   for (int item = next_item(&L.work[1], lane); item < quads; item = next_item(&L.work[1], lane)) {
     const TileTask tt(wave_task(c, k, (item << 2) + ((c.tid >> 4) & 3)), il);
-    T xi, yi, zi, xj, yj, zj;
-    tile_coords(c, tt, xi, yi, zi, xj, yj, zj);
-    const T si = L.scr[tt.i], sdi = L.sd[tt.i];
+    T xi, yi, zi, xj, yj, zj, si, sj;
+    tile_coords(c, tt, xi, yi, zi, xj, yj, zj, si, sj);
+    const T sdi = L.irad[tt.i];
     const T si2 = si * si;
     const T si3 = si2 * si;
-    const T sj = L.scr[tt.j0];
     T sj2 = sj * sj;
     T sj3 = sj2 * sj;
-    T sdj = L.sd[tt.j0];
+    T sdj = L.irad[tt.j0];
     const unsigned ei = static_cast<unsigned>(tt.i);
     int ej = tt.j0 << 9;
     T fxi = T(0), fyi = T(0), fzi = T(0);
@@ -1158,16 +1122,16 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
       run(std::true_type{});
     }
     if (tt.ivalid) {
-      lds_add(&L.fx[tt.i], P::fixed(fxi * frc_scale));
-      lds_add(&L.fy[tt.i], P::fixed(fyi * frc_scale));
-      lds_add(&L.fz[tt.i], P::fixed(fzi * frc_scale));
+      lds_add(&L.frc[tt.i].x, P::fixed(fxi * frc_scale));
+      lds_add(&L.frc[tt.i].y, P::fixed(fyi * frc_scale));
+      lds_add(&L.frc[tt.i].z, P::fixed(fzi * frc_scale));
     }
     const int jl_home = tt.jl_home();
     if (jl_home < tt.nj) {
       const int j = tt.jb + jl_home;
-      lds_add(&L.fx[j], P::fixed(gxj * frc_scale));
-      lds_add(&L.fy[j], P::fixed(gyj * frc_scale));
-      lds_add(&L.fz[j], P::fixed(gzj * frc_scale));
+      lds_add(&L.frc[j].x, P::fixed(gxj * frc_scale));
+      lds_add(&L.frc[j].y, P::fixed(gyj * frc_scale));
+      lds_add(&L.frc[j].z, P::fixed(gzj * frc_scale));
     }
   }
   deriv_drain(c, q, qn, lane, k.frc_bits);
@@ -1201,34 +1165,41 @@ __device__ __forceinline__ float dot(const Vec3f &a, const Vec3f &b) {
   return (a.x * b.x) + (a.y * b.y) + (a.z * b.z);
 }
 
-template <typename C> struct ValenceCtxT {
-  const C *cx, *cy, *cz;
+template <typename T> struct ValenceCtxT {
+  const AtomPos<T> *pos;
   const int *gidx;
   double crd_scale;
   float crd_scale_f;
-  long long *fx, *fy, *fz;
+  AtomFrc *frc;
+  __device__ __forceinline__ explicit ValenceCtxT(const StageCtx<T> &c)
+      : pos(c.L.pos), gidx(c.L.gidx), crd_scale(static_cast<double>(c.crd_scale)),
+        crd_scale_f(static_cast<float>(c.crd_scale)), frc(c.L.frc) {}
   // Absolute position (A) of LDS atom a of a system whose coordinate origin is org (fixed
   // precision at inv_gpos).
   __device__ __forceinline__ Vec3 absolute(int a, const long long *org, double inv_gpos) const {
-    return {(static_cast<double>(org[0]) * inv_gpos) + (static_cast<double>(cx[a]) * crd_scale),
-            (static_cast<double>(org[1]) * inv_gpos) + (static_cast<double>(cy[a]) * crd_scale),
-            (static_cast<double>(org[2]) * inv_gpos) + (static_cast<double>(cz[a]) * crd_scale)};
+    const AtomPos<T> p = pos[a];
+    return {(static_cast<double>(org[0]) * inv_gpos) + (static_cast<double>(p.x) * crd_scale),
+            (static_cast<double>(org[1]) * inv_gpos) + (static_cast<double>(p.y) * crd_scale),
+            (static_cast<double>(org[2]) * inv_gpos) + (static_cast<double>(p.z) * crd_scale)};
   }
   // Single-precision displacement: the LDS coordinates' difference is exact, then rounded once.
   __device__ __forceinline__ Vec3f dispf(int from, int to) const {
-    return {static_cast<float>(cx[to] - cx[from]) * crd_scale_f,
-            static_cast<float>(cy[to] - cy[from]) * crd_scale_f,
-            static_cast<float>(cz[to] - cz[from]) * crd_scale_f};
+    const AtomPos<T> a = pos[from], b = pos[to];
+    return {static_cast<float>(b.x - a.x) * crd_scale_f,
+            static_cast<float>(b.y - a.y) * crd_scale_f,
+            static_cast<float>(b.z - a.z) * crd_scale_f};
   }
   __device__ __forceinline__ Vec3 disp(int from, int to) const {
-    return {(static_cast<double>(cx[to]) - static_cast<double>(cx[from])) * crd_scale,
-            (static_cast<double>(cy[to]) - static_cast<double>(cy[from])) * crd_scale,
-            (static_cast<double>(cz[to]) - static_cast<double>(cz[from])) * crd_scale};
+    const AtomPos<T> a = pos[from], b = pos[to];
+    return {(static_cast<double>(b.x) - static_cast<double>(a.x)) * crd_scale,
+            (static_cast<double>(b.y) - static_cast<double>(a.y)) * crd_scale,
+            (static_cast<double>(b.z) - static_cast<double>(a.z)) * crd_scale};
   }
   __device__ __forceinline__ void add(int a, long long vx, long long vy, long long vz) const {
-    lds_add(&fx[a], vx);
-    lds_add(&fy[a], vy);
-    lds_add(&fz[a], vz);
+    AtomFrc *f = frc + a;
+    lds_add(&f->x, vx);
+    lds_add(&f->y, vy);
+    lds_add(&f->z, vz);
   }
 };
 
@@ -1588,7 +1559,7 @@ __device__ __forceinline__ double image_angle(double x) {
 
 // One restraint of the system at LDS base `base`; returns its penalty.
 template <bool FORCES, typename V>
-__device__ double eval_restraint(const V &v, const stormm_restraint &t, int base,
+__device__ __forceinline__ double eval_restraint(const V &v, const stormm_restraint &t, int base,
                                  const long long *org, double inv_gpos, int step,
                                  double fscale) {
   const double2 w = restraint_mixture(step, t.init_step, t.final_step);
@@ -1709,48 +1680,49 @@ __device__ double eval_restraint(const V &v, const stormm_restraint &t, int base
   return e.z;
 }
 
-// Valence term t of the work unit (nothing when t is past the unit's last term).
+// Valence term t of the work unit (nothing when t is past the unit's last term).  A kind's
+// parameters lie in term order, so they are fetched together with the term's atoms.
 template <typename T, bool FORCES, bool CLASH>
-__device__ void valence_term(StageCtx<T> &c, const MMKit &k, int kind, int t) {
-  const int *pre = c.L.vpre + (kind * (kMaxWuSystems + 1));
-  if (t >= pre[c.wu.sys_count]) {
+__device__ __forceinline__ void valence_term(StageCtx<T> &c, const MMKit &k, int kind, int t) {
+  const int n = c.wu.sys_count;
+  const int count = (kind == kVBond) ? c.wu.bond_count :
+                    (kind == kVAngle) ? c.wu.angl_count :
+                                        c.wu.term_count - c.wu.bond_count - c.wu.angl_count;
+  if (t >= count) {
     return;
   }
   const double fscale = ldexp(1.0, k.frc_bits);
   const double nrg_scale = ldexp(1.0, k.nrg_bits);
-  ValenceCtxT<typename Prec<T>::crd_t> v;
-  v.cx = c.L.cx;
-  v.cy = c.L.cy;
-  v.cz = c.L.cz;
-  v.gidx = c.L.gidx;
-  v.crd_scale = static_cast<double>(c.crd_scale);
-  v.crd_scale_f = static_cast<float>(c.crd_scale);
-  v.fx = c.L.fx;
-  v.fy = c.L.fy;
-  v.fz = c.L.fz;
+  const ValenceCtxT<T> v(c);
   // The system's terms of this kind, in its template's bonds / angles / dihedrals order.
-  const int slot = find_slot(pre, c.wu.sys_count, t);
+  const int slot = (kind == kVBond) ? find_slot<&WuSys::bond_pre>(c.L.sys, n, t) :
+                   (kind == kVAngle) ? find_slot<&WuSys::angl_pre>(c.L.sys, n, t) :
+                                       find_slot<&WuSys::dihe_pre>(c.L.sys, n, t);
   const WuSys &ws = c.L.sys[slot];
+  const int local = t - ((kind == kVBond) ? ws.bond_pre :
+                         (kind == kVAngle) ? ws.angl_pre : ws.dihe_pre);
   const int kind_first = (kind == kVBond) ? 0 :
                          (kind == kVAngle) ? ws.bond_count : ws.bond_count + ws.angl_count;
-  const int4 vt = k.vterms[ws.term_first + kind_first + (t - pre[slot])];
+  const int par = local + ((kind == kVBond) ? ws.bond_par :
+                           (kind == kVAngle) ? ws.angl_par : ws.dihe_par);
+  const int4 vt = k.vterms[ws.term_first + kind_first + local];
   const int i = ws.lds_base + (vt.y & 0xffff), j = ws.lds_base + (vt.y >> 16);
   const int kk = ws.lds_base + (vt.z & 0xffff), l = ws.lds_base + (vt.z >> 16);
   long long *nrg = &c.L.nrg[slot * 16];
   if (kind == kVBond) {
-    const double2 p = k.bond_par[vt.w];
+    const double2 p = k.bond_par[par];
     lds_add(&nrg[kBond], fix64(eval_bond<FORCES>(v, i, j, p.x, p.y, fscale) * nrg_scale));
   }
   else if (kind == kVAngle) {
-    const double2 p = k.angl_par[vt.w];
+    const double2 p = k.angl_par[par];
     lds_add(&nrg[kAngle], fix64(eval_angle<FORCES>(v, i, j, kk, p.x, p.y, fscale) * nrg_scale));
   }
   else if (std::is_same<T, float>::value) {
-    const DiheParam p = k.dihe_par[vt.w];
+    const DiheParam p = k.dihe_par[par];
     const float e = eval_dihedral_f<FORCES>(v, i, j, kk, l, p, k.frc_bits);
     lds_add(&nrg[p.improper ? kImproperDihedral : kProperDihedral],
             fix64(static_cast<double>(e) * nrg_scale));
-    const double2 a14 = k.dihe14[vt.w];
+    const double2 a14 = k.dihe14[par];
     if (a14.x > 0.0) {
       float ele, vdw;
       const bool con = CLASH && (c.L.clash_on[slot] != 0);
@@ -1763,10 +1735,10 @@ __device__ void valence_term(StageCtx<T> &c, const MMKit &k, int kind, int t) {
     }
   }
   else {
-    const DiheParam p = k.dihe_par[vt.w];
+    const DiheParam p = k.dihe_par[par];
     const double e = eval_dihedral<FORCES>(v, i, j, kk, l, p, fscale);
     lds_add(&nrg[p.improper ? kImproperDihedral : kProperDihedral], fix64(e * nrg_scale));
-    const double2 a14 = k.dihe14[vt.w];
+    const double2 a14 = k.dihe14[par];
     if (a14.x > 0.0) {
       double ele, vdw;
       const bool con = CLASH && (c.L.clash_on[slot] != 0);
@@ -1782,7 +1754,7 @@ __device__ void valence_term(StageCtx<T> &c, const MMKit &k, int kind, int t) {
 
 // Valence terms on their own (evaluations without pair tiles), in chunks of 64 per wavefront.
 template <typename T, bool FORCES, bool CLASH>
-__device__ void stage_valence(StageCtx<T> &c, const MMKit &k) {
+__device__ __forceinline__ void stage_valence(StageCtx<T> &c, const MMKit &k) {
   const int lane = c.tid & 63;
   const int chunks = valence_chunks(c);
   for (int item = next_item(&c.L.work[2], lane); item < chunks;
@@ -1795,20 +1767,11 @@ __device__ void stage_valence(StageCtx<T> &c, const MMKit &k) {
 // Restraints of the unit's systems, one thread each, in a stage of their own so that their
 // double-precision code stays out of the register budget of the tile loops.
 template <typename T, bool FORCES>
-__device__ void stage_restraints(StageCtx<T> &c, const MMKit &k) {
+__device__ __forceinline__ void stage_restraints(StageCtx<T> &c, const MMKit &k) {
   const double fscale = ldexp(1.0, k.frc_bits);
   const double nrg_scale = ldexp(1.0, k.nrg_bits);
   const double inv_gpos = ldexp(1.0, -(k.gpos_bits - c.org_shift));
-  ValenceCtxT<typename Prec<T>::crd_t> v;
-  v.cx = c.L.cx;
-  v.cy = c.L.cy;
-  v.cz = c.L.cz;
-  v.gidx = c.L.gidx;
-  v.crd_scale = static_cast<double>(c.crd_scale);
-  v.crd_scale_f = static_cast<float>(c.crd_scale);
-  v.fx = c.L.fx;
-  v.fy = c.L.fy;
-  v.fz = c.L.fz;
+  const ValenceCtxT<T> v(c);
   for (int r = c.tid; r < c.wu.rst_count; r += c.nthr) {
     int slot = 0, u = r;
     while (u >= c.L.sys[slot].rst_count) {
@@ -1834,7 +1797,7 @@ __device__ void stage_restraints(StageCtx<T> &c, const MMKit &k) {
 template <typename T, bool FORCES, bool CLASH, bool RESTRAINTS = true>
 __device__ __forceinline__ void evaluate_wu(StageCtx<T> &c, const MMKit &k, int terms) {
   const bool lj_table = (c.wu.lj_table != 0);
-  stage_load_coords<T, CLASH>(c, k);
+  stage_load<T, CLASH>(c, k);
   // With GB the valence terms ride along with the Born-integral tiles.
   const bool val = (terms & kTermValence) != 0;
   if (c.gb) {
@@ -1882,12 +1845,12 @@ __device__ __forceinline__ void stage_store(StageCtx<T> &c, const MMKit &k, bool
     // stored values and split into word and overflow word.
     long long *frc[3] = {k.xfrc, k.yfrc, k.zfrc};
     int *ovr[3] = {k.xfrc_ovrf, k.yfrc_ovrf, k.zfrc_ovrf};
-    const long long *lds[3] = {L.fx, L.fy, L.fz};
     for (int a = c.tid; a < c.wu.lds_atoms; a += c.nthr) {
       const int g = L.gidx[a];
       if (g >= 0) {
+        const long long sum[3] = {L.frc[a].x, L.frc[a].y, L.frc[a].z};
         for (int d = 0; d < 3; d++) {
-          __int128 v = static_cast<__int128>(lds[d][a]) << k.frc_store_shift;
+          __int128 v = static_cast<__int128>(sum[d]) << k.frc_store_shift;
           if (!k.store_overwrite) {
             v += i95_value(frc[d][g], ovr[d][g]);
           }
@@ -1901,14 +1864,14 @@ __device__ __forceinline__ void stage_store(StageCtx<T> &c, const MMKit &k, bool
       const int g = L.gidx[a];
       if (g >= 0) {
         if (k.store_overwrite) {
-          k.xfrc[g] = L.fx[a];
-          k.yfrc[g] = L.fy[a];
-          k.zfrc[g] = L.fz[a];
+          k.xfrc[g] = L.frc[a].x;
+          k.yfrc[g] = L.frc[a].y;
+          k.zfrc[g] = L.frc[a].z;
         }
         else {
-          k.xfrc[g] += L.fx[a];
-          k.yfrc[g] += L.fy[a];
-          k.zfrc[g] += L.fz[a];
+          k.xfrc[g] += L.frc[a].x;
+          k.yfrc[g] += L.frc[a].y;
+          k.zfrc[g] += L.frc[a].z;
         }
       }
     }

@@ -14,7 +14,6 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
   init_ctx<T>(c, k, blockIdx.x, terms);
-  stage_load_params<T>(c, k);
   evaluate_wu<T, FORCES, CLASH>(c, k, terms);
   stage_store<T, FORCES>(c, k, eval_energy != 0);
 }

@@ -511,7 +511,6 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
   const int terms = kTermNonbonded | kTermValence;
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
   init_ctx<T>(c, k, blockIdx.x, terms);
-  stage_load_params<T>(c, k);
   if (pending_move >= 0) {
     // Move factors of the unit's systems (line_step as in k_line_advance, on the exact sum of
     // the 13 ScoreCard components).  The coordinate stage reads them after its first barrier.

@@ -278,6 +278,9 @@ static int add_template(const stormm_topology_batch *b, const SystemTerms &t, in
   }
   // Valence terms with system-relative atom indices.
   tp.term_first = static_cast<int>(P.vterms.size());
+  tp.bond_par = static_cast<int>(P.bond_par.size());
+  tp.angl_par = static_cast<int>(P.angl_par.size());
+  tp.dihe_par = static_cast<int>(P.dihe_par.size());
   for (int e = 0; e < t.bond_count; e++) {
     const int k = t.bond_first + e;
     const int i = b->bond_atoms[2 * k], j = b->bond_atoms[2 * k + 1];
@@ -698,6 +701,9 @@ void compact_templates(TemplateStore &ts, const std::vector<char> &keep, std::ve
     tp.task_first = task_first;
     // Valence terms with their parameters (a dihedral's 1:4 factors share its index).
     const int term_first = static_cast<int>(out.vterms.size());
+    tp.bond_par = static_cast<int>(out.bond_par.size());
+    tp.angl_par = static_cast<int>(out.angl_par.size());
+    tp.dihe_par = static_cast<int>(out.dihe_par.size());
     for (int i = 0; i < tp.term_count; i++) {
       int4 v = ts.vterms[tp.term_first + i];
       if (v.x == kVBond) {
@@ -752,12 +758,8 @@ int fill_atom_parameters(const stormm_topology_batch *b, const SystemTerms &t, i
     }
     const double pr = (b->pb_radii != nullptr) ? b->pb_radii[src] : 0.0;
     const double sc = (b->gb_screen != nullptr) ? b->gb_screen[src] : 0.0;
-    ap.pbr[g] = pr;
     ap.rho[g] = pr - 0.09;
     ap.scr[g] = sc * (pr - 0.09);
-    ap.alpha[g] = sm.alpha;
-    ap.beta[g] = sm.beta;
-    ap.gamma[g] = sm.gamma;
     if (sm.igb != 0 && ap.rho[g] <= 0.0) {
       return fail(STORMM_ERR_INVALID_ARGUMENT, "Born radius must exceed 0.09 A (system " +
                                                    std::to_string(s) + ")");
@@ -780,6 +782,10 @@ int append_work_unit(const std::vector<int> &systems, int lj_table,
   d.term_count = 0;
   d.lj_table = lj_table;
   d.rst_count = 0;
+  d.clean_count = 0;
+  d.bond_count = 0;
+  d.angl_count = 0;
+  d.pad = 0;
   int lds = 0;
   for (int s : systems) {
     const TopoTemplate &tp = ts.templates[sys_template[s]];
@@ -800,7 +806,20 @@ int append_work_unit(const std::vector<int> &systems, int lj_table,
     ws.lj_nt = tp.lj_nt;
     ws.rst_first = (rst_first != nullptr) ? (*rst_first)[s] : 0;
     ws.rst_count = (rst_count != nullptr) ? (*rst_count)[s] : 0;
+    ws.clean_pre = d.clean_count;
+    ws.offd_pre = d.offd_count - d.clean_count;
+    ws.diag_pre = d.task_count - d.offd_count;
+    ws.bond_pre = d.bond_count;
+    ws.angl_pre = d.angl_count;
+    ws.dihe_pre = d.term_count - d.bond_count - d.angl_count;
+    ws.bond_par = tp.bond_par;
+    ws.angl_par = tp.angl_par;
+    ws.dihe_par = tp.dihe_par;
+    ws.pad[0] = ws.pad[1] = ws.pad[2] = 0;
     wu_sys.push_back(ws);
+    d.clean_count += tp.clean_count;
+    d.bond_count += tp.bond_count;
+    d.angl_count += tp.angl_count;
     d.offd_count += tp.offd_count;
     d.task_count += tp.offd_count + tp.diag_count;
     d.term_count += tp.term_count;

@@ -34,6 +34,7 @@ struct TopoTemplate {
   int task_first = 0, offd_count = 0, clean_count = 0, diag_count = 0;
   int term_first = 0, term_count = 0;
   int bond_count = 0, angl_count = 0, dihe_count = 0;
+  int bond_par = 0, angl_par = 0, dihe_par = 0;  // first parameter of each kind, in term order
   int lj_off = 0, lj_nt = 0;
   bool combining = false;
   bool lb = false;        // the LJ interactions follow Lorentz-Berthelot combining
@@ -80,7 +81,7 @@ struct SolventModel {
 
 // Per-atom parameter arrays (one entry per padded global atom).
 struct AtomParams {
-  std::vector<double> q, ljp1, ljp2, rho, scr, pbr, alpha, beta, gamma;
+  std::vector<double> q, ljp1, ljp2, rho, scr;
   std::vector<int> lj_type;
   void assign(size_t n) {
     q.assign(n, 0.0);
@@ -88,10 +89,6 @@ struct AtomParams {
     ljp2.assign(n, 0.0);
     rho.assign(n, 0.0);
     scr.assign(n, 0.0);
-    pbr.assign(n, 0.0);
-    alpha.assign(n, 0.0);
-    beta.assign(n, 0.0);
-    gamma.assign(n, 0.0);
     lj_type.assign(n, 0);
   }
 };

@@ -26,8 +26,8 @@ using namespace stormm_amd;
 
 namespace {
 
-// Device bytes per resident atom: int64 coordinates, forces, previous forces and CG direction
-// (12 x 8) plus nine double parameters and the LJ type.
+// Device bytes counted per resident atom: int64 coordinates, forces, previous forces and CG
+// direction (12 x 8), nine doubles (five parameters and room for four) and the LJ type.
 constexpr size_t kPoolBytesPerAtom = (12 * 8) + (9 * 8) + 4;
 // Device bytes per system slot: layout (2 ints), step / stop flag (2 ints), RMS force, nine
 // line-search doubles and a ScoreCard row.
@@ -83,7 +83,7 @@ struct stormm_pool {
   std::vector<int> slot_range;          // range of each resident slot
   // Device state.
   DevMem xcrd, ycrd, zcrd, xfrc, yfrc, zfrc, xprv, yprv, zprv, xcg, ycg, zcg;
-  DevMem q, ljp1, ljp2, rho, scr, pbr, alpha, beta, gamma, lj_type;
+  DevMem q, ljp1, ljp2, rho, scr, lj_type;
   DevMem starts, natoms, steps, done, rms, line, scorecard, status;
   // Energy history per slot: hist_len ScoreCard rows, one every cfg.minimize.
   // diagnostic_print_frequency cycles (none when that is 0).
@@ -167,8 +167,7 @@ extern "C" int stormm_pool_create(const stormm_pool_config *cfg, stormm_pool **o
     HIP_TRY(d->alloc(na * sizeof(long long)));
     HIP_TRY(hipMemset(d->ptr, 0, na * sizeof(long long)));
   }
-  for (DevMem *d : {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr, &p->pbr, &p->alpha, &p->beta,
-                    &p->gamma}) {
+  for (DevMem *d : {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr}) {
     HIP_TRY(d->alloc(na * sizeof(double)));
   }
   HIP_TRY(p->lj_type.alloc(na * sizeof(int)));
@@ -464,10 +463,6 @@ static int admit_entries(stormm_pool *pool, const stormm_topology_batch *batch,
   HIP_TRY(put(p->ljp2, ap.ljp2.data(), sizeof(double)));
   HIP_TRY(put(p->rho, ap.rho.data(), sizeof(double)));
   HIP_TRY(put(p->scr, ap.scr.data(), sizeof(double)));
-  HIP_TRY(put(p->pbr, ap.pbr.data(), sizeof(double)));
-  HIP_TRY(put(p->alpha, ap.alpha.data(), sizeof(double)));
-  HIP_TRY(put(p->beta, ap.beta.data(), sizeof(double)));
-  HIP_TRY(put(p->gamma, ap.gamma.data(), sizeof(double)));
   HIP_TRY(put(p->lj_type, ap.lj_type.data(), sizeof(int)));
   off = 0;
   int rid;
@@ -614,10 +609,9 @@ static MMKit pool_mm_kit(stormm_pool *p, int nwu, int maxa, int block, const WuD
   k.ljab14 = p->ljab14.as<double2>();
   k.rho = p->rho.as<double>();
   k.scr = p->scr.as<double>();
-  k.pbr = p->pbr.as<double>();
-  k.gb_alpha = p->alpha.as<double>();
-  k.gb_beta = p->beta.as<double>();
-  k.gb_gamma = p->gamma.as<double>();
+  k.gb_alpha = p->sm.alpha;
+  k.gb_beta = p->sm.beta;
+  k.gb_gamma = p->sm.gamma;
   k.xcrd = p->xcrd.as<long long>();
   k.ycrd = p->ycrd.as<long long>();
   k.zcrd = p->zcrd.as<long long>();
