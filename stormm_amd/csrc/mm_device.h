@@ -267,35 +267,49 @@ template <> struct EvalBlockLimit<double> {
 };
 
 // ------------------------------------------------------------------------------------------
-// Work-unit LDS layout.  What the pair loops read of one atom lies together, so that a lane
-// fetches it with one address and one or two wide reads: with one array per quantity the tile
-// set-up and the near-pair passes spent a third of their vector instructions on addresses.
+// Work-unit LDS layout.  Everything the pair loops read or add to of one atom lies in one record,
+// so that a lane reaches all of it from one address, with wide reads and constant offsets: with
+// one array per quantity the tile set-up and the near-pair passes spent a third of their vector
+// instructions on addresses.  The record's 80 bytes (144 in double precision) put the same field
+// of 16 consecutive atoms in different LDS banks (20 l mod 64 banks differ for l = 0..15).
 // ------------------------------------------------------------------------------------------
 template <typename T> struct alignas(16) AtomPos {
   typename Prec<T>::crd_t x, y, z;
   T scr;                    // screened radius
 };
-template <typename T> struct alignas(2 * sizeof(T)) AtomRad {
-  T rho, irho;              // offset radius and its inverse
-};
 template <typename T> struct alignas(16) AtomNb {
   T q, p1, p2;              // charge and Lennard-Jones parameters
   T rad;                    // effective Born radius
 };
-struct AtomFrc {
-  long long x, y, z;        // 24 bytes: consecutive atoms' components fall in different banks
+template <typename T> struct alignas(2 * sizeof(T)) AtomRad {
+  T rho, irho;              // offset radius and its inverse
 };
+template <typename T> struct AtomFields {
+  AtomPos<T> pos;
+  AtomNb<T> nb;
+  AtomRad<T> rr;
+  union {
+    long long psi;          // Born-radius integral; from the radii stage on dR/dpsi (a double)
+    T sd;                   // chain-rule factor, from the chain stage on
+  };
+  long long fx, fy, fz;     // forces
+  long long dedr;           // dE/dR
+};
+template <typename T> struct AtomRec;
+template <> struct AtomRec<float> : AtomFields<float> {};
+template <> struct AtomRec<double> : AtomFields<double> {
+  double pad[2];
+};
+static_assert(sizeof(AtomRec<float>) == 80 && sizeof(AtomRec<double>) == 144,
+              "atom records keep 16 consecutive atoms' fields in different LDS banks");
 
 template <typename T> struct WuLds {
   using crd_t = typename Prec<T>::crd_t;
   int4 *tasks;              // the unit's tile tasks, placed at their systems' LDS bases
-  AtomPos<T> *pos;
-  AtomNb<T> *nb;
-  AtomRad<T> *rr;
-  AtomFrc *frc;
-  long long *psi, *dedr, *nrg, *org;
+  AtomRec<T> *atom;
+  long long *nrg, *org;
   double *move;             // per system: pending line move (coordinate units per direction unit)
-  T *irad;                  // inverse Born radius; after the pair stage the chain-rule factor
+  T *irad;                  // inverse Born radius
   int *gidx, *slot;
   WuSys *sys;
   int *work;                // per-stage work-item counters (kStageCounters)
@@ -306,8 +320,7 @@ template <typename T> struct WuLds {
   static __host__ __device__ size_t bytes(int maxa, int waves) {
     const size_t m = static_cast<size_t>(maxa);
     return (kMaxWuTasks * sizeof(int4)) +
-           (m * (sizeof(AtomPos<T>) + sizeof(AtomNb<T>) + sizeof(AtomRad<T>) + sizeof(AtomFrc))) +
-           (kMaxWuSystems * sizeof(WuSys)) + (2 * m * sizeof(long long)) +
+           (m * sizeof(AtomRec<T>)) + (kMaxWuSystems * sizeof(WuSys)) +
            (kMaxWuSystems * 16 * sizeof(long long)) + (3 * kMaxWuSystems * sizeof(long long)) +
            (kMaxWuSystems * sizeof(double)) + (m * sizeof(T)) + (2 * kMaxWuSystems * sizeof(T)) +
            (2 * m * sizeof(int)) + (kStageCounters * sizeof(int)) +
@@ -325,13 +338,8 @@ template <typename T> struct WuLds {
     };
     const size_t m = static_cast<size_t>(maxa);
     tasks = reinterpret_cast<int4 *>(take(kMaxWuTasks * sizeof(int4)));
-    pos = reinterpret_cast<AtomPos<T> *>(take(m * sizeof(AtomPos<T>)));
-    nb = reinterpret_cast<AtomNb<T> *>(take(m * sizeof(AtomNb<T>)));
-    rr = reinterpret_cast<AtomRad<T> *>(take(m * sizeof(AtomRad<T>)));
-    frc = reinterpret_cast<AtomFrc *>(take(m * sizeof(AtomFrc)));
+    atom = reinterpret_cast<AtomRec<T> *>(take(m * sizeof(AtomRec<T>)));
     sys = reinterpret_cast<WuSys *>(take(kMaxWuSystems * sizeof(WuSys)));
-    psi = reinterpret_cast<long long *>(take(m * sizeof(long long)));
-    dedr = reinterpret_cast<long long *>(take(m * sizeof(long long)));
     nrg = reinterpret_cast<long long *>(take(kMaxWuSystems * 16 * sizeof(long long)));
     org = reinterpret_cast<long long *>(take(3 * kMaxWuSystems * sizeof(long long)));
     move = reinterpret_cast<double *>(take(kMaxWuSystems * sizeof(double)));

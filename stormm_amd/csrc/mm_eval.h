@@ -113,9 +113,6 @@ __device__ __forceinline__ void stage_load(StageCtx<T> &c, const MMKit &k) {
     const int g = gs + local;
     L.gidx[a] = valid ? g : -1;
     L.slot[a] = s;
-    L.psi[a] = 0;
-    L.dedr[a] = 0;
-    L.frc[a] = {0, 0, 0};
     L.irad[a] = T(1);
     AtomPos<T> pos = {0, 0, 0, T(0)};
     AtomNb<T> nb = {T(0), T(0), T(0), T(1)};
@@ -185,9 +182,13 @@ __device__ __forceinline__ void stage_load(StageCtx<T> &c, const MMKit &k) {
         atomicOr(k.status, static_cast<int>(kStatusCoordinateRange));
       }
     }
-    L.pos[a] = pos;
-    L.nb[a] = nb;
-    L.rr[a] = rr;
+    AtomRec<T> &r = L.atom[a];
+    r.pos = pos;
+    r.nb = nb;
+    r.rr = rr;
+    r.psi = 0;
+    r.fx = r.fy = r.fz = 0;
+    r.dedr = 0;
   }
   // The unit's tile tasks, read once per evaluation: the clean off-diagonal tasks of every
   // system, then their other off-diagonal tasks, then the diagonal ones, each with its system's
@@ -332,8 +333,9 @@ struct TileTask {
 template <typename T>
 __device__ __forceinline__ void tile_coords(const StageCtx<T> &c, const TileTask &tt, T &xi,
                                             T &yi, T &zi, T &xj, T &yj, T &zj, T &si, T &sj) {
-  const AtomPos<T> *pos = c.L.pos;
-  const AtomPos<T> bi = pos[tt.ib], bj = pos[tt.jb], pi = pos[tt.i], pj = pos[tt.j0];
+  const AtomRec<T> *atom = c.L.atom;
+  const AtomPos<T> bi = atom[tt.ib].pos, bj = atom[tt.jb].pos;
+  const AtomPos<T> pi = atom[tt.i].pos, pj = atom[tt.j0].pos;
   const auto ox = tile_centre(bi.x, bj.x);
   const auto oy = tile_centre(bi.y, bj.y);
   const auto oz = tile_centre(bi.z, bj.z);
@@ -425,61 +427,118 @@ __device__ __forceinline__ void valence_chunk(StageCtx<T> &c, const MMKit &k, in
   valence_term<T, FORCES, CLASH>(c, k, kind, (local << 6) + lane);
 }
 
-// Near-field pair queue of a wavefront.  Entries pack the LDS indices of the pair (9 bits each)
-// and which of the two directions (onto i, onto j) lies within 4 screened radii.
-constexpr unsigned kNearI = 1u << 18;
-constexpr unsigned kNearJ = 1u << 19;
+// Near-field pair queue of a wavefront.  An entry packs the byte offsets of the pair's atom
+// records (in double precision halved, to fit 16 bits) and which of the two directions (onto i,
+// onto j) lies within 4 screened radii: j << 16 | i | near_i << 1 | near_j, where the offsets'
+// low bits are free.
+constexpr unsigned kNearI = 2u;
+constexpr unsigned kNearJ = 1u;
+template <typename T> struct NearIndex {
+  static constexpr int kShift = (sizeof(T) == 4) ? 0 : 1;
+  static constexpr unsigned kMask = 0xfff8u;
+  static_assert(((kMaxWuAtoms - 1) * sizeof(AtomRec<T>)) >> kShift <= 0xffffu,
+                "record offsets do not fit a near-queue entry");
+  static_assert(((sizeof(AtomRec<T>) >> kShift) & ~kMask) == 0,
+                "record offsets need their low bits for the near flags");
+  // The halves of an entry's two parts, which nearq_push doubles.
+  static __device__ __forceinline__ unsigned half_i(int i) {
+    return static_cast<unsigned>(i) * static_cast<unsigned>(sizeof(AtomRec<T>) >> (kShift + 1));
+  }
+  static __device__ __forceinline__ int half_j(int j) {
+    return static_cast<int>(half_i(j) << 16);
+  }
+  static __device__ __forceinline__ AtomRec<T> &record(AtomRec<T> *atom, unsigned off) {
+    return *reinterpret_cast<AtomRec<T> *>(reinterpret_cast<unsigned char *>(atom) +
+                                           (off << kShift));
+  }
+};
 
-__device__ __forceinline__ unsigned near_entry(int i, int j, bool near_i, bool near_j) {
-  return static_cast<unsigned>(i) | (static_cast<unsigned>(j) << 9) | (near_i ? kNearI : 0u) |
-         (near_j ? kNearJ : 0u);
+// LDS byte address of a pointer into the block's dynamic LDS.
+__device__ __forceinline__ unsigned lds_address(const void *p) {
+  return static_cast<unsigned>(reinterpret_cast<size_t>(
+      (const __attribute__((address_space(3))) unsigned char *)p));
 }
 
-// Appends the entries of the lanes with `need` set, in lane order; n is wave-uniform.  Every
-// lane stores: the lanes with an entry to n, n + 1, ..., the others to the slots after them
-// (the r-th lane without an entry, counting from lane 0, to n + 63 - r, which is at least
-// n + count because at most 64 - count lanes have none), which later pushes overwrite (before a
-// group of steps the queue holds at most 63 entries and a group pushes at most 4 x 64, so every
-// store stays inside the queue's stride).  The step thus has no branch, which would split it
-// and keep the rotated operands from folding into their instructions.  rlane4 is 4 (63 - lane),
-// a byte offset.
-__device__ __forceinline__ void nearq_push(unsigned *q, int &n, bool near_i, bool near_j,
-                                           unsigned entry, int rlane4) {
-  // The mask is the union of the two directions' ballots (each a comparison's lane mask).
-  const bool need = near_i || near_j;
-  const unsigned long long m = __builtin_amdgcn_ballot_w64(near_i) |
-                               __builtin_amdgcn_ballot_w64(near_j);
-  const int below = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32),
-                                              __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m),
-                                                                        0u));
-  // For a lane without an entry, below + 63 - lane = 63 - r.
-  unsigned char *slot = reinterpret_cast<unsigned char *>(q + n) + (below << 2);
-  *reinterpret_cast<unsigned *>(slot + (need ? 0 : rlane4)) = entry;
+// Appends the entries of the lanes with a direction that is not far, in lane order, to the queue
+// at LDS byte address q holding n entries (both wavefront-uniform).  All 64 lanes must run it.
+// ei = half_i(i); ej = half_j of the j atom at step 0, rotated K lanes here.  Five
+// vector instructions: the two flags enter as carries of the additions that join the indices
+// (the first reads ej through DPP) and the store runs under the lanes' own mask, set and restored
+// with scalar instructions inside one statement, so that the step stays one basic block.  A push
+// made of selects and spare slots for the lanes without an entry took nine of a Born-integral
+// step's 37 instructions; the stages are bound by vector-instruction issue.
+template <int K>
+__device__ __forceinline__ void nearq_push(unsigned q, int &n, bool far_i, bool far_j,
+                                           unsigned ei, int ej) {
+  // From the comparisons the step selects by: a ballot of their negations compares once more.
+  const unsigned long long mi = ~__builtin_amdgcn_ballot_w64(far_i);
+  const unsigned long long mj = ~__builtin_amdgcn_ballot_w64(far_j);
+  const unsigned long long m = mi | mj;
+  const unsigned lo = static_cast<unsigned>(m), hi = static_cast<unsigned>(m >> 32);
+  const unsigned base = q + (static_cast<unsigned>(n) << 2);
+  unsigned entry, slot;
+  unsigned long long all;
+  // The two scalar instructions ahead of the DPP read cover the wait that a vector write of ej
+  // just before would need.
+  if constexpr (K == 0) {
+    asm volatile("s_mov_b64 vcc, %[mi]\n\t"
+                 "v_addc_co_u32_e32 %[e], vcc, %[ej], %[ei], vcc\n\t"
+                 "s_mov_b64 vcc, %[mj]\n\t"
+                 "v_addc_co_u32_e32 %[e], vcc, %[e], %[e], vcc\n\t"
+                 "v_mbcnt_lo_u32_b32 %[s], %[lo], 0\n\t"
+                 "v_mbcnt_hi_u32_b32 %[s], %[hi], %[s]\n\t"
+                 "v_lshl_add_u32 %[s], %[s], 2, %[base]\n\t"
+                 "s_mov_b64 %[x], exec\n\t"
+                 "s_mov_b64 exec, %[m]\n\t"
+                 "ds_write_b32 %[s], %[e]\n\t"
+                 "s_mov_b64 exec, %[x]"
+                 : [e] "=&v"(entry), [s] "=&v"(slot), [x] "=&s"(all)
+                 : [mi] "s"(mi), [mj] "s"(mj), [m] "s"(m), [lo] "s"(lo), [hi] "s"(hi),
+                   [base] "s"(base), [ei] "v"(ei), [ej] "v"(ej)
+                 : "vcc", "memory");
+  }
+  else {
+    asm volatile("s_mov_b64 vcc, %[mi]\n\t"
+                 "s_nop 0\n\t"
+                 "v_addc_co_u32_dpp %[e], vcc, %[ej], %[ei], vcc row_ror:%[k] row_mask:0xf "
+                 "bank_mask:0xf\n\t"
+                 "s_mov_b64 vcc, %[mj]\n\t"
+                 "v_addc_co_u32_e32 %[e], vcc, %[e], %[e], vcc\n\t"
+                 "v_mbcnt_lo_u32_b32 %[s], %[lo], 0\n\t"
+                 "v_mbcnt_hi_u32_b32 %[s], %[hi], %[s]\n\t"
+                 "v_lshl_add_u32 %[s], %[s], 2, %[base]\n\t"
+                 "s_mov_b64 %[x], exec\n\t"
+                 "s_mov_b64 exec, %[m]\n\t"
+                 "ds_write_b32 %[s], %[e]\n\t"
+                 "s_mov_b64 exec, %[x]"
+                 : [e] "=&v"(entry), [s] "=&v"(slot), [x] "=&s"(all)
+                 : [mi] "s"(mi), [mj] "s"(mj), [m] "s"(m), [lo] "s"(lo), [hi] "s"(hi),
+                   [base] "s"(base), [ei] "v"(ei), [ej] "v"(ej), [k] "n"(K)
+                 : "vcc", "memory");
+  }
   n += __popcll(m);
-  __builtin_amdgcn_wave_barrier();
 }
 
 // The Born-integral and derivative stages run their rotation steps in groups of kStepGroup with
 // compile-time rotation counts inside a group; the j-side data move kStepGroup lanes between
 // groups, and the near-pair queue is drained after each group, taking 64 entries at a time from
-// its end.  Before a group the queue holds at most 63 entries, so a group's last push starts at
-// entry 63 + (kStepGroup - 1) x 64 at most and stores its 64 lanes below that plus 64.
+// its end.  Before a group the queue holds at most 63 entries, and a group pushes at most 64 in
+// each step.
 constexpr int kStepGroup = 4;
-static_assert(63 + ((kStepGroup - 1) * 64) + 64 <= kNearQueue,
-              "near queue too short for a step group");
+static_assert(63 + (kStepGroup * 64) <= kNearQueue, "near queue too short for a step group");
 
 // Geometry of a queued pair, recomputed from the LDS coordinates.
 template <typename T> struct NearPair {
-  int i, j;
+  AtomRec<T> &i, &j;
   bool near_i, near_j;
   T dx, dy, dz, r2, invr, r, si, sj;
-  __device__ __forceinline__ NearPair(const StageCtx<T> &c, unsigned e) {
+  __device__ __forceinline__ NearPair(const StageCtx<T> &c, unsigned e)
+      : i(NearIndex<T>::record(c.L.atom, e & NearIndex<T>::kMask)),
+        j(NearIndex<T>::record(c.L.atom, e >> 16)) {
     using P = Prec<T>;
-    i = static_cast<int>(e & 0x1ffu);
-    j = static_cast<int>((e >> 9) & 0x1ffu);
     near_i = (e & kNearI) != 0u;
     near_j = (e & kNearJ) != 0u;
-    const AtomPos<T> pi = c.L.pos[i], pj = c.L.pos[j];
+    const AtomPos<T> pi = i.pos, pj = j.pos;
     dx = crd_delta(pj.x, pi.x, c.crd_scale);
     dy = crd_delta(pj.y, pi.y, c.crd_scale);
     dz = crd_delta(pj.z, pi.z, c.crd_scale);
@@ -495,17 +554,16 @@ template <typename T> struct NearPair {
 template <typename T>
 __device__ __forceinline__ void psi_drain(StageCtx<T> &c, const unsigned *q, int count,
                                           int lane) {
-  WuLds<T> &L = c.L;
   if (lane < count) {
     const NearPair<T> p(c, q[lane]);
-    const AtomRad<T> ri = L.rr[p.i], rj = L.rr[p.j];
+    const AtomRad<T> ri = p.i.rr, rj = p.j.rr;
     if (p.near_i) {
       const T t = psi_near(p.r, p.r2, p.invr, ri.rho, ri.irho, p.sj);
-      lds_add(&L.psi[p.i], fixed_contrib(t, kPsiBits));
+      lds_add(&p.i.psi, fixed_contrib(t, kPsiBits));
     }
     if (p.near_j) {
       const T t = psi_near(p.r, p.r2, p.invr, rj.rho, rj.irho, p.si);
-      lds_add(&L.psi[p.j], fixed_contrib(t, kPsiBits));
+      lds_add(&p.j.psi, fixed_contrib(t, kPsiBits));
     }
   }
 }
@@ -524,10 +582,10 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
   WuLds<T> &L = c.L;
   const int il = c.tid & 15;
   const int lane = c.tid & 63;
-  const int rlane4 = (63 - lane) << 2;
   // Wavefront-uniform, so the queue's base address stays in scalar registers.
   const int wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
-  unsigned *q = L.nearq + (wave * kNearQueueStride);
+  const unsigned *q = L.nearq + (wave * kNearQueueStride);
+  const unsigned qaddr = lds_address(q);
   int qn = 0;
   const double psi_scale = ldexp(1.0, kPsiBits);
   const int quads = (c.wu.task_count + 3) >> 2;
@@ -545,9 +603,8 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
     const T si3 = si2 * si;
     T sj2 = sj * sj;
     T sj3 = sj2 * sj;
-    // Queue entry bits of the pair: i in bits 0..8, the j atom in bits 9..17.
-    const unsigned ei = static_cast<unsigned>(tt.i);
-    int ej = tt.j0 << 9;
+    const unsigned ei = NearIndex<T>::half_i(tt.i);
+    int ej = NearIndex<T>::half_j(tt.j0);
     T acci = T(0), accj = T(0);
     unsigned vbits = tt.valid;
     // Off-diagonal tiles need no pair mask (their padding atoms sit far away); a wavefront whose
@@ -580,10 +637,7 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
           const T tj = psi_series(x_j) * (si3 * invr4);
           acci -= far_i ? ti : T(0);
           accj = row_rotate(accj) - (far_j ? tj : T(0));
-          nearq_push(q, qn, !far_i, !far_j,
-                     ei | static_cast<unsigned>(row_ror<K>(ej)) | (far_i ? 0u : kNearI) |
-                         (far_j ? 0u : kNearJ),
-                     rlane4);
+          nearq_push<K>(qaddr, qn, far_i, far_j, ei, ej);
         };
         unrolled_steps(step, std::integer_sequence<int, 0, 1, 2, 3>{});
         settle(acci);
@@ -607,13 +661,13 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
       run(std::true_type{});
     }
     if (tt.ivalid) {
-      lds_add(&L.psi[tt.i], Prec<double>::fixed(static_cast<double>(acci) * psi_scale));
+      lds_add(&L.atom[tt.i].psi, Prec<double>::fixed(static_cast<double>(acci) * psi_scale));
     }
     // After the last step the j sums sit nsteps - 1 lanes right of the lanes that loaded them.
     const int jl_home = tt.jl_home();
     if (jl_home < tt.nj) {
-      lds_add(&L.psi[tt.jb + jl_home], Prec<double>::fixed(static_cast<double>(accj) *
-                                                           psi_scale));
+      lds_add(&L.atom[tt.jb + jl_home].psi,
+              Prec<double>::fixed(static_cast<double>(accj) * psi_scale));
     }
   }
   psi_drain(c, q, qn, lane);
@@ -633,7 +687,7 @@ __device__ __forceinline__ void stage_radii(StageCtx<T> &c, const MMKit &k, doub
     if (g < 0) {
       continue;
     }
-    const double psi = static_cast<double>(L.psi[a]) * ldexp(1.0, -kPsiBits);
+    const double psi = static_cast<double>(L.atom[a].psi) * ldexp(1.0, -kPsiBits);
     const double rho = k.rho[g];
     double R;
     if (k.igb == 1) {
@@ -651,10 +705,10 @@ __device__ __forceinline__ void stage_radii(StageCtx<T> &c, const MMKit &k, doub
         // in the accumulator slot whose psi is no longer needed.
         const double dr_dpsi = (al - ((2.0 * be) - (3.0 * ga * fipsi)) * fipsi) *
                                (1.0 - thi * thi) * rho / pbr;
-        L.psi[a] = __double_as_longlong(dr_dpsi);
+        L.atom[a].psi = __double_as_longlong(dr_dpsi);
       }
     }
-    L.nb[a].rad = static_cast<T>(R);
+    L.atom[a].nb.rad = static_cast<T>(R);
     L.irad[a] = static_cast<T>(1.0 / R);
     // q holds charge * sqrt(Coulomb), so q^2 = Coulomb * charge^2.
     const double qg = k.q[g];
@@ -667,7 +721,7 @@ __device__ __forceinline__ void stage_radii(StageCtx<T> &c, const MMKit &k, doub
                                                                                   nrg_scale)));
     if (FORCES) {
       const double sdi = atmqd2h - (kGbKscale * k.kappa * atmq2h * expmkf * R);
-      L.dedr[a] = static_cast<long long>(__builtin_rint(sdi * ldexp(1.0, kDedrBits)));
+      L.atom[a].dedr = static_cast<long long>(__builtin_rint(sdi * ldexp(1.0, kDedrBits)));
     }
   }
   (void)coulomb_inv_scaled;
@@ -750,6 +804,8 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
   const T kap = T(k.kappa * kGbKscale);
   const bool use_kappa = (k.kappa != 0.0);
   const T dielfac0 = T(1) - inv_diel;
+  // The steps leave out the 1/2 of the radius derivatives (a power of two: no rounding).
+  const T dri_scale = T(0.5) * dedr_scale;
   for (int t = row; t < c.wu.task_count; t += nrows) {
     const Task tk = fetch_task(c, k, t);
     const TileTask tt(tk, il);
@@ -757,7 +813,7 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
     const unsigned nbmask = tt.valid & ~step_mask(emask, tt.jl0);
     T xi, yi, zi, xj, yj, zj, si, sj;
     tile_coords(c, tt, xi, yi, zi, xj, yj, zj, si, sj);
-    const AtomNb<T> ni = L.nb[tt.i], nj = L.nb[tt.j0];
+    const AtomNb<T> ni = L.atom[tt.i].nb, nj = L.atom[tt.j0].nb;
     const T qi = ni.q, p1i = ni.p1, p2i = ni.p2, Ri = ni.rad;
     T qj = nj.q, p1j = nj.p1, p2j = nj.p2, Rj = nj.rad;
     // exp(-r^2 / (4 Ri Rj)) = GbExp(r^2 * (1 / Rj) * (scale / Ri)).
@@ -833,7 +889,7 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
             e_gb -= egb;
             if (FORCES) {
               fmag += temp6 * (T(1) - (T(0.25) * efac));
-              const T temp5 = T(0.5) * efac * temp6 * (rr + (T(0.25) * r2));
+              const T temp5 = efac * temp6 * (rr + (T(0.25) * r2));
               dri += temp5;
               drj = row_rotate(drj) + temp5;
             }
@@ -937,22 +993,23 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
     }
     if (FORCES) {
       if (tt.ivalid) {
-        lds_add(&L.frc[tt.i].x, P::fixed(fxi * frc_scale));
-        lds_add(&L.frc[tt.i].y, P::fixed(fyi * frc_scale));
-        lds_add(&L.frc[tt.i].z, P::fixed(fzi * frc_scale));
+        AtomRec<T> &ri = L.atom[tt.i];
+        lds_add(&ri.fx, P::fixed(fxi * frc_scale));
+        lds_add(&ri.fy, P::fixed(fyi * frc_scale));
+        lds_add(&ri.fz, P::fixed(fzi * frc_scale));
         if (GB) {
-          lds_add(&L.dedr[tt.i], P::fixed(Ri * dri * dedr_scale));
+          lds_add(&ri.dedr, P::fixed(Ri * dri * dri_scale));
         }
       }
       // After the last step the j sums sit nsteps - 1 lanes right of the lanes that loaded them.
       const int jl_home = tt.jl_home();
       if (jl_home < tt.nj) {
-        const int j = tt.jb + jl_home;
-        lds_add(&L.frc[j].x, P::fixed(fxj * frc_scale));
-        lds_add(&L.frc[j].y, P::fixed(fyj * frc_scale));
-        lds_add(&L.frc[j].z, P::fixed(fzj * frc_scale));
+        AtomRec<T> &rj = L.atom[tt.jb + jl_home];
+        lds_add(&rj.fx, P::fixed(fxj * frc_scale));
+        lds_add(&rj.fy, P::fixed(fyj * frc_scale));
+        lds_add(&rj.fz, P::fixed(fzj * frc_scale));
         if (GB) {
-          lds_add(&L.dedr[j], P::fixed(L.nb[j].rad * drj * dedr_scale));
+          lds_add(&rj.dedr, P::fixed(rj.nb.rad * drj * dri_scale));
         }
       }
     }
@@ -972,23 +1029,23 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
 
 // ------------------------------------------------------------------------------------------
 // OBC chain rule on the accumulated radius derivatives, src/Potential/nonbonded_potential.tpp:
-// 985-1017.  The HCT model uses the accumulated values as they stand.  The factors take the place
-// of the inverse radii, which the pair stage was the last to read.
+// 985-1017.  The HCT model uses the accumulated values as they stand.  The factor takes the place
+// of the atom's dR/dpsi.
 template <typename T>
 __device__ __forceinline__ void stage_chain(StageCtx<T> &c, const MMKit &k) {
   WuLds<T> &L = c.L;
   for (int a = c.tid; a < c.wu.lds_atoms; a += c.nthr) {
     const int g = L.gidx[a];
     if (g < 0) {
-      L.irad[a] = T(0);
+      L.atom[a].sd = T(0);
       continue;
     }
-    double sdi = static_cast<double>(L.dedr[a]) * ldexp(1.0, -kDedrBits);
+    double sdi = static_cast<double>(L.atom[a].dedr) * ldexp(1.0, -kDedrBits);
     if (k.igb != 1) {
       // The radii stage left dR/dpsi in the psi slot.
-      sdi *= __longlong_as_double(L.psi[a]);
+      sdi *= __longlong_as_double(L.atom[a].psi);
     }
-    L.irad[a] = static_cast<T>(sdi);
+    L.atom[a].sd = static_cast<T>(sdi);
   }
   __syncthreads();
 }
@@ -998,27 +1055,26 @@ __device__ __forceinline__ void stage_chain(StageCtx<T> &c, const MMKit &k) {
 template <typename T>
 __device__ __forceinline__ void deriv_drain(StageCtx<T> &c, const unsigned *q, int count,
                                             int lane, int frc_bits) {
-  WuLds<T> &L = c.L;
   if (lane < count) {
     const NearPair<T> p(c, q[lane]);
-    const AtomRad<T> ri = L.rr[p.i], rj = L.rr[p.j];
+    const AtomRad<T> ri = p.i.rr, rj = p.j.rr;
     const T invr2 = p.invr * p.invr;
     T fmag = T(0);
     if (p.near_i) {
-      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, ri.rho, ri.irho, p.sj) * L.irad[p.i];
+      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, ri.rho, ri.irho, p.sj) * p.i.sd;
     }
     if (p.near_j) {
-      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, rj.rho, rj.irho, p.si) * L.irad[p.j];
+      fmag += dpsi_near(p.r, p.r2, p.invr, invr2, rj.rho, rj.irho, p.si) * p.j.sd;
     }
     const long long fx = fixed_contrib(fmag * p.dx, frc_bits);
     const long long fy = fixed_contrib(fmag * p.dy, frc_bits);
     const long long fz = fixed_contrib(fmag * p.dz, frc_bits);
-    lds_add(&L.frc[p.i].x, -fx);
-    lds_add(&L.frc[p.i].y, -fy);
-    lds_add(&L.frc[p.i].z, -fz);
-    lds_add(&L.frc[p.j].x, fx);
-    lds_add(&L.frc[p.j].y, fy);
-    lds_add(&L.frc[p.j].z, fz);
+    lds_add(&p.i.fx, -fx);
+    lds_add(&p.i.fy, -fy);
+    lds_add(&p.i.fz, -fz);
+    lds_add(&p.j.fx, fx);
+    lds_add(&p.j.fy, fy);
+    lds_add(&p.j.fz, fz);
   }
 }
 
@@ -1033,10 +1089,10 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
   WuLds<T> &L = c.L;
   const int il = c.tid & 15;
   const int lane = c.tid & 63;
-  const int rlane4 = (63 - lane) << 2;
   // Wavefront-uniform, so the queue's base address stays in scalar registers.
   const int wave = __builtin_amdgcn_readfirstlane(c.tid >> 6);
-  unsigned *q = L.nearq + (wave * kNearQueueStride);
+  const unsigned *q = L.nearq + (wave * kNearQueueStride);
+  const unsigned qaddr = lds_address(q);
   int qn = 0;
   const T frc_scale = T(ldexp(1.0, k.frc_bits));
   const int quads = (c.wu.task_count + 3) >> 2;
@@ -1044,14 +1100,14 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
     const TileTask tt(wave_task(c, k, (item << 2) + ((c.tid >> 4) & 3)), il);
     T xi, yi, zi, xj, yj, zj, si, sj;
     tile_coords(c, tt, xi, yi, zi, xj, yj, zj, si, sj);
-    const T sdi = L.irad[tt.i];
+    const T sdi = L.atom[tt.i].sd;
     const T si2 = si * si;
     const T si3 = si2 * si;
     T sj2 = sj * sj;
     T sj3 = sj2 * sj;
-    T sdj = L.irad[tt.j0];
-    const unsigned ei = static_cast<unsigned>(tt.i);
-    int ej = tt.j0 << 9;
+    T sdj = L.atom[tt.j0].sd;
+    const unsigned ei = NearIndex<T>::half_i(tt.i);
+    int ej = NearIndex<T>::half_j(tt.j0);
     T fxi = T(0), fyi = T(0), fzi = T(0);
     T gxj = T(0), gyj = T(0), gzj = T(0);
     unsigned vbits = tt.valid;
@@ -1092,10 +1148,7 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
           gxj = row_rotate(gxj) + fdx;
           gyj = row_rotate(gyj) + fdy;
           gzj = row_rotate(gzj) + fdz;
-          nearq_push(q, qn, !far_i, !far_j,
-                     ei | static_cast<unsigned>(row_ror<K>(ej)) | (far_i ? 0u : kNearI) |
-                         (far_j ? 0u : kNearJ),
-                     rlane4);
+          nearq_push<K>(qaddr, qn, far_i, far_j, ei, ej);
         };
         unrolled_steps(step, std::integer_sequence<int, 0, 1, 2, 3>{});
         settle(fxi);
@@ -1122,16 +1175,17 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
       run(std::true_type{});
     }
     if (tt.ivalid) {
-      lds_add(&L.frc[tt.i].x, P::fixed(fxi * frc_scale));
-      lds_add(&L.frc[tt.i].y, P::fixed(fyi * frc_scale));
-      lds_add(&L.frc[tt.i].z, P::fixed(fzi * frc_scale));
+      AtomRec<T> &ri = L.atom[tt.i];
+      lds_add(&ri.fx, P::fixed(fxi * frc_scale));
+      lds_add(&ri.fy, P::fixed(fyi * frc_scale));
+      lds_add(&ri.fz, P::fixed(fzi * frc_scale));
     }
     const int jl_home = tt.jl_home();
     if (jl_home < tt.nj) {
-      const int j = tt.jb + jl_home;
-      lds_add(&L.frc[j].x, P::fixed(gxj * frc_scale));
-      lds_add(&L.frc[j].y, P::fixed(gyj * frc_scale));
-      lds_add(&L.frc[j].z, P::fixed(gzj * frc_scale));
+      AtomRec<T> &rj = L.atom[tt.jb + jl_home];
+      lds_add(&rj.fx, P::fixed(gxj * frc_scale));
+      lds_add(&rj.fy, P::fixed(gyj * frc_scale));
+      lds_add(&rj.fz, P::fixed(gzj * frc_scale));
     }
   }
   deriv_drain(c, q, qn, lane, k.frc_bits);
@@ -1166,40 +1220,39 @@ __device__ __forceinline__ float dot(const Vec3f &a, const Vec3f &b) {
 }
 
 template <typename T> struct ValenceCtxT {
-  const AtomPos<T> *pos;
+  AtomRec<T> *atom;
   const int *gidx;
   double crd_scale;
   float crd_scale_f;
-  AtomFrc *frc;
   __device__ __forceinline__ explicit ValenceCtxT(const StageCtx<T> &c)
-      : pos(c.L.pos), gidx(c.L.gidx), crd_scale(static_cast<double>(c.crd_scale)),
-        crd_scale_f(static_cast<float>(c.crd_scale)), frc(c.L.frc) {}
+      : atom(c.L.atom), gidx(c.L.gidx), crd_scale(static_cast<double>(c.crd_scale)),
+        crd_scale_f(static_cast<float>(c.crd_scale)) {}
   // Absolute position (A) of LDS atom a of a system whose coordinate origin is org (fixed
   // precision at inv_gpos).
   __device__ __forceinline__ Vec3 absolute(int a, const long long *org, double inv_gpos) const {
-    const AtomPos<T> p = pos[a];
+    const AtomPos<T> p = atom[a].pos;
     return {(static_cast<double>(org[0]) * inv_gpos) + (static_cast<double>(p.x) * crd_scale),
             (static_cast<double>(org[1]) * inv_gpos) + (static_cast<double>(p.y) * crd_scale),
             (static_cast<double>(org[2]) * inv_gpos) + (static_cast<double>(p.z) * crd_scale)};
   }
   // Single-precision displacement: the LDS coordinates' difference is exact, then rounded once.
   __device__ __forceinline__ Vec3f dispf(int from, int to) const {
-    const AtomPos<T> a = pos[from], b = pos[to];
+    const AtomPos<T> a = atom[from].pos, b = atom[to].pos;
     return {static_cast<float>(b.x - a.x) * crd_scale_f,
             static_cast<float>(b.y - a.y) * crd_scale_f,
             static_cast<float>(b.z - a.z) * crd_scale_f};
   }
   __device__ __forceinline__ Vec3 disp(int from, int to) const {
-    const AtomPos<T> a = pos[from], b = pos[to];
+    const AtomPos<T> a = atom[from].pos, b = atom[to].pos;
     return {(static_cast<double>(b.x) - static_cast<double>(a.x)) * crd_scale,
             (static_cast<double>(b.y) - static_cast<double>(a.y)) * crd_scale,
             (static_cast<double>(b.z) - static_cast<double>(a.z)) * crd_scale};
   }
   __device__ __forceinline__ void add(int a, long long vx, long long vy, long long vz) const {
-    AtomFrc *f = frc + a;
-    lds_add(&f->x, vx);
-    lds_add(&f->y, vy);
-    lds_add(&f->z, vz);
+    AtomRec<T> &r = atom[a];
+    lds_add(&r.fx, vx);
+    lds_add(&r.fy, vy);
+    lds_add(&r.fz, vz);
   }
 };
 
@@ -1848,7 +1901,7 @@ __device__ __forceinline__ void stage_store(StageCtx<T> &c, const MMKit &k, bool
     for (int a = c.tid; a < c.wu.lds_atoms; a += c.nthr) {
       const int g = L.gidx[a];
       if (g >= 0) {
-        const long long sum[3] = {L.frc[a].x, L.frc[a].y, L.frc[a].z};
+        const long long sum[3] = {L.atom[a].fx, L.atom[a].fy, L.atom[a].fz};
         for (int d = 0; d < 3; d++) {
           __int128 v = static_cast<__int128>(sum[d]) << k.frc_store_shift;
           if (!k.store_overwrite) {
@@ -1864,14 +1917,14 @@ __device__ __forceinline__ void stage_store(StageCtx<T> &c, const MMKit &k, bool
       const int g = L.gidx[a];
       if (g >= 0) {
         if (k.store_overwrite) {
-          k.xfrc[g] = L.frc[a].x;
-          k.yfrc[g] = L.frc[a].y;
-          k.zfrc[g] = L.frc[a].z;
+          k.xfrc[g] = L.atom[a].fx;
+          k.yfrc[g] = L.atom[a].fy;
+          k.zfrc[g] = L.atom[a].fz;
         }
         else {
-          k.xfrc[g] += L.frc[a].x;
-          k.yfrc[g] += L.frc[a].y;
-          k.zfrc[g] += L.frc[a].z;
+          k.xfrc[g] += L.atom[a].fx;
+          k.yfrc[g] += L.atom[a].fy;
+          k.zfrc[g] += L.atom[a].fz;
         }
       }
     }
