@@ -528,7 +528,7 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
 template <typename T, bool FORCES, bool CLASH>
 static hipError_t launch_cycle_t(const MMKit &k, const CycleKit &ck, int pending_move,
                                  hipStream_t stream) {
-  const int block = std::min(k.block, EvalBlockLimit<T>::value);
+  const int block = eval_block<T>(k);
   const size_t lds = WuLds<T>::bytes(k.maxa, block / 64);
   auto fn = k_min_cycle<T, FORCES, CLASH>;
   hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),

@@ -905,8 +905,8 @@ int build_plan(const stormm_topology_batch *b, const stormm_launch_shape *shape_
                                              "[16, 512]");
   }
   const int wu_per_cu = (shape.target_wu_per_cu > 0) ? shape.target_wu_per_cu : 2;
-  P.block = (shape.block_threads > 0) ? shape.block_threads : kEvalBlock;
-  if (P.block != 256 && P.block != 512 && P.block != 1024) {
+  P.block = std::max(shape.block_threads, 0);
+  if (P.block != 0 && P.block != 256 && P.block != 512 && P.block != 1024) {
     return fail(STORMM_ERR_INVALID_ARGUMENT, "block_threads must be 256, 512 or 1024");
   }
   const int ns = b->system_count;
@@ -962,6 +962,7 @@ int build_plan(const stormm_topology_batch *b, const stormm_launch_shape *shape_
 
   // Work units.
   const int cus = cu_count_or_default();
+  P.cus = cus;
   std::vector<double> cost(ns);
   std::vector<int> sys_index(ns);
   for (int s = 0; s < ns; s++) {

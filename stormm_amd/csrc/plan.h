@@ -99,7 +99,8 @@ struct SynthesisPlan {
   int padded_atoms = 0;
   SolventModel sm;
   int maxa = 0;
-  int block = kEvalBlock;
+  int block = 0;  // threads per block asked for (0: eval_block's choice)
+  int cus = 256;
   std::vector<int> atom_starts, atom_counts;
   AtomParams ap;
   std::vector<char> lj_table_mode;

@@ -66,6 +66,7 @@ struct stormm_pool {
   stormm_pool_config cfg;
   SolventModel sm;
   int cap_atoms = 0, cap_slots = 0;
+  int cus = 256;  // compute units of the device
   size_t template_budget = 0;
   int batch_counter = 0;
   // Host state.
@@ -158,6 +159,7 @@ extern "C" int stormm_pool_create(const stormm_pool_config *cfg, stormm_pool **o
   p->cap_atoms = static_cast<int>(std::min<size_t>(atoms / kGlobalPad * kGlobalPad,
                                                    static_cast<size_t>(1) << 30));
   p->cap_slots = cfg->max_systems;
+  p->cus = cu_count_or_default();
   if (p->cap_atoms < kGlobalPad) {
     return fail(STORMM_ERR_CAPACITY, "budget holds no atoms");
   }
@@ -584,6 +586,7 @@ static MMKit pool_mm_kit(stormm_pool *p, int nwu, int maxa, int block, const WuD
   k.nwu = nwu;
   k.maxa = round_up(std::max(maxa, kTile), kTile);
   k.block = block;
+  k.cus = p->cus;
   k.gpos_bits = p->cfg.gpos_bits;
   k.frc_bits = p->cfg.frc_bits;
   k.nrg_bits = p->cfg.nrg_bits;
@@ -681,12 +684,12 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
   const stormm_launch_shape &sh = p->cfg.shape;
   const int cap = (sh.wu_atom_capacity > 0) ? sh.wu_atom_capacity : kMaxWuAtoms;
   const int per_cu = (sh.target_wu_per_cu > 0) ? sh.target_wu_per_cu : 2;
-  const int block = (sh.block_threads > 0) ? sh.block_threads : kEvalBlock;
+  const int block = std::max(sh.block_threads, 0);
   std::vector<std::vector<int>> bins;
   std::vector<int> modes;
   // The resident set changes every call; balancing units one by one (largest first) serves
   // these short launches better than the compute-unit groups of the batch synthesis.
-  pack_systems(cost, natom, table, cap, cu_count_or_default(), per_cu, false, bins, modes);
+  pack_systems(cost, natom, table, cap, p->cus, per_cu, false, bins, modes);
   std::vector<WuDesc> wu;
   std::vector<WuSys> wu_sys;
   int maxa = 0;

@@ -167,6 +167,7 @@ extern "C" int stormm_synthesis_create(const stormm_topology_batch *batch,
   k.nwu = static_cast<int>(P.wu.size());
   k.maxa = round_up(std::max(P.maxa, kTile), kTile);
   k.block = P.block;
+  k.cus = P.cus;
   k.igb = P.sm.igb;
   k.dielectric = P.sm.dielectric;
   k.kappa = P.sm.kappa;
