@@ -121,6 +121,11 @@ struct WuSys {
 };
 static_assert(sizeof(WuSys) % sizeof(int4) == 0, "work-unit systems are copied 16 bytes at a time");
 
+// One block of an evaluation in parts (mm_parts.hip): part `part` of `parts` of work unit `unit`.
+struct WuPart {
+  int unit, part, parts, pad;
+};
+
 // One 16 x 16 tile task of a template: x = first atom of the i tile | (first atom of the j tile
 // << 16), relative to the system; y = (diagonal << 8) | (ni << 12) | (nj << 20); z =
 // exclusion-mask offset (-1 when the tile holds no excluded pair); w = unused.  When a work unit
@@ -184,6 +189,12 @@ struct MMKit {
   int clash_cycles, clash_cycle, clash_step_offset;
   const int *clash_step;
   double clash_r0, clash_ratio;
+  // Evaluation in parts: the blocks, and per atom the sums that the parts of a unit share, the
+  // Born-radius integral (zero at rest), dE/dR and dR/dpsi.  nparts == 0: one block per unit.
+  int nparts;
+  const WuPart *parts;
+  long long *part_psi, *part_dedr;
+  double *part_drdpsi;
   // Restraints (src/Potential/valence_potential.tpp:2090-2160) and the step number their
   // parameters are mixed at: rst_step, or, when rst_step_sys holds each system's cycle count,
   // minimizer_step(rst_step_sys[system] + rst_cycle_offset, rst_move, rst_clash_cycles).

@@ -7,6 +7,11 @@ namespace stormm_amd {
 
 hipError_t launch_mm_eval(int precision, const MMKit &k, int terms, int eval_force,
                           int eval_energy, hipStream_t stream);
+// The same evaluation in parts (k.nparts blocks over k.parts; with GB the part arrays, part_psi
+// zero).  A force evaluation leaves part_psi zero; after an energy-only one the caller clears it.
+// Not for 95-bit forces.
+hipError_t launch_mm_parts(int precision, const MMKit &k, int terms, int eval_force,
+                           int eval_energy, hipStream_t stream);
 hipError_t launch_fill(long long *a, long long *b, long long *c, size_t n, hipStream_t stream);
 // Zeroes three int arrays of n entries (overflow words).
 hipError_t launch_fill_int(int *a, int *b, int *c, size_t n, hipStream_t stream);
@@ -67,6 +72,7 @@ struct LineKit {
   double inv_frc_scale, gpos_scale;
   double *l_move, *s_move, *mfac_a, *mfac_b, *mfac_c, *nrg_a, *nrg_b, *nrg_c, *nrg_d;
   int dp_mode;
+  long long *clear;       // per-atom array set to zero for every system (null: none)
 };
 hipError_t launch_conjugate_gradient(const CgKit &k, int step, int sd_cycles,
                                      hipStream_t stream);

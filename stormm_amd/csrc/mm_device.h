@@ -270,14 +270,14 @@ template <> struct EvalBlockLimit<double> {
 // compute unit to itself, and 16 wavefronts hide the latencies that 8 leave open (24 systems of
 // 487 atoms 196 -> 161 us); with more units two blocks of 8 share it, whose barriers do not
 // coincide (1024 systems 110 us against 125).
-template <typename T> inline int eval_block(const MMKit &k) {
+template <typename T> inline int eval_block(const MMKit &k, int blocks) {
   if (k.block > 0) {
     return (k.block < EvalBlockLimit<T>::value) ? k.block : EvalBlockLimit<T>::value;
   }
   if (sizeof(T) == 8) {
     return kMaxEvalBlockDouble;
   }
-  return (k.nwu <= k.cus) ? kEvalBlockSparse : kEvalBlock;
+  return (blocks <= k.cus) ? kEvalBlockSparse : kEvalBlock;
 }
 
 // ------------------------------------------------------------------------------------------

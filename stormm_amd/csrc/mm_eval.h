@@ -27,6 +27,7 @@ template <typename T> struct StageCtx {
   int cycle;         // minimization cycle of this evaluation (clash-damping schedule)
   int rst_step;      // restraint step number when the kit gives no per-system cycle counts
   bool gb;
+  int part = 0, parts = 1;  // this block's share of the unit's tile tasks and valence chunks
   bool move_pending = false;  // stage_load adds L.move[slot] x direction first
   __device__ StageCtx(unsigned char *smem, int maxa, int waves) : L(smem, maxa, waves) {}
 };
@@ -68,7 +69,10 @@ __device__ __forceinline__ long long moved(const long long *crd, const long long
 // itself, so that after the system table the tasks, parameters and coordinates all arrive in one
 // round trip to memory: the set-up is latency, 4 us of a block's time with a barrier and a round
 // trip for each of them.
-template <typename T, bool CLASH>
+// PHASE, in an evaluation in parts: the pair phase also loads the atoms' Born-radius integrals, the
+// derivative phase their dE/dR and dR/dpsi.
+enum PartPhase : int { kPartPsi = 0, kPartPairs = 1, kPartDeriv = 2, kWhole = 3 };
+template <typename T, bool CLASH, int PHASE = kWhole>
 __device__ __forceinline__ void stage_load(StageCtx<T> &c, const MMKit &k) {
   WuLds<T> &L = c.L;
   const WuDesc &wu = c.wu;
@@ -189,6 +193,13 @@ __device__ __forceinline__ void stage_load(StageCtx<T> &c, const MMKit &k) {
     r.psi = 0;
     r.fx = r.fy = r.fz = 0;
     r.dedr = 0;
+    if (PHASE == kPartPairs && valid && c.gb) {
+      r.psi = k.part_psi[g];
+    }
+    if (PHASE == kPartDeriv && valid) {
+      r.psi = __double_as_longlong(k.part_drdpsi[g]);
+      r.dedr = k.part_dedr[g];
+    }
   }
   // The unit's tile tasks, read once per evaluation: the clean off-diagonal tasks of every
   // system, then their other off-diagonal tasks, then the diagonal ones, each with its system's
@@ -383,12 +394,14 @@ __device__ __forceinline__ Task wave_task(const StageCtx<T> &c, const MMKit &k, 
 // Work items of a stage are taken by the wavefronts of the block one at a time from a counter in
 // LDS, so a wavefront that finishes early takes more items (the result does not depend on which
 // wavefront took which item: every contribution goes to integer accumulators).
-__device__ __forceinline__ int next_item(int *counter, int lane) {
+// In an evaluation in parts a block takes every parts-th item.
+template <typename T>
+__device__ __forceinline__ int next_item(const StageCtx<T> &c, int counter, int lane) {
   int item = 0;
   if (lane == 0) {
-    item = atomicAdd(counter, 1);
+    item = atomicAdd(&c.L.work[counter], 1);
   }
-  return __builtin_amdgcn_readfirstlane(item);
+  return (__builtin_amdgcn_readfirstlane(item) * c.parts) + c.part;
 }
 
 // Item i of a stage holding `quads` tile-task quads and `chunks` chunks of 64 valence terms, the
@@ -590,7 +603,7 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
   const double psi_scale = ldexp(1.0, kPsiBits);
   const int quads = (c.wu.task_count + 3) >> 2;
   const int items = quads + val_chunks;
-  for (int item = next_item(&L.work[0], lane); item < items; item = next_item(&L.work[0], lane)) {
+  for (int item = next_item(c, 0, lane); item < items; item = next_item(c, 0, lane)) {
     const int it = stage_item(item, quads, val_chunks);
     if (it >= 0) {
       valence_chunk<T, FORCES, CLASH>(c, k, it, lane);
@@ -717,6 +730,9 @@ __device__ __forceinline__ void stage_radii(StageCtx<T> &c, const MMKit &k, doub
     const double atmq2h = 0.5 * qg * qg;
     const double atmqd2h = atmq2h * dielfac;
     const double contrib = -atmqd2h / R;
+    if (c.part != 0) {
+      continue;  // the unit's first part adds the self terms
+    }
     lds_add(&L.nrg[L.slot[a] * 16 + kGb], static_cast<long long>(__builtin_rint(contrib *
                                                                                   nrg_scale)));
     if (FORCES) {
@@ -806,7 +822,7 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
   const T dielfac0 = T(1) - inv_diel;
   // The steps leave out the 1/2 of the radius derivatives (a power of two: no rounding).
   const T dri_scale = T(0.5) * dedr_scale;
-  for (int t = row; t < c.wu.task_count; t += nrows) {
+  for (int t = row + (c.part * nrows); t < c.wu.task_count; t += nrows * c.parts) {
     const Task tk = fetch_task(c, k, t);
     const TileTask tt(tk, il);
     const unsigned emask = (tk.z >= 0 && tt.ivalid) ? k.masks[tk.z + il] : 0u;
@@ -1096,7 +1112,7 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
   int qn = 0;
   const T frc_scale = T(ldexp(1.0, k.frc_bits));
   const int quads = (c.wu.task_count + 3) >> 2;
-  for (int item = next_item(&L.work[1], lane); item < quads; item = next_item(&L.work[1], lane)) {
+  for (int item = next_item(c, 1, lane); item < quads; item = next_item(c, 1, lane)) {
     const TileTask tt(wave_task(c, k, (item << 2) + ((c.tid >> 4) & 3)), il);
     T xi, yi, zi, xj, yj, zj, si, sj;
     tile_coords(c, tt, xi, yi, zi, xj, yj, zj, si, sj);
@@ -1810,8 +1826,7 @@ template <typename T, bool FORCES, bool CLASH>
 __device__ __forceinline__ void stage_valence(StageCtx<T> &c, const MMKit &k) {
   const int lane = c.tid & 63;
   const int chunks = valence_chunks(c);
-  for (int item = next_item(&c.L.work[2], lane); item < chunks;
-       item = next_item(&c.L.work[2], lane)) {
+  for (int item = next_item(c, 2, lane); item < chunks; item = next_item(c, 2, lane)) {
     valence_chunk<T, FORCES, CLASH>(c, k, item, lane);
   }
   __syncthreads();
@@ -1843,13 +1858,31 @@ __device__ __forceinline__ void stage_restraints(StageCtx<T> &c, const MMKit &k)
   __syncthreads();
 }
 
+// The pair stage for the unit's Lennard-Jones form and solvent.
+template <typename T, bool FORCES, bool CLASH>
+__device__ __forceinline__ void evaluate_pairs(StageCtx<T> &c, const MMKit &k) {
+  if (c.wu.lj_table != 0) {
+    if (c.gb) {
+      stage_pairs<T, FORCES, true, true, CLASH>(c, k);
+    }
+    else {
+      stage_pairs<T, FORCES, true, false, CLASH>(c, k);
+    }
+  }
+  else if (c.gb) {
+    stage_pairs<T, FORCES, false, true, CLASH>(c, k);
+  }
+  else {
+    stage_pairs<T, FORCES, false, false, CLASH>(c, k);
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // One evaluation of the selected terms on the coordinates currently in global memory, leaving
 // forces (FORCES) and energies in the LDS accumulators.  RESTRAINTS = false leaves the restraint
 // stage out of the instantiation (for callers that never see restrained work units).
 template <typename T, bool FORCES, bool CLASH, bool RESTRAINTS = true>
 __device__ __forceinline__ void evaluate_wu(StageCtx<T> &c, const MMKit &k, int terms) {
-  const bool lj_table = (c.wu.lj_table != 0);
   stage_load<T, CLASH>(c, k);
   // With GB the valence terms ride along with the Born-integral tiles.
   const bool val = (terms & kTermValence) != 0;
@@ -1858,22 +1891,7 @@ __device__ __forceinline__ void evaluate_wu(StageCtx<T> &c, const MMKit &k, int 
     stage_radii<T, FORCES>(c, k, 0.0);
   }
   if (terms & kTermNonbonded) {
-    if (lj_table) {
-      if (c.gb) {
-        stage_pairs<T, FORCES, true, true, CLASH>(c, k);
-      }
-      else {
-        stage_pairs<T, FORCES, true, false, CLASH>(c, k);
-      }
-    }
-    else {
-      if (c.gb) {
-        stage_pairs<T, FORCES, false, true, CLASH>(c, k);
-      }
-      else {
-        stage_pairs<T, FORCES, false, false, CLASH>(c, k);
-      }
-    }
+    evaluate_pairs<T, FORCES, CLASH>(c, k);
   }
   if (FORCES && c.gb) {
     stage_chain<T>(c, k);

@@ -20,7 +20,7 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
 
 template <typename T, bool FORCES, bool CLASH>
 static hipError_t launch_eval_t(const MMKit &k, int terms, int eval_energy, hipStream_t stream) {
-  const int block = eval_block<T>(k);
+  const int block = eval_block<T>(k, k.nwu);
   const size_t lds = WuLds<T>::bytes(k.maxa, block / 64);
   auto fn = k_mm_eval<T, FORCES, CLASH>;
   hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),

@@ -433,6 +433,11 @@ __global__ void __launch_bounds__(64 * kLineWaves) k_line_advance(LineKit k, int
     return;
   }
   const int s = (k.slots != nullptr) ? k.slots[e] : e;
+  if (k.clear != nullptr) {
+    for (int i = lane; i < k.sys_natom[s]; i += 64) {
+      k.clear[k.sys_start[s] + i] = 0;
+    }
+  }
   if (k.done != nullptr && k.done[s] != 0) {
     return;
   }
@@ -528,7 +533,7 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
 template <typename T, bool FORCES, bool CLASH>
 static hipError_t launch_cycle_t(const MMKit &k, const CycleKit &ck, int pending_move,
                                  hipStream_t stream) {
-  const int block = eval_block<T>(k);
+  const int block = eval_block<T>(k, k.nwu);
   const size_t lds = WuLds<T>::bytes(k.maxa, block / 64);
   auto fn = k_min_cycle<T, FORCES, CLASH>;
   hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),

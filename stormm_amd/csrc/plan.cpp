@@ -8,6 +8,15 @@
 
 namespace stormm_amd {
 
+// An evaluation in parts, in the cost model's units: the least work worth a block, and when the
+// largest unit is worth it.  Measured with one unit to a compute unit, one block takes about
+// 6 us + cost / 54, the parts (three launches with a set-up each, and their radii computed in
+// every part) 25 us + share / 23; the line lies a little above where the two meet, since a
+// minimization's moves then take launches of their own.
+constexpr double kMinPartCost = 300.0;
+constexpr double kPartsFactor = 2.4;
+constexpr double kPartsOverhead = 1800.0;
+
 constexpr double kPi = 3.14159265358979323846264338327950288;
 
 // Per-type sigma and epsilon when the table follows Lorentz-Berthelot combining.
@@ -514,12 +523,73 @@ static void pack_lpt(const std::vector<double> &cost, const std::vector<int> &na
   }
 }
 
+// Units and their parts for a batch whose largest system would keep one compute unit busy long
+// after the others are done.  The systems above an even share of the work take units of their
+// own and as many blocks as they hold shares; the others are joined to units of about a share.
+// Returns false (nothing changed) where one block per unit is the better choice.
+static bool pack_parts(const std::vector<double> &cost, const std::vector<int> &natom,
+                       const std::vector<char> &table_mode, int cap, int cus,
+                       std::vector<std::vector<int>> &bins_out, std::vector<int> &mode_out,
+                       std::vector<WuPart> &parts) {
+  double total = 0.0, most = 0.0;
+  for (double c : cost) {
+    total += c;
+    most = std::max(most, c);
+  }
+  double share = std::max(total / cus, kMinPartCost);
+  std::vector<std::vector<int>> bins;
+  std::vector<int> modes;
+  std::vector<WuPart> blocks;
+  // The smallest share (in steps of a twentieth) whose blocks the device holds one to a compute
+  // unit: one block more would share its compute unit and end last.
+  for (; most > (kPartsFactor * share) + kPartsOverhead; share *= 1.05) {
+    double small = 0.0;
+    int large = 0;
+    for (double c : cost) {
+      if (c > share) {
+        large++;
+      }
+      else {
+        small += c;
+      }
+    }
+    const int units = large + static_cast<int>(std::ceil(small / share));
+    if (units > cus) {
+      continue;
+    }
+    pack_lpt(cost, natom, table_mode, cap, units, bins, modes);
+    blocks.clear();
+    for (size_t u = 0; u < bins.size(); u++) {
+      double c = 0.0;
+      for (int s : bins[u]) {
+        c += cost[s];
+      }
+      // Joined systems may exceed the share a little; only a large system is worth dividing.
+      const int n = (c > 1.5 * share) ? static_cast<int>(std::ceil(c / share)) : 1;
+      for (int p = 0; p < n; p++) {
+        blocks.push_back({static_cast<int>(u), p, n, 0});
+      }
+    }
+    if (static_cast<int>(blocks.size()) <= cus) {
+      bins_out = std::move(bins);
+      mode_out = std::move(modes);
+      parts = std::move(blocks);
+      return true;
+    }
+  }
+  return false;
+}
+
 void pack_systems(const std::vector<double> &cost, const std::vector<int> &natom,
                   const std::vector<char> &table_mode, int cap, int groups, int per_group,
                   bool grouped, std::vector<std::vector<int>> &bins_out,
-                  std::vector<int> &mode_out) {
+                  std::vector<int> &mode_out, std::vector<WuPart> &parts) {
   groups = std::max(1, groups);
   per_group = std::max(1, per_group);
+  parts.clear();
+  if (pack_parts(cost, natom, table_mode, cap, groups, bins_out, mode_out, parts)) {
+    return;
+  }
   if (!grouped ||
       !pack_grouped(cost, natom, table_mode, cap, groups, per_group, bins_out, mode_out)) {
     pack_lpt(cost, natom, table_mode, cap, groups * per_group, bins_out, mode_out);
@@ -971,7 +1041,8 @@ int build_plan(const stormm_topology_batch *b, const stormm_launch_shape *shape_
   }
   std::vector<std::vector<int>> bins;
   std::vector<int> bin_mode;
-  pack_systems(cost, P.atom_counts, P.lj_table_mode, cap, cus, wu_per_cu, true, bins, bin_mode);
+  pack_systems(cost, P.atom_counts, P.lj_table_mode, cap, cus, wu_per_cu, true, bins, bin_mode,
+               P.parts);
   P.maxa = 0;
   for (size_t u = 0; u < bins.size(); u++) {
     P.maxa = std::max(P.maxa, append_work_unit(bins[u], bin_mode[u], sys_index, P.atom_starts,

@@ -108,6 +108,7 @@ struct SynthesisPlan {
   std::vector<int> sys_template;
   std::vector<WuDesc> wu;
   std::vector<WuSys> wu_sys;
+  std::vector<WuPart> parts;  // blocks of an evaluation in parts (empty: one block per unit)
   long long pairs = 0;
   long long task_count = 0;
   long long vterm_count = 0;
@@ -140,7 +141,7 @@ int fill_atom_parameters(const stormm_topology_batch *b, const SystemTerms &t, i
 void pack_systems(const std::vector<double> &cost, const std::vector<int> &natom,
                   const std::vector<char> &table_mode, int cap, int groups, int per_group,
                   bool grouped, std::vector<std::vector<int>> &bins_out,
-                  std::vector<int> &mode_out);
+                  std::vector<int> &mode_out, std::vector<WuPart> &parts);
 
 // Appends one work unit holding `systems` (indices into the per-system arrays); returns its
 // LDS atom count.  `sys_index` gives each system's number in the kernels' per-system arrays;

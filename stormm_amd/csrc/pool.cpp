@@ -27,7 +27,8 @@ using namespace stormm_amd;
 namespace {
 
 // Device bytes counted per resident atom: int64 coordinates, forces, previous forces and CG
-// direction (12 x 8), nine doubles (five parameters and room for four) and the LJ type.
+// direction (12 x 8), nine 8-byte values (five parameters, the three sums of evaluations in parts
+// and room for one) and the LJ type.
 constexpr size_t kPoolBytesPerAtom = (12 * 8) + (9 * 8) + 4;
 // Device bytes per system slot: layout (2 ints), step / stop flag (2 ints), RMS force, nine
 // line-search doubles and a ScoreCard row.
@@ -85,6 +86,9 @@ struct stormm_pool {
   // Device state.
   DevMem xcrd, ycrd, zcrd, xfrc, yfrc, zfrc, xprv, yprv, zprv, xcg, ycg, zcg;
   DevMem q, ljp1, ljp2, rho, scr, lj_type;
+  // Per-atom sums of evaluations in parts (the integrals zero at rest unless part_dirty).
+  DevMem part_psi, part_dedr, part_drdpsi, parts;
+  bool part_dirty = false;
   DevMem starts, natoms, steps, done, rms, line, scorecard, status;
   // Energy history per slot: hist_len ScoreCard rows, one every cfg.minimize.
   // diagnostic_print_frequency cycles (none when that is 0).
@@ -171,6 +175,10 @@ extern "C" int stormm_pool_create(const stormm_pool_config *cfg, stormm_pool **o
   }
   for (DevMem *d : {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr}) {
     HIP_TRY(d->alloc(na * sizeof(double)));
+  }
+  for (DevMem *d : {&p->part_psi, &p->part_dedr, &p->part_drdpsi}) {
+    HIP_TRY(d->alloc(na * sizeof(long long)));
+    HIP_TRY(hipMemset(d->ptr, 0, na * sizeof(long long)));
   }
   HIP_TRY(p->lj_type.alloc(na * sizeof(int)));
   HIP_TRY(p->starts.alloc(ns * sizeof(int)));
@@ -687,9 +695,10 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
   const int block = std::max(sh.block_threads, 0);
   std::vector<std::vector<int>> bins;
   std::vector<int> modes;
+  std::vector<WuPart> parts;
   // The resident set changes every call; balancing units one by one (largest first) serves
   // these short launches better than the compute-unit groups of the batch synthesis.
-  pack_systems(cost, natom, table, cap, p->cus, per_cu, false, bins, modes);
+  pack_systems(cost, natom, table, cap, p->cus, per_cu, false, bins, modes, parts);
   std::vector<WuDesc> wu;
   std::vector<WuSys> wu_sys;
   int maxa = 0;
@@ -701,13 +710,19 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
                                            std::to_string(kMaxWuTasks) + " tile tasks");
     }
   }
+  const size_t part_bytes = parts.size() * sizeof(WuPart);
   const size_t wu_bytes = wu.size() * sizeof(WuDesc);
   const size_t wu_sys_bytes = wu_sys.size() * sizeof(WuSys);
   const size_t act_bytes = act.size() * sizeof(int);
   WuDesc *d_wu;
   WuSys *d_wu_sys;
   int *d_active;
+  WuPart *d_parts;
   if (staging.base == nullptr) {
+    if (p->parts.bytes < part_bytes) {
+      HIP_TRY(p->parts.alloc(2 * part_bytes));
+    }
+    d_parts = p->parts.as<WuPart>();
     if (p->wu.bytes < wu_bytes) {
       HIP_TRY(p->wu.alloc(2 * wu_bytes));
     }
@@ -719,7 +734,8 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
     d_active = p->active.as<int>();
   }
   else {
-    const size_t need = align256(wu_bytes) + align256(wu_sys_bytes) + align256(act_bytes);
+    const size_t need = align256(wu_bytes) + align256(wu_sys_bytes) + align256(act_bytes) +
+                        align256(part_bytes);
     if (need > staging.bytes) {
       return fail(STORMM_ERR_CAPACITY,
                   "the call's work units need " + std::to_string(need) + " bytes of staging (" +
@@ -731,12 +747,24 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
     d_wu = reinterpret_cast<WuDesc *>(b);
     d_wu_sys = reinterpret_cast<WuSys *>(b + align256(wu_bytes));
     d_active = reinterpret_cast<int *>(b + align256(wu_bytes) + align256(wu_sys_bytes));
+    d_parts = reinterpret_cast<WuPart *>(b + align256(wu_bytes) + align256(wu_sys_bytes) +
+                                         align256(act_bytes));
   }
   HIP_TRY(hipMemcpy(d_wu, wu.data(), wu_bytes, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_wu_sys, wu_sys.data(), wu_sys_bytes, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_active, act.data(), act_bytes, hipMemcpyHostToDevice));
+  if (!parts.empty()) {
+    HIP_TRY(hipMemcpy(d_parts, parts.data(), part_bytes, hipMemcpyHostToDevice));
+  }
   const int prec = (p->cfg.precision == STORMM_PREC_DOUBLE) ? 0 : 1;
-  const MMKit mm = pool_mm_kit(p, static_cast<int>(wu.size()), maxa, block, d_wu, d_wu_sys);
+  MMKit mm = pool_mm_kit(p, static_cast<int>(wu.size()), maxa, block, d_wu, d_wu_sys);
+  if (!parts.empty()) {
+    mm.nparts = static_cast<int>(parts.size());
+    mm.parts = d_parts;
+    mm.part_psi = p->part_psi.as<long long>();
+    mm.part_dedr = p->part_dedr.as<long long>();
+    mm.part_drdpsi = p->part_drdpsi.as<double>();
+  }
   CgKit cg;
   std::memset(&cg, 0, sizeof(cg));
   cg.nsys = na;
@@ -802,6 +830,8 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
   lk.nrg_c = v + 7 * n;
   lk.nrg_d = v + 8 * n;
   lk.dp_mode = cg.dp_mode;
+  // Each line move clears the Born-radius integrals that an evaluation in parts left.
+  lk.clear = mm.part_psi;
   const int terms = kTermNonbonded | kTermValence;
   const int sd = p->cfg.minimize.steepest_descent_cycles;
   // Clash damping follows each system's own cycle count (hpc_minimization.cu:269-281): the
@@ -821,19 +851,37 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
   // The reference's per-cycle sequence (src/MolecularMechanics/hpc_minimization.cu:262-405):
   // force + energy evaluation, conjugate-gradient direction, then four line moves separated by
   // energy evaluations.  Stores overwrite, so no force or ScoreCard zeroing is launched.
+  auto evaluate = [&](const MMKit &k, int force) {
+    return (k.nparts > 0) ? launch_mm_parts(prec, k, terms, force, 1, st)
+                          : launch_mm_eval(prec, k, terms, force, 1, st);
+  };
+  auto clear_sums = [&]() {
+    return launch_fill(p->part_psi.as<long long>(), nullptr, nullptr,
+                       static_cast<size_t>(p->cap_atoms), st);
+  };
+  if (mm.nparts > 0) {
+    if (p->part_dirty) {
+      HIP_TRY(clear_sums());
+    }
+    p->part_dirty = true;
+  }
   for (int c = 0; c < cycles; c++) {
     const bool damp = (min_step + c < cdcyc);
-    HIP_TRY(launch_mm_eval(prec, damp ? mf_clash : mm, terms, 1, 1, st));
+    HIP_TRY(evaluate(damp ? mf_clash : mm, 1));
     HIP_TRY(launch_conjugate_gradient(cg, 0, sd, st));
     for (int move = 0; move < 4; move++) {
       if (move > 0) {
-        HIP_TRY(launch_mm_eval(prec, damp ? me_clash : mm, terms, 0, 1, st));
+        HIP_TRY(evaluate(damp ? me_clash : mm, 0));
       }
       HIP_TRY(launch_line_advance(lk, move, st));
     }
   }
   // Energies at the coordinates the call leaves.
-  HIP_TRY(launch_mm_eval(prec, mm, terms, 0, 1, st));
+  HIP_TRY(evaluate(mm, 0));
+  if (mm.nparts > 0) {
+    HIP_TRY(clear_sums());
+    p->part_dirty = false;
+  }
   if (staging.base != nullptr) {
     // The staging region is shared by every call on the device: it must not be rewritten
     // before this call's kernels have read it.

@@ -46,7 +46,7 @@ struct stormm_synthesis {
   SynthesisPlan plan;
   DevMem atom_starts, atom_counts, q, ljp1, ljp2, lj_type, ljab, ljab14, rho, scr,
       wu, wu_sys, tasks, masks, vterms, bond_par, angl_par, dihe_par,
-      dihe14, status, cycles_run, rms_force, stop_flags, rst;
+      dihe14, status, cycles_run, rms_force, stop_flags, rst, parts;
   MMKit kit;
 };
 
@@ -57,6 +57,14 @@ struct stormm_phasespace {
   // Overflow words of the same arrays (value = ovrf 2^63 + word above the plain limits).
   DevMem xcrd_o, ycrd_o, zcrd_o, xfrc_o, yfrc_o, zfrc_o, xprv_o, yprv_o, zprv_o, xcg_o, ycg_o,
       zcg_o;
+  // Per-atom sums of a force evaluation in parts.  They belong to the phase space because such an
+  // evaluation already owns its force arrays: two of them on one phase space at a time would race
+  // on the forces.  Energy-only evaluations, which may run side by side on different streams with
+  // their own ScoreCards, use one block per unit (a minimization, which moves the coordinates,
+  // owns the phase space and runs both kinds in parts).
+  DevMem part_psi, part_dedr, part_drdpsi;
+  // The integrals may not be zero: a launch sequence that should have cleared them failed.
+  bool part_dirty = false;
 };
 
 struct stormm_scorecard {
@@ -154,6 +162,7 @@ extern "C" int stormm_synthesis_create(const stormm_topology_batch *batch,
   HIP_TRY(ag->dihe_par.upload(P.ts.dihe_par));
   HIP_TRY(ag->dihe14.upload(P.ts.dihe14));
   HIP_TRY(ag->rst.upload(P.rst));
+  HIP_TRY(ag->parts.upload(P.parts));
   std::vector<int> zero_status(1, 0);
   HIP_TRY(ag->status.upload(zero_status));
   std::vector<int> zi(P.nsys, 0);
@@ -195,6 +204,7 @@ extern "C" int stormm_synthesis_create(const stormm_topology_batch *batch,
   k.gb_gamma = P.sm.gamma;
   k.status = ag->status.as<int>();
   k.rst = ag->rst.as<stormm_restraint>();
+  k.parts = ag->parts.as<WuPart>();
   *out = ag.release();
   return STORMM_OK;
 }
@@ -284,6 +294,12 @@ extern "C" int stormm_phasespace_create(const stormm_synthesis *ag, int32_t gpos
   for (DevMem *d : ovrf) {
     HIP_TRY(d->alloc(na * sizeof(int)));
     HIP_TRY(hipMemset(d->ptr, 0, na * sizeof(int)));
+  }
+  if (!ag->plan.parts.empty() && ag->plan.sm.igb != 0) {
+    for (DevMem *d : {&ps->part_psi, &ps->part_dedr, &ps->part_drdpsi}) {
+      HIP_TRY(d->alloc(na * sizeof(long long)));
+      HIP_TRY(hipMemset(d->ptr, 0, na * sizeof(long long)));
+    }
   }
   *out = ps.release();
   return STORMM_OK;
@@ -1234,7 +1250,38 @@ static MMKit make_kit(const stormm_synthesis *ag, const stormm_ps_writer &w, con
   k.rst_cycle_offset = 0;
   k.rst_move = 0;
   k.rst_clash_cycles = 0;
+  k.nparts = 0;
   return k;
+}
+
+// Turns the kit to the evaluation in parts when the synthesis has parts and a phase-space handle
+// (null: caller-owned arrays) lends its per-atom sums.  Returns whether it did.
+static bool use_parts(MMKit &k, const stormm_synthesis *ag, stormm_phasespace *ps) {
+  if (ps == nullptr || ag->plan.parts.empty() || wide_forces(ps)) {
+    return false;
+  }
+  k.nparts = static_cast<int>(ag->plan.parts.size());
+  k.part_psi = ps->part_psi.as<long long>();
+  k.part_dedr = ps->part_dedr.as<long long>();
+  k.part_drdpsi = ps->part_drdpsi.as<double>();
+  return true;
+}
+
+// Zeroes the Born-radius integrals of an evaluation in parts (nothing without GB).
+static hipError_t clear_part_sums(const MMKit &k, const stormm_synthesis *ag,
+                                  hipStream_t stream) {
+  return (k.part_psi != nullptr)
+             ? launch_fill(k.part_psi, nullptr, nullptr,
+                           static_cast<size_t>(ag->plan.padded_atoms), stream)
+             : hipSuccess;
+}
+
+// One evaluation with the kit's blocks.
+static hipError_t launch_eval(int precision, const MMKit &k, int terms, int eval_force,
+                              int eval_energy, hipStream_t stream) {
+  return (k.nparts > 0)
+             ? launch_mm_parts(precision, k, terms, eval_force, eval_energy, stream)
+             : launch_mm_eval(precision, k, terms, eval_force, eval_energy, stream);
 }
 
 // Whether the damped kernels run for clash parameters (d, r): the reference launches them when
@@ -1280,10 +1327,29 @@ static int check_mincon(const stormm_minimize_controls *mc) {
   return STORMM_OK;
 }
 
+// An evaluation on caller-owned arrays (ps null) or a phase space's own: force evaluations of the
+// non-bonded terms run in parts where the synthesis has them.
+static hipError_t launch_eval_on(stormm_phasespace *ps, const stormm_synthesis *ag, int precision,
+                                 MMKit k, int terms, int eval_force, int eval_energy,
+                                 hipStream_t stream) {
+  if (!eval_force || (terms & kTermNonbonded) == 0 || !use_parts(k, ag, ps)) {
+    return launch_mm_eval(precision, k, terms, eval_force, eval_energy, stream);
+  }
+  hipError_t err = ps->part_dirty ? clear_part_sums(k, ag, stream) : hipSuccess;
+  if (err == hipSuccess) {
+    ps->part_dirty = true;
+    err = launch_mm_parts(precision, k, terms, eval_force, eval_energy, stream);
+  }
+  if (err == hipSuccess) {
+    ps->part_dirty = false;
+  }
+  return err;
+}
+
 static int launch_terms(int32_t precision, const stormm_synthesis *ag,
                         const stormm_ps_writer &w, const ScView &sc, int terms,
                         int32_t eval_force, int32_t eval_energy, double clash_d, double clash_r,
-                        int step, void *stream) {
+                        int step, stormm_phasespace *ps, void *stream) {
   int rc = check_writer(ag, &w, precision, &sc, false);
   if (rc != STORMM_OK) {
     return rc;
@@ -1297,8 +1363,9 @@ static int launch_terms(int32_t precision, const stormm_synthesis *ag,
   MMKit k = make_kit(ag, w, &sc);
   set_clash(k, precision, clash_d, clash_r);
   k.rst_step = step;
-  HIP_TRY(launch_mm_eval(precision == STORMM_PREC_DOUBLE ? 0 : 1, k, terms, eval_force ? 1 : 0,
-                         eval_energy ? 1 : 0, static_cast<hipStream_t>(stream)));
+  HIP_TRY(launch_eval_on(ps, ag, precision == STORMM_PREC_DOUBLE ? 0 : 1, k, terms,
+                         eval_force ? 1 : 0, eval_energy ? 1 : 0,
+                         static_cast<hipStream_t>(stream)));
   return STORMM_OK;
 }
 
@@ -1314,7 +1381,7 @@ static int launch_terms_handles(int32_t precision, const stormm_synthesis *ag,
   stormm_ps_writer w;
   stormm_phasespace_writer(ps, &w);
   return launch_terms(precision, ag, w, sc_view(sc), terms, eval_force, eval_energy, clash_d,
-                      clash_r, (ctrl != nullptr) ? ctrl->step : 0, stream);
+                      clash_r, (ctrl != nullptr) ? ctrl->step : 0, ps, stream);
 }
 
 static int launch_terms_kit(int32_t precision, const stormm_synthesis *ag,
@@ -1330,7 +1397,7 @@ static int launch_terms_kit(int32_t precision, const stormm_synthesis *ag,
     return fail(STORMM_ERR_INVALID_ARGUMENT, "null phase-space writer");
   }
   return launch_terms(precision, ag, *psw, sc, terms, eval_force, eval_energy, clash_d, clash_r,
-                      (ctrl != nullptr) ? ctrl->step : 0, stream);
+                      (ctrl != nullptr) ? ctrl->step : 0, nullptr, stream);
 }
 
 extern "C" int stormm_launch_nonbonded(int32_t precision, const stormm_synthesis *ag,
@@ -1559,7 +1626,8 @@ extern "C" int stormm_launch_line_advance_kit(int32_t precision, const stormm_sy
 // evaluation per energy point.
 static int minimize_stepwise(int32_t precision, const stormm_synthesis *ag,
                              const stormm_ps_writer &w, const stormm_minimize_controls *mc,
-                             const ScView &sc, const LmView &lm, hipStream_t stream) {
+                             const ScView &sc, const LmView &lm, stormm_phasespace *ps,
+                             hipStream_t stream) {
   // The reference's per-cycle launch sequence (src/MolecularMechanics/hpc_minimization.cu:
   // 262-405).  The evaluations overwrite the force arrays and ScoreCard rows, which stands in
   // for the force and ScoreCard zeroing launches that precede them there.
@@ -1571,6 +1639,12 @@ static int minimize_stepwise(int32_t precision, const stormm_synthesis *ag,
   const int prec = (precision == STORMM_PREC_DOUBLE) ? 0 : 1;
   MMKit k = make_kit(ag, w, &sc);
   k.store_overwrite = 1;
+  LineKit lk = make_line_kit(ag, w, sc, lm, precision);
+  if (use_parts(k, ag, ps)) {
+    // The line move after each evaluation clears the Born-radius integrals for the next one.
+    lk.clear = k.part_psi;
+    HIP_TRY(clear_part_sums(k, ag, stream));
+  }
   CgKit cg = make_cg_kit(ag, w, precision);
   cg.hist = sc.hist;
   const int terms = kTermNonbonded | kTermValence;
@@ -1585,22 +1659,21 @@ static int minimize_stepwise(int32_t precision, const stormm_synthesis *ag,
     }
     set_clash(k, precision, cd, cr);
     k.rst_step = minimizer_step(cyc, 0, cdcyc);
-    HIP_TRY(launch_mm_eval(prec, k, terms, 1, 1, stream));
+    HIP_TRY(launch_eval(prec, k, terms, 1, 1, stream));
     step += 1;
     HIP_TRY(launch_conjugate_gradient(cg, step, mc->steepest_descent_cycles, stream));
     for (int move = 0; move < 4; move++) {
       if (move > 0) {
         k.rst_step = minimizer_step(cyc, move, cdcyc);
-        HIP_TRY(launch_mm_eval(prec, k, terms, 0, 1, stream));
+        HIP_TRY(launch_eval(prec, k, terms, 0, 1, stream));
       }
-      if ((rc = line_advance(precision, ag, w, sc, lm, move, stream)) != STORMM_OK) {
-        return rc;
-      }
+      HIP_TRY(launch_line_advance(lk, move, stream));
     }
   }
   set_clash(k, precision, 0.0, 0.0);
   k.rst_step = minimizer_step(mc->total_cycles, 1, cdcyc);
-  HIP_TRY(launch_mm_eval(prec, k, terms, 0, 1, stream));
+  HIP_TRY(launch_eval(prec, k, terms, 0, 1, stream));
+  HIP_TRY(clear_part_sums(k, ag, stream));
   return STORMM_OK;
 }
 
@@ -1618,13 +1691,13 @@ static hipError_t capture_cycle(int prec, const MMKit &kf, const MMKit *ke, cons
   if (err != hipSuccess) {
     return err;
   }
-  hipError_t e2 = launch_mm_eval(prec, kf, terms, 1, 1, cap);
+  hipError_t e2 = launch_eval(prec, kf, terms, 1, 1, cap);
   if (e2 == hipSuccess) {
     e2 = launch_conjugate_gradient(cg, 0, sd, cap);
   }
   for (int move = 0; move < 4 && e2 == hipSuccess; move++) {
     if (move > 0) {
-      e2 = launch_mm_eval(prec, ke[move - 1], terms, 0, 1, cap);
+      e2 = launch_eval(prec, ke[move - 1], terms, 0, 1, cap);
     }
     if (e2 == hipSuccess) {
       e2 = launch_line_advance(lk, move, cap);
@@ -1642,7 +1715,8 @@ static hipError_t capture_cycle(int prec, const MMKit &kf, const MMKit *ke, cons
 
 static int minimize_graph(int32_t precision, const stormm_synthesis *ag_c,
                           const stormm_ps_writer &w, const stormm_minimize_controls *mc,
-                          const ScView &sc, const LmView &lm, hipStream_t stream) {
+                          const ScView &sc, const LmView &lm, stormm_phasespace *ps,
+                          hipStream_t stream) {
   stormm_synthesis *ag = const_cast<stormm_synthesis *>(ag_c);
   int rc = stormm_ps_writer_prime_conjugate_gradient(&w, ag->plan.padded_atoms, stream);
   if (rc != STORMM_OK) {
@@ -1665,6 +1739,10 @@ static int minimize_graph(int32_t precision, const stormm_synthesis *ag_c,
   cg.max_steps = mc->total_cycles;
   LineKit lk = make_line_kit(ag, w, sc, lm, precision);
   lk.done = ag->stop_flags.as<int>();
+  if (use_parts(k, ag, ps)) {
+    lk.clear = k.part_psi;
+    HIP_TRY(clear_part_sums(k, ag, stream));
+  }
   const int terms = kTermNonbonded | kTermValence;
   const int sd = mc->steepest_descent_cycles;
   const int cdcyc = std::min(mc->clash_damping_cycles, mc->total_cycles);
@@ -1709,7 +1787,10 @@ static int minimize_graph(int32_t precision, const stormm_synthesis *ag_c,
     MMKit kfin = k;
     kfin.rst_step_sys = nullptr;
     kfin.rst_step = minimizer_step(mc->total_cycles, 1, cdcyc);
-    err = launch_mm_eval(prec, kfin, terms, 0, 1, stream);
+    err = launch_eval(prec, kfin, terms, 0, 1, stream);
+  }
+  if (err == hipSuccess) {
+    err = clear_part_sums(k, ag, stream);
   }
   if (err == hipSuccess) {
     err = hipStreamSynchronize(stream);
@@ -1747,8 +1828,27 @@ enum class FusedIssue {
 // Launches of one fused cycle: the force evaluation (making the previous cycle's last line move
 // first), the conjugate-gradient update, and three energy evaluations, each making the line move
 // that follows the evaluation before it.
+//
+// Evaluations in parts make no moves: their cycle is the per-step sequence, each line move in a
+// launch of its own that also clears the parts' Born-radius integrals.
 static hipError_t launch_fused_cycle(int prec, const MMKit &kf, const MMKit &ke,
                                      const CycleKit &ck, int sd_cycles, hipStream_t st) {
+  if (kf.nparts > 0) {
+    const int terms = kTermNonbonded | kTermValence;
+    hipError_t err = launch_mm_parts(prec, kf, terms, 1, 1, st);
+    if (err == hipSuccess) {
+      err = launch_conjugate_gradient(ck.cg, 0, sd_cycles, st);
+    }
+    for (int move = 0; move < 4 && err == hipSuccess; move++) {
+      if (move > 0) {
+        err = launch_mm_parts(prec, ke, terms, 0, 1, st);
+      }
+      if (err == hipSuccess) {
+        err = launch_line_advance(ck.line, move, st);
+      }
+    }
+    return err;
+  }
   hipError_t err = launch_min_cycle(prec, kf, ck, true, 3, st);
   if (err == hipSuccess) {
     err = launch_conjugate_gradient(ck.cg, 0, sd_cycles, st);
@@ -1785,7 +1885,7 @@ static hipError_t capture_fused_cycle(int prec, const MMKit &kf, const MMKit &ke
 static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
                           const stormm_ps_writer &w, const stormm_minimize_controls *mc,
                           const ScView &sc, const LmView &lm, const CycleState &cs,
-                          hipStream_t stream, FusedIssue how) {
+                          stormm_phasespace *ps, hipStream_t stream, FusedIssue how) {
   if (!ag->plan.rst.empty()) {
     return fail(STORMM_ERR_STATE, "the fused-cycle minimizer does not evaluate restraints; "
                                   "minimize a restrained synthesis with the per-step (0) or "
@@ -1810,6 +1910,10 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
   ck.cg.max_steps = mc->total_cycles;
   ck.line = make_line_kit(ag, w, sc, lm, precision);
   ck.line.done = cs.done;
+  const bool in_parts = use_parts(k, ag, ps);
+  if (in_parts) {
+    ck.line.clear = k.part_psi;
+  }
   const int sd = mc->steepest_descent_cycles;
   const int cdcyc = std::min(mc->clash_damping_cycles, mc->total_cycles);
   // Damped evaluations read the cycle count before this cycle's direction update advances it
@@ -1849,6 +1953,9 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
     err = launch_fill(reinterpret_cast<long long *>(cs.rms), nullptr, nullptr,
                       static_cast<size_t>(ns), issue);
   }
+  if (err == hipSuccess && in_parts) {
+    err = clear_part_sums(k, ag, issue);
+  }
   if (how == FusedIssue::kCycleGraph) {
     if (err == hipSuccess) {
       err = capture_fused_cycle(prec, k, k, ck, sd, cap, &graph[0], &exec[0]);
@@ -1868,8 +1975,11 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
   }
   if (err == hipSuccess) {
     // The final energies, after the last cycle's last move.
-    err = (mc->total_cycles > 0) ? launch_min_cycle(prec, kfin, ck, false, 3, issue)
-                                 : launch_mm_eval(prec, kfin, terms, 0, 1, issue);
+    err = (mc->total_cycles > 0 && !in_parts) ? launch_min_cycle(prec, kfin, ck, false, 3, issue)
+                                              : launch_eval(prec, kfin, terms, 0, 1, issue);
+  }
+  if (err == hipSuccess && in_parts) {
+    err = clear_part_sums(k, ag, issue);
   }
   if (how == FusedIssue::kWholeGraph) {
     const hipError_t e1 = hipStreamEndCapture(cap, &graph[0]);
@@ -1903,7 +2013,7 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
 
 static int minimize(int32_t precision, const stormm_synthesis *ag, const stormm_ps_writer &w,
                     const stormm_minimize_controls *mincon, const ScView &sc, const LmView &lm,
-                    int32_t persistent, void *stream) {
+                    int32_t persistent, stormm_phasespace *ps, void *stream) {
   int rc = check_writer(ag, &w, precision, &sc, true);
   if (rc != STORMM_OK) {
     return rc;
@@ -1924,11 +2034,14 @@ static int minimize(int32_t precision, const stormm_synthesis *ag, const stormm_
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   stormm_synthesis *agm = const_cast<stormm_synthesis *>(ag);
+  if (ps != nullptr) {
+    ps->part_dirty = true;
+  }
   if (persistent == 0) {
-    rc = minimize_stepwise(precision, ag, w, mincon, sch, lm, st);
+    rc = minimize_stepwise(precision, ag, w, mincon, sch, lm, ps, st);
   }
   else if (persistent == 2) {
-    rc = minimize_graph(precision, ag, w, mincon, sch, lm, st);
+    rc = minimize_graph(precision, ag, w, mincon, sch, lm, ps, st);
   }
   else {
     CycleState cs;
@@ -1937,7 +2050,10 @@ static int minimize(int32_t precision, const stormm_synthesis *ag, const stormm_
     cs.rms = agm->rms_force.as<double>();
     const FusedIssue how = (persistent == 1) ? FusedIssue::kWholeGraph :
                            (persistent == 3) ? FusedIssue::kCycleGraph : FusedIssue::kDirect;
-    rc = minimize_fused(precision, ag, w, mincon, sch, lm, cs, st, how);
+    rc = minimize_fused(precision, ag, w, mincon, sch, lm, cs, ps, st, how);
+  }
+  if (rc == STORMM_OK && ps != nullptr) {
+    ps->part_dirty = false;
   }
   if (rc == STORMM_OK) {
     rc = finish_history(mincon, sch, (persistent == 0) ? nullptr : agm->cycles_run.as<int>(),
@@ -1964,7 +2080,8 @@ extern "C" int stormm_launch_minimization(int32_t precision, const stormm_synthe
   }
   stormm_ps_writer w;
   stormm_phasespace_writer(ps, &w);
-  return minimize(precision, ag, w, mincon, sc_view(sc), lm_view(lm), persistent, stream);
+  return minimize(precision, ag, w, mincon, sc_view(sc), lm_view(lm), persistent, ps,
+                  stream);
 }
 
 extern "C" int stormm_launch_minimization_kit(int32_t precision, const stormm_synthesis *ag,
@@ -1985,7 +2102,7 @@ extern "C" int stormm_launch_minimization_kit(int32_t precision, const stormm_sy
   if (rc != STORMM_OK) {
     return rc;
   }
-  return minimize(precision, ag, *psw, mincon, sc, lm, persistent, stream);
+  return minimize(precision, ag, *psw, mincon, sc, lm, persistent, nullptr, stream);
 }
 
 // The fused-cycle minimizer on caller-owned arrays with its per-system state in the library's
@@ -2037,7 +2154,7 @@ extern "C" int stormm_launch_minimization_kit_noalloc(int32_t precision,
   cs.rms = reinterpret_cast<double *>(static_cast<unsigned char *>(base) +
                                       (static_cast<size_t>(kNoAllocMaxSystems) * 8));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  rc = minimize_fused(precision, ag, *psw, mincon, sc, lm, cs, st, FusedIssue::kDirect);
+  rc = minimize_fused(precision, ag, *psw, mincon, sc, lm, cs, nullptr, st, FusedIssue::kDirect);
   if (rc == STORMM_OK) {
     rc = finish_history(mincon, sc, cs.steps, st);
   }
@@ -2138,7 +2255,7 @@ extern "C" int stormm_time_launch(int32_t precision, const stormm_synthesis *ag,
   const int prec = (precision == STORMM_PREC_DOUBLE) ? 0 : 1;
   HIP_TRY(hipEventRecord(e0, st));
   for (int r = 0; r < repeats; r++) {
-    HIP_TRY(launch_mm_eval(prec, k, terms, eval_force, 1, st));
+    HIP_TRY(launch_eval_on(ps, ag, prec, k, terms, eval_force, 1, st));
   }
   HIP_TRY(hipEventRecord(e1, st));
   HIP_TRY(hipEventSynchronize(e1));
