@@ -1821,9 +1821,15 @@ struct CycleState {
 // How the fused cycle kernels are issued.
 enum class FusedIssue {
   kDirect,      // launched one by one on the caller's stream; the call returns at once
-  kWholeGraph,  // the whole run captured in one HIP graph, launched once; returns when done
+  kChunkGraph,  // the damped and first cycles one by one, the rest as replays of a HIP graph of
+                // kChunkCycles cycles captured meanwhile; returns when done
   kCycleGraph   // one cycle captured (plus a clash-damped one) and replayed; returns when done
 };
+
+// Cycles of a chunk graph.  Capturing and instantiating a graph costs the host 6 us a kernel, all
+// of it before the first kernel starts when the whole run is captured (0.65 ms of a 3.2 ms run of
+// 20 cycles); one chunk is captured while the device runs at least as many cycles issued directly.
+constexpr int kChunkCycles = 8;
 
 // Launches of one fused cycle: the force evaluation (making the previous cycle's last line move
 // first), the conjugate-gradient update, and three energy evaluations, each making the line move
@@ -1859,15 +1865,18 @@ static hipError_t launch_fused_cycle(int prec, const MMKit &kf, const MMKit &ke,
   return err;
 }
 
-// Captures one fused cycle into an executable graph.
+// Captures `cycles` fused cycles into an executable graph.
 static hipError_t capture_fused_cycle(int prec, const MMKit &kf, const MMKit &ke,
-                                      const CycleKit &ck, int sd_cycles, hipStream_t cap,
-                                      hipGraph_t *graph, hipGraphExec_t *exec) {
+                                      const CycleKit &ck, int sd_cycles, int cycles,
+                                      hipStream_t cap, hipGraph_t *graph, hipGraphExec_t *exec) {
   hipError_t err = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
   if (err != hipSuccess) {
     return err;
   }
-  const hipError_t e2 = launch_fused_cycle(prec, kf, ke, ck, sd_cycles, cap);
+  hipError_t e2 = hipSuccess;
+  for (int c = 0; c < cycles && e2 == hipSuccess; c++) {
+    e2 = launch_fused_cycle(prec, kf, ke, ck, sd_cycles, cap);
+  }
   err = hipStreamEndCapture(cap, graph);
   if (err == hipSuccess) {
     err = e2;
@@ -1933,35 +1942,32 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
   hipStream_t cap = nullptr;
   hipGraph_t graph[2] = {nullptr, nullptr};
   hipGraphExec_t exec[2] = {nullptr, nullptr};
-  hipStream_t issue = stream;
   hipError_t err = hipSuccess;
-  if (how != FusedIssue::kDirect) {
+  // Cycles issued one by one before the chunks.
+  const int lead = std::max(cdcyc, kChunkCycles);
+  const int chunks = (how == FusedIssue::kChunkGraph && mc->total_cycles >= lead + 2 * kChunkCycles)
+                         ? (mc->total_cycles - lead) / kChunkCycles : 0;
+  if (how == FusedIssue::kCycleGraph || chunks > 0) {
     HIP_TRY(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
   }
-  if (how == FusedIssue::kWholeGraph) {
-    err = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
-    issue = cap;
-  }
+  err = (stormm_ps_writer_prime_conjugate_gradient(&w, ag->plan.padded_atoms, stream) ==
+         STORMM_OK) ? hipSuccess : hipErrorInvalidValue;
   if (err == hipSuccess) {
-    err = (stormm_ps_writer_prime_conjugate_gradient(&w, ag->plan.padded_atoms, issue) ==
-           STORMM_OK) ? hipSuccess : hipErrorInvalidValue;
-  }
-  if (err == hipSuccess) {
-    err = launch_fill_int(cs.steps, cs.done, cs.done, static_cast<size_t>(ns), issue);
+    err = launch_fill_int(cs.steps, cs.done, cs.done, static_cast<size_t>(ns), stream);
   }
   if (err == hipSuccess) {
     err = launch_fill(reinterpret_cast<long long *>(cs.rms), nullptr, nullptr,
-                      static_cast<size_t>(ns), issue);
+                      static_cast<size_t>(ns), stream);
   }
   if (err == hipSuccess && in_parts) {
-    err = clear_part_sums(k, ag, issue);
+    err = clear_part_sums(k, ag, stream);
   }
   if (how == FusedIssue::kCycleGraph) {
     if (err == hipSuccess) {
-      err = capture_fused_cycle(prec, k, k, ck, sd, cap, &graph[0], &exec[0]);
+      err = capture_fused_cycle(prec, k, k, ck, sd, 1, cap, &graph[0], &exec[0]);
     }
     if (err == hipSuccess && cdcyc > 0) {
-      err = capture_fused_cycle(prec, kf_clash, ke_clash, ck, sd, cap, &graph[1], &exec[1]);
+      err = capture_fused_cycle(prec, kf_clash, ke_clash, ck, sd, 1, cap, &graph[1], &exec[1]);
     }
     for (int c = 0; c < mc->total_cycles && err == hipSuccess; c++) {
       err = hipGraphLaunch(exec[(c < cdcyc) ? 1 : 0], stream);
@@ -1969,29 +1975,26 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
   }
   else {
     for (int c = 0; c < mc->total_cycles && err == hipSuccess; c++) {
+      if (chunks > 0 && c == lead) {
+        err = capture_fused_cycle(prec, k, k, ck, sd, kChunkCycles, cap, &graph[0], &exec[0]);
+        for (int g = 0; g < chunks && err == hipSuccess; g++) {
+          err = hipGraphLaunch(exec[0], stream);
+        }
+        c += (chunks * kChunkCycles) - 1;
+        continue;
+      }
       const bool damped = (c < cdcyc);
-      err = launch_fused_cycle(prec, damped ? kf_clash : k, damped ? ke_clash : k, ck, sd, issue);
+      err = launch_fused_cycle(prec, damped ? kf_clash : k, damped ? ke_clash : k, ck, sd,
+                               stream);
     }
   }
   if (err == hipSuccess) {
     // The final energies, after the last cycle's last move.
-    err = (mc->total_cycles > 0 && !in_parts) ? launch_min_cycle(prec, kfin, ck, false, 3, issue)
-                                              : launch_eval(prec, kfin, terms, 0, 1, issue);
+    err = (mc->total_cycles > 0 && !in_parts) ? launch_min_cycle(prec, kfin, ck, false, 3, stream)
+                                              : launch_eval(prec, kfin, terms, 0, 1, stream);
   }
   if (err == hipSuccess && in_parts) {
-    err = clear_part_sums(k, ag, issue);
-  }
-  if (how == FusedIssue::kWholeGraph) {
-    const hipError_t e1 = hipStreamEndCapture(cap, &graph[0]);
-    if (err == hipSuccess) {
-      err = e1;
-    }
-    if (err == hipSuccess) {
-      err = hipGraphInstantiate(&exec[0], graph[0], nullptr, nullptr, 0);
-    }
-    if (err == hipSuccess) {
-      err = hipGraphLaunch(exec[0], stream);
-    }
+    err = clear_part_sums(k, ag, stream);
   }
   if (how != FusedIssue::kDirect) {
     if (err == hipSuccess) {
@@ -2005,7 +2008,9 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
         (void)hipGraphDestroy(graph[g]);
       }
     }
-    (void)hipStreamDestroy(cap);
+    if (cap != nullptr) {
+      (void)hipStreamDestroy(cap);
+    }
   }
   HIP_TRY(err);
   return STORMM_OK;
@@ -2048,7 +2053,7 @@ static int minimize(int32_t precision, const stormm_synthesis *ag, const stormm_
     cs.steps = agm->cycles_run.as<int>();
     cs.done = agm->stop_flags.as<int>();
     cs.rms = agm->rms_force.as<double>();
-    const FusedIssue how = (persistent == 1) ? FusedIssue::kWholeGraph :
+    const FusedIssue how = (persistent == 1) ? FusedIssue::kChunkGraph :
                            (persistent == 3) ? FusedIssue::kCycleGraph : FusedIssue::kDirect;
     rc = minimize_fused(precision, ag, w, mincon, sch, lm, cs, ps, st, how);
   }

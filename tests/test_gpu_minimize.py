@@ -132,3 +132,24 @@ def test_convergence_threshold_stops_systems():
     res = minimize(topos, coords, "single", 300, persistent=True, rms=0.5)
     assert np.all(res["cycles"] <= 300)
     assert np.all((res["rms"] <= 0.5) | (res["cycles"] == 300))
+
+
+@pytest.mark.parametrize("cycles,clash", [(1, 0), (8, 8), (23, 5), (24, 0), (25, 25), (43, 20)])
+def test_chunked_run_equals_single_launches(cycles, clash):
+    """Mode 1 around its chunk graph's limits (eight cycles led by at least eight issued one by one)
+    against the same kernels launched one by one, twice in a row on the same objects."""
+    topos, coords = synthetic.uniform_batch(5, 16, 40, seed=61, gb=True, perturb=0.3)
+    mc = S.minimize_controls(cycles, min(4, cycles), 0.01, 0.0, clash_cycles=clash)
+    got = []
+    for mode in (1, 4):
+        ag = S.AtomGraphSynthesis(topos)
+        ps = S.PhaseSpaceSynthesis(ag, 32, 23)
+        sc = S.ScoreCard(ag.system_count, 26)
+        lm = S.LineMinimization(ag.system_count, 0.01)
+        ps.upload(coords)
+        for _ in range(2):
+            S.launch_minimization("single", ag, ps, mc, sc, lm, persistent=mode)
+        got.append((np.concatenate(ps.fixed()[0]), sc.accumulators(),
+                    ag.minimization_status()[0]))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
