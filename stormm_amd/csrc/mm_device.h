@@ -19,7 +19,8 @@ constexpr double kGbOffset = 0.09;      // src/Constants/generalized_born.h:112
 
 // ------------------------------------------------------------------------------------------
 // Precision traits.  Single precision uses the hardware transcendental units (v_rsq, v_rcp,
-// v_log, v_exp); double precision uses the correctly rounded library routines.
+// v_log, v_exp); double precision refines the hardware estimates and has its own exponential and
+// logarithm for the arguments that occur.
 // ------------------------------------------------------------------------------------------
 // Nearest integer (ties to even, as rint) of a double as int64.  For |x| < 2^51, adding
 // 1.5 * 2^52 rounds x to an integer held in the low bits of the sum's bit pattern; subtracting
@@ -56,24 +57,74 @@ template <> struct Prec<float> {
 
 template <> struct Prec<double> {
   using crd_t = double;
-  // The hardware estimates refined by two Newton-Raphson steps, y <- y + y (1 - x y) for the
-  // reciprocal and y <- y + (y / 2) (1 - x y^2) for the reciprocal square root: each step about
-  // squares the estimate's relative error, so two reach the last few bits of a double.  For
+  // The hardware estimates leave residuals e = 1 - x y (reciprocal) and 1 - x y^2 (reciprocal
+  // square root) of at most 2^-24 and 2^-23 (measured over a full octave); the binomial series
+  // y (1 + e + e^2) and y (1 + e / 2 + 3 e^2 / 8) leave about e^3, below the last bit.  Three and
+  // five instructions after the estimate, where two Newton-Raphson steps took four and eight.  For
   // positive, finite, normal arguments (distances and radii here).
   static __device__ __forceinline__ double rsqrt(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
   }
   static __device__ __forceinline__ double rcp(double x) {
-    double y = __builtin_amdgcn_rcp(x);
-    y = fma(y, fma(-x, y, 1.0), y);
-    return fma(y, fma(-x, y, 1.0), y);
+    const double y = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, y, 1.0);
+    return fma(y, fma(e, e, e), y);
   }
   static __device__ __forceinline__ double sqrt(double x) { return ::sqrt(x); }
   static __device__ __forceinline__ double cbrt(double x) { return ::cbrt(x); }
-  static __device__ __forceinline__ double log(double x) { return ::log(x); }
-  static __device__ __forceinline__ double exp(double x) { return ::exp(x); }
+  // Natural logarithm of a positive normal number m 2^e, sqrt(1/2) <= m < sqrt(2): e ln 2 +
+  // 2 artanh(f), f = (m - 1) / (m + 1), with (artanh(f) / f - 1) / f^2 interpolated at Chebyshev
+  // nodes over f^2 <= 0.0295 (relative error 4e-18 before rounding).  Its arguments here are
+  // ratios of distances; the library function's handling of other arguments is not needed.
+  static __device__ __forceinline__ double log(double x) {
+    double m = __builtin_amdgcn_frexp_mant(x);
+    int e = __builtin_amdgcn_frexp_exp(x);
+    const bool low = m < 0.70710678118654752440;
+    m = low ? m + m : m;
+    e -= low ? 1 : 0;
+    const double f = (m - 1.0) * rcp(m + 1.0);
+    const double s = f * f;
+    double h = 0.07308292712444311;
+    h = fma(h, s, 0.07665855309105386);
+    h = fma(h, s, 0.09091444727837474);
+    h = fma(h, s, 0.11111105565129939);
+    h = fma(h, s, 0.14285714313001635);
+    h = fma(h, s, 0.19999999999949722);
+    h = fma(h, s, 0.3333333333333335);
+    const double f2 = f + f;
+    return fma(static_cast<double>(e), 0.69314718055994530942, fma(f2, s * h, f2));
+  }
+  // exp(x) for x <= 0, the only sign the GB terms need: x = k ln 2 + r, |r| <= ln 2 / 2, and
+  // exp(r) = 1 + r + r^2 g(r) with g interpolated at Chebyshev nodes (relative error 2e-17 before
+  // rounding).  The bound at -1000 (where the result is zero) keeps k an int; the rounding of
+  // k ln 2 leaves an absolute error below 2e-17.  17 instructions; the library function, which
+  // takes any argument, 22.
+  static __device__ __forceinline__ double exp(double x) {
+    const double z = fmax(x, -1000.0);
+    const double k = __builtin_rint(z * 1.4426950408889634074);
+    const double r = fma(k, -0.69314718055994530942, z);
+    double g = 2.510038549551032e-08;
+    g = fma(g, r, 2.7620088445409746e-07);
+    g = fma(g, r, 2.7557268459997064e-06);
+    g = fma(g, r, 2.4801521295954376e-05);
+    g = fma(g, r, 0.00019841269863053618);
+    g = fma(g, r, 0.0013888888917213717);
+    g = fma(g, r, 0.008333333333330062);
+    g = fma(g, r, 0.04166666666662413);
+    g = fma(g, r, 0.16666666666666669);
+    g = fma(g, r, 0.5000000000000001);
+    g = fma(g, r, 1.0);
+    g = fma(g, r, 1.0);
+    return __builtin_ldexp(g, static_cast<int>(k));
+  }
+  // tanh(x) = (1 - t) / (1 + t) with t = exp(-2 |x|): the GB radii need its absolute error
+  // (2e-16), not its relative error near zero.
+  static __device__ __forceinline__ double tanh(double x) {
+    const double t = exp(-2.0 * fabs(x));
+    return copysign((1.0 - t) * rcp(1.0 + t), x);
+  }
   static __device__ __forceinline__ long long fixed(double x) { return round_to_ll(x); }
 };
 
@@ -312,7 +363,8 @@ template <typename T> struct AtomFields {
 template <typename T> struct AtomRec;
 template <> struct AtomRec<float> : AtomFields<float> {};
 template <> struct AtomRec<double> : AtomFields<double> {
-  double pad[2];
+  double irad;              // inverse Born radius (single precision keeps it in WuLds::irad)
+  double pad;
 };
 static_assert(sizeof(AtomRec<float>) == 80 && sizeof(AtomRec<double>) == 144,
               "atom records keep 16 consecutive atoms' fields in different LDS banks");
@@ -323,7 +375,7 @@ template <typename T> struct WuLds {
   AtomRec<T> *atom;
   long long *nrg, *org;
   double *move;             // per system: pending line move (coordinate units per direction unit)
-  T *irad;                  // inverse Born radius
+  T *irad;                  // inverse Born radius (single precision)
   int *gidx, *slot;
   WuSys *sys;
   int *work;                // per-stage work-item counters (kStageCounters)
@@ -369,6 +421,28 @@ template <typename T> struct WuLds {
   }
 };
 
+// Inverse Born radius of LDS atom a.
+__device__ __forceinline__ float &inv_radius(const WuLds<float> &L, int a) { return L.irad[a]; }
+__device__ __forceinline__ double &inv_radius(const WuLds<double> &L, int a) {
+  return L.atom[a].irad;
+}
+
+// The j atoms of a tile in double precision.  A 64-bit value has no DPP operand form, so rotating
+// it takes two moves: 16 of the 114 vector instructions of a pair step.  A step reads the j atom
+// it meets from the atom records instead, whose byte offset (one 32-bit value) rotates.
+struct JRecords {
+  AtomRec<double> *atom;
+  int off;
+  __device__ __forceinline__ JRecords(AtomRec<double> *records, int j0)
+      : atom(records), off(j0 * static_cast<int>(sizeof(AtomRec<double>))) {}
+  // The record of the atom that the lane meets K steps on.
+  template <int K> __device__ __forceinline__ const AtomRec<double> &at() const {
+    return *reinterpret_cast<const AtomRec<double> *>(
+        reinterpret_cast<const unsigned char *>(atom) + row_ror<K>(off));
+  }
+  template <int K> __device__ __forceinline__ void rotate() { off = row_ror<K>(off); }
+};
+
 // Displacement between two LDS coordinates in Angstroms.
 __device__ __forceinline__ float crd_delta(int a, int b, float scale) {
   return static_cast<float>(a - b) * scale;
@@ -376,8 +450,8 @@ __device__ __forceinline__ float crd_delta(int a, int b, float scale) {
 __device__ __forceinline__ double crd_delta(double a, double b, double) { return a - b; }
 
 // exp(-r^2 / (4 Ri Rj)) of the GB pair function as eval(r^2 * (1 / Rj) * (kScale / Ri)): the
-// hardware base-2 exponential in single precision (kScale carries log2 e), the library
-// exponential in double precision.
+// hardware base-2 exponential in single precision (kScale carries log2 e), Prec's in double
+// precision.
 template <typename T> struct GbExp;
 template <> struct GbExp<float> {
   static constexpr float kScale = -0.25f * 1.44269504088896340736f;
@@ -385,7 +459,7 @@ template <> struct GbExp<float> {
 };
 template <> struct GbExp<double> {
   static constexpr double kScale = -0.25;
-  static __device__ __forceinline__ double eval(double x) { return ::exp(x); }
+  static __device__ __forceinline__ double eval(double x) { return Prec<double>::exp(x); }
 };
 
 // Coordinates of a pair tile's atoms in Angstroms in the working precision.  Single precision

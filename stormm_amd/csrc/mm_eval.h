@@ -117,8 +117,12 @@ __device__ __forceinline__ void stage_load(StageCtx<T> &c, const MMKit &k) {
     const int g = gs + local;
     L.gidx[a] = valid ? g : -1;
     L.slot[a] = s;
-    L.irad[a] = T(1);
-    AtomPos<T> pos = {0, 0, 0, T(0)};
+    // In double precision the tile loops read j atoms from LDS as they come, so the padding slots
+    // hold their far-away position themselves.
+    const auto far = (sizeof(T) == 8) ? -FarAway<T>::kCrd : T(0);
+    AtomPos<T> pos = {static_cast<typename Prec<T>::crd_t>(far),
+                      static_cast<typename Prec<T>::crd_t>(far),
+                      static_cast<typename Prec<T>::crd_t>(far), T(0)};
     AtomNb<T> nb = {T(0), T(0), T(0), T(1)};
     AtomRad<T> rr = {T(1), T(1)};
     if (valid) {
@@ -193,6 +197,7 @@ __device__ __forceinline__ void stage_load(StageCtx<T> &c, const MMKit &k) {
     r.psi = 0;
     r.fx = r.fy = r.fz = 0;
     r.dedr = 0;
+    inv_radius(L, a) = T(1);
     if (PHASE == kPartPairs && valid && c.gb) {
       r.psi = k.part_psi[g];
     }
@@ -360,6 +365,46 @@ __device__ __forceinline__ void tile_coords(const StageCtx<T> &c, const TileTask
   si = pi.scr;
   sj = pj.scr;
 }
+
+// The j atom that a lane meets K rotation steps on: in double precision its record's fields, read
+// from LDS, in single precision nothing (the rotated registers serve).
+template <typename T> struct JAtom {
+  AtomPos<T> pos;
+  AtomNb<T> nb;
+  T irad, sd;
+  T s2, s3;                 // screened radius squared and cubed
+};
+template <int K> __device__ __forceinline__ JAtom<double> j_atom(const JRecords &j) {
+  const AtomRec<double> &r = j.at<K>();
+  JAtom<double> a;
+  a.pos = r.pos;
+  a.nb = r.nb;
+  a.irad = r.irad;
+  a.sd = r.sd;
+  a.s2 = r.pos.scr * r.pos.scr;
+  a.s3 = a.s2 * r.pos.scr;
+  return a;
+}
+struct NoRecords {
+  __device__ __forceinline__ NoRecords(AtomRec<float> *, int) {}
+  template <int K> __device__ __forceinline__ void rotate() {}
+};
+template <int K> __device__ __forceinline__ JAtom<float> j_atom(const NoRecords &) {
+  return JAtom<float>();
+}
+template <typename T>
+using JSource = std::conditional_t<sizeof(T) == 8, JRecords, NoRecords>;
+// A j value at step K: the record's field, or the register rotated K lanes (at the place of its
+// use, so that the rotation folds into the instruction that reads it).
+template <int K> __device__ __forceinline__ double j_value(double field, double) {
+  return field;
+}
+template <int K> __device__ __forceinline__ float j_value(float, float reg) {
+  return row_ror<K>(reg);
+}
+// Moves a register of j values on by K lanes (single precision).
+template <int K> __device__ __forceinline__ void j_rotate(double &) {}
+template <int K> __device__ __forceinline__ void j_rotate(float &reg) { reg = row_ror<K>(reg); }
 
 // True on every lane when `b` holds on every active lane of the wavefront.
 __device__ __forceinline__ bool wave_all(bool b) {
@@ -620,6 +665,7 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
     int ej = NearIndex<T>::half_j(tt.j0);
     T acci = T(0), accj = T(0);
     unsigned vbits = tt.valid;
+    JSource<T> jrec(c.L.atom, tt.j0);
     // Off-diagonal tiles need no pair mask (their padding atoms sit far away); a wavefront whose
     // four tiles are all off-diagonal runs the 16 steps without one.  On diagonal tiles the mask
     // removes each lane's own atom and the second copy of each pair.
@@ -635,18 +681,19 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
           // An absent pair is put far away: both directions are then far-field with terms
           // that round to exactly zero, so no validity test follows.
           const bool valid = !MASKED || (((vbits >> K) & 1u) != 0u);
-          const T dx = row_ror<K>(xj) - xi;
-          const T dy = row_ror<K>(yj) - yi;
-          const T dz = row_ror<K>(zj) - zi;
+          const JAtom<T> aj = j_atom<K>(jrec);
+          const T dx = j_value<K>(aj.pos.x, xj) - xi;
+          const T dy = j_value<K>(aj.pos.y, yj) - yi;
+          const T dz = j_value<K>(aj.pos.z, zj) - zi;
           const T r2c = (dx * dx) + (dy * dy) + (dz * dz);
           const T r2 = valid ? r2c : FarAway<T>::kR2;
           const T invr2 = P::rcp(r2);
           const T invr4 = invr2 * invr2;
-          const T x_i = row_ror<K>(sj2) * invr2;
+          const T x_i = j_value<K>(aj.s2, sj2) * invr2;
           const T x_j = si2 * invr2;
           const bool far_i = x_i < T(0.0625);
           const bool far_j = x_j < T(0.0625);
-          const T ti = psi_series(x_i) * (row_ror<K>(sj3) * invr4);
+          const T ti = psi_series(x_i) * (j_value<K>(aj.s3, sj3) * invr4);
           const T tj = psi_series(x_j) * (si3 * invr4);
           acci -= far_i ? ti : T(0);
           accj = row_rotate(accj) - (far_j ? tj : T(0));
@@ -655,11 +702,12 @@ __device__ __forceinline__ void stage_psi(StageCtx<T> &c, const MMKit &k, int va
         unrolled_steps(step, std::integer_sequence<int, 0, 1, 2, 3>{});
         settle(acci);
         vbits >>= kStepGroup;
-        xj = row_ror<kStepGroup>(xj);
-        yj = row_ror<kStepGroup>(yj);
-        zj = row_ror<kStepGroup>(zj);
-        sj2 = row_ror<kStepGroup>(sj2);
-        sj3 = row_ror<kStepGroup>(sj3);
+        jrec.template rotate<kStepGroup>();
+        j_rotate<kStepGroup>(xj);
+        j_rotate<kStepGroup>(yj);
+        j_rotate<kStepGroup>(zj);
+        j_rotate<kStepGroup>(sj2);
+        j_rotate<kStepGroup>(sj3);
         ej = row_ror<kStepGroup>(ej);
         while (qn >= 64) {
           psi_drain(c, q + (qn - 64), 64, lane);
@@ -702,34 +750,37 @@ __device__ __forceinline__ void stage_radii(StageCtx<T> &c, const MMKit &k, doub
     }
     const double psi = static_cast<double>(L.atom[a].psi) * ldexp(1.0, -kPsiBits);
     const double rho = k.rho[g];
-    double R;
+    using D = Prec<double>;
+    double R, invR;
     if (k.igb == 1) {
-      R = 1.0 / ((1.0 / rho) + psi);
-      R = (R < 0.0) ? 30.0 : R;
+      invR = D::rcp(rho) + psi;
+      R = (invR < 0.0) ? 30.0 : 1.0 / invR;
+      invR = 1.0 / R;
     }
     else {
       const double fipsi = psi * (-rho);
       const double al = k.gb_alpha, be = k.gb_beta, ga = k.gb_gamma;
-      const double pbr = rho + kGbOffset;  // intrinsic radius
-      const double thi = tanh((al - (be * fipsi) + (ga * fipsi * fipsi)) * fipsi);
-      R = 1.0 / ((1.0 / rho) - thi / pbr);
+      const double inv_pbr = D::rcp(rho + kGbOffset);  // of the intrinsic radius
+      const double thi = D::tanh((al - (be * fipsi) + (ga * fipsi * fipsi)) * fipsi);
+      invR = D::rcp(rho) - (thi * inv_pbr);
+      R = D::rcp(invR);
       if (FORCES) {
         // dR/dpsi of the OBC model (nonbonded_potential.tpp:985-1017), kept for the chain rule
         // in the accumulator slot whose psi is no longer needed.
         const double dr_dpsi = (al - ((2.0 * be) - (3.0 * ga * fipsi)) * fipsi) *
-                               (1.0 - thi * thi) * rho / pbr;
+                               (1.0 - thi * thi) * rho * inv_pbr;
         L.atom[a].psi = __double_as_longlong(dr_dpsi);
       }
     }
     L.atom[a].nb.rad = static_cast<T>(R);
-    L.irad[a] = static_cast<T>(1.0 / R);
+    inv_radius(L, a) = static_cast<T>(invR);
     // q holds charge * sqrt(Coulomb), so q^2 = Coulomb * charge^2.
     const double qg = k.q[g];
-    const double expmkf = ((k.kappa != 0.0) ? exp(-kGbKscale * k.kappa * R) : 1.0) * inv_diel;
+    const double expmkf = ((k.kappa != 0.0) ? D::exp(-kGbKscale * k.kappa * R) : 1.0) * inv_diel;
     const double dielfac = 1.0 - expmkf;
     const double atmq2h = 0.5 * qg * qg;
     const double atmqd2h = atmq2h * dielfac;
-    const double contrib = -atmqd2h / R;
+    const double contrib = -atmqd2h * invR;
     if (c.part != 0) {
       continue;  // the unit's first part adds the self terms
     }
@@ -833,8 +884,9 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
     const T qi = ni.q, p1i = ni.p1, p2i = ni.p2, Ri = ni.rad;
     T qj = nj.q, p1j = nj.p1, p2j = nj.p2, Rj = nj.rad;
     // exp(-r^2 / (4 Ri Rj)) = GbExp(r^2 * (1 / Rj) * (scale / Ri)).
-    T iRj = GB ? L.irad[tt.j0] : T(0);
-    const T iRi = GB ? L.irad[tt.i] * GbExp<T>::kScale : T(0);
+    T iRj = GB ? inv_radius(L, tt.j0) : T(0);
+    const T iRi = GB ? inv_radius(L, tt.i) * GbExp<T>::kScale : T(0);
+    JSource<T> jrec(c.L.atom, tt.j0);
     T fxi = T(0), fyi = T(0), fzi = T(0), dri = T(0);
     T fxj = T(0), fyj = T(0), fzj = T(0), drj = T(0);
     // Each lane sums its energies over the task in the calculation precision and converts the
@@ -875,17 +927,18 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
           }
           const bool valid = !MASKED || (((vbits >> K) & 1u) != 0u);
           const bool nbok = !MASKED || (((nbbits >> K) & 1u) != 0u);
-          const T dx = row_ror<K>(xj) - xi;
-          const T dy = row_ror<K>(yj) - yi;
-          const T dz = row_ror<K>(zj) - zi;
+          const JAtom<T> aj = j_atom<K>(jrec);
+          const T dx = j_value<K>(aj.pos.x, xj) - xi;
+          const T dy = j_value<K>(aj.pos.y, yj) - yi;
+          const T dz = j_value<K>(aj.pos.z, zj) - zi;
           const T r2c = (dx * dx) + (dy * dy) + (dz * dz);
           const T r2 = valid ? r2c : T(1);
-          const T qiqj = row_ror<K>(qj) * qi;
+          const T qiqj = j_value<K>(aj.nb.q, qj) * qi;
           T fmag = T(0);
           if (GB) {
             const T qgb = valid ? qiqj : T(0);
-            const T rr = row_ror<K>(Rj) * Ri;
-            const T efac = GbExp<T>::eval(r2 * (row_ror<K>(iRj) * iRi));
+            const T rr = j_value<K>(aj.nb.rad, Rj) * Ri;
+            const T efac = GbExp<T>::eval(r2 * (j_value<K>(aj.irad, iRj) * iRi));
             const T fgb2 = r2 + (rr * efac);
             const T fgbi = P::rsqrt(fgb2);
             // egb = qq (1 - exp(-kappa fgb) / diel) / fgb, temp6 = -(dE/dfgb) / fgb.
@@ -912,8 +965,8 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
           }
           const T qnb = nbok ? qiqj : T(0);
           if (CLASH && clash_on) {
-            const T pj1 = row_ror<K>(p1j);
-            const T pj2 = row_ror<K>(p2j);
+            const T pj1 = j_value<K>(aj.nb.p1, p1j);
+            const T pj2 = j_value<K>(aj.nb.p2, p2j);
             T lja, ljb, sigma;
             if (LJTABLE) {
               const double2 ab = ljrow[static_cast<int>(pj1)];
@@ -939,7 +992,7 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
             const T eqq = qnb * invr;
             e_qq += eqq;
             if (LJTABLE) {
-              const double2 ab = ljrow[static_cast<int>(row_ror<K>(p1j))];
+              const double2 ab = ljrow[static_cast<int>(j_value<K>(aj.nb.p1, p1j))];
               const T lja = nbok ? static_cast<T>(ab.x) : T(0);
               const T ljb = nbok ? static_cast<T>(ab.y) : T(0);
               const T invr4 = invr2 * invr2;
@@ -949,10 +1002,10 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
               }
             }
             else {
-              const T sig = row_ror<K>(p1j) + p1i;
+              const T sig = j_value<K>(aj.nb.p1, p1j) + p1i;
               const T s2 = sig * sig * invr2;
               const T s6 = s2 * s2 * s2;
-              const T e4c = row_ror<K>(p2j) * p2i;
+              const T e4c = j_value<K>(aj.nb.p2, p2j) * p2i;
               const T e4 = nbok ? e4c : T(0);
               const T e4s6 = e4 * s6;
               e_lj += e4s6 * (s6 - T(1));
@@ -979,15 +1032,16 @@ __device__ __forceinline__ void stage_pairs(StageCtx<T> &c, const MMKit &k) {
         unrolled_steps(step, std::make_integer_sequence<int, kGroup>{});
         vbits >>= kGroup;
         nbbits >>= kGroup;
-        xj = row_ror<kGroup>(xj);
-        yj = row_ror<kGroup>(yj);
-        zj = row_ror<kGroup>(zj);
-        qj = row_ror<kGroup>(qj);
-        p1j = row_ror<kGroup>(p1j);
-        p2j = row_ror<kGroup>(p2j);
+        jrec.template rotate<kGroup>();
+        j_rotate<kGroup>(xj);
+        j_rotate<kGroup>(yj);
+        j_rotate<kGroup>(zj);
+        j_rotate<kGroup>(qj);
+        j_rotate<kGroup>(p1j);
+        j_rotate<kGroup>(p2j);
         if (GB) {
-          Rj = row_ror<kGroup>(Rj);
-          iRj = row_ror<kGroup>(iRj);
+          j_rotate<kGroup>(Rj);
+          j_rotate<kGroup>(iRj);
         }
       }
     };
@@ -1127,6 +1181,7 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
     T fxi = T(0), fyi = T(0), fzi = T(0);
     T gxj = T(0), gyj = T(0), gzj = T(0);
     unsigned vbits = tt.valid;
+    JSource<T> jrec(c.L.atom, tt.j0);
     // Wavefronts of four off-diagonal tiles run without a pair mask, as in stage_psi.
     auto run = [&](auto mc) {
       constexpr bool MASKED = decltype(mc)::value;
@@ -1139,21 +1194,22 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
           }
           // Absent pairs are put far away, as in stage_psi.
           const bool valid = !MASKED || (((vbits >> K) & 1u) != 0u);
-          const T dx = row_ror<K>(xj) - xi;
-          const T dy = row_ror<K>(yj) - yi;
-          const T dz = row_ror<K>(zj) - zi;
+          const JAtom<T> aj = j_atom<K>(jrec);
+          const T dx = j_value<K>(aj.pos.x, xj) - xi;
+          const T dy = j_value<K>(aj.pos.y, yj) - yi;
+          const T dz = j_value<K>(aj.pos.z, zj) - zi;
           const T r2c = (dx * dx) + (dy * dy) + (dz * dz);
           const T r2 = valid ? r2c : FarAway<T>::kR2;
           const T invr2 = P::rcp(r2);
           const T invr6 = invr2 * invr2 * invr2;
-          const T x_i = row_ror<K>(sj2) * invr2;
+          const T x_i = j_value<K>(aj.s2, sj2) * invr2;
           const T x_j = si2 * invr2;
           const bool far_i = x_i < T(0.0625);
           const bool far_j = x_j < T(0.0625);
           // Both series are evaluated on every lane and selected, which keeps the step free of
           // branches.
-          const T ti = dpsi_series(x_i) * (row_ror<K>(sj3) * (invr6 * sdi));
-          const T tj = dpsi_series(x_j) * (row_ror<K>(sdj) * (invr6 * si3));
+          const T ti = dpsi_series(x_i) * (j_value<K>(aj.s3, sj3) * (invr6 * sdi));
+          const T tj = dpsi_series(x_j) * (j_value<K>(aj.sd, sdj) * (invr6 * si3));
           const T fmag = (far_i ? ti : T(0)) + (far_j ? tj : T(0));
           const T fdx = fmag * dx;
           const T fdy = fmag * dy;
@@ -1171,12 +1227,13 @@ __device__ __forceinline__ void stage_deriv(StageCtx<T> &c, const MMKit &k) {
         settle(fyi);
         settle(fzi);
         vbits >>= kStepGroup;
-        xj = row_ror<kStepGroup>(xj);
-        yj = row_ror<kStepGroup>(yj);
-        zj = row_ror<kStepGroup>(zj);
-        sj2 = row_ror<kStepGroup>(sj2);
-        sj3 = row_ror<kStepGroup>(sj3);
-        sdj = row_ror<kStepGroup>(sdj);
+        jrec.template rotate<kStepGroup>();
+        j_rotate<kStepGroup>(xj);
+        j_rotate<kStepGroup>(yj);
+        j_rotate<kStepGroup>(zj);
+        j_rotate<kStepGroup>(sj2);
+        j_rotate<kStepGroup>(sj3);
+        j_rotate<kStepGroup>(sdj);
         ej = row_ror<kStepGroup>(ej);
         while (qn >= 64) {
           deriv_drain(c, q + (qn - 64), 64, lane, k.frc_bits);
@@ -1279,10 +1336,12 @@ template <bool FORCES, typename V>
 __device__ __forceinline__ double eval_bond(const V &v, int i, int j, double kb,
                                             double r0, double fscale) {
   const Vec3 d = v.disp(i, j);
-  const double dr = sqrt(dot(d, d));
+  const double d2 = dot(d, d);
+  const double inv = Prec<double>::rsqrt(d2);
+  const double dr = (d2 > 0.0) ? d2 * inv : 0.0;
   const double dl = dr - r0;
   if (FORCES) {
-    const double fmag = 2.0 * kb * dl / dr;
+    const double fmag = 2.0 * kb * dl * inv;
     const long long ix = fix64(fmag * d.x * fscale);
     const long long iy = fix64(fmag * d.y * fscale);
     const long long iz = fix64(fmag * d.z * fscale);
@@ -1298,17 +1357,18 @@ __device__ __forceinline__ double eval_angle(const V &v, int i, int j, int kk,
                                              double ka, double th0, double fscale) {
   const Vec3 ba = v.disp(j, i);
   const Vec3 bc = v.disp(j, kk);
-  const double mgba = dot(ba, ba);
-  const double mgbc = dot(bc, bc);
-  const double invbabc = 1.0 / sqrt(mgba * mgbc);
+  const double invba = Prec<double>::rsqrt(dot(ba, ba));
+  const double invbc = Prec<double>::rsqrt(dot(bc, bc));
+  const double invbabc = invba * invbc;
   double costheta = dot(ba, bc) * invbabc;
   costheta = (costheta < -1.0) ? -1.0 : ((costheta > 1.0) ? 1.0 : costheta);
   const double theta = acos(costheta);
   const double dtheta = theta - th0;
   if (FORCES) {
-    const double dA = -2.0 * ka * dtheta / sqrt(1.0 - (costheta * costheta));
-    const double sqba = dA / mgba;
-    const double sqbc = dA / mgbc;
+    const double dA = -2.0 * ka * dtheta *
+                      Prec<double>::rsqrt(1.0 - (costheta * costheta));
+    const double sqba = dA * invba * invba;
+    const double sqbc = dA * invbc * invbc;
     const double mbabc = dA * invbabc;
     const long long iax = fix64(((bc.x * mbabc) - (costheta * ba.x * sqba)) * fscale);
     const long long iay = fix64(((bc.y * mbabc) - (costheta * ba.y * sqba)) * fscale);
