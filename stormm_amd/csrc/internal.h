@@ -44,14 +44,14 @@ constexpr int kOriginBits = 38;
 constexpr int kMaxPlainGposBits = 38;
 constexpr int kMaxPlainFrcBits = 40;
 // Threads of an evaluation block: the fewest and the most a launch may use, and the defaults
-// (eval_block).  Double-precision kernels hold 155-168 registers per lane, which three wavefronts
-// on a SIMD leave free: one block of 12 wavefronts fills a compute unit that two of 8 do not fit
-// (1024 systems 212 -> 199 us, energies of 4096 systems 161 -> 151 us against 512 threads).
+// (eval_block).
 constexpr int kEvalBlock = 512;
 constexpr int kEvalBlockSparse = 1024;
 constexpr int kMinEvalBlock = 256;
 constexpr int kMaxEvalBlock = 1024;
-constexpr int kMaxEvalBlockDouble = 768;
+constexpr int kMaxEvalBlockDoubleClash = 768;
+constexpr int kSmallUnitDouble = 128;  // atoms
+constexpr size_t kLdsPerCu = 160 * 1024;
 // Entries of each wavefront's LDS queue of near-field Born-integral pairs.  A wave drains 64
 // entries at a time whenever the queue holds at least 64 after a group of four rotation steps,
 // each of which adds at most 64 (and stores its lanes without an entry just past the new

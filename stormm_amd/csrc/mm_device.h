@@ -308,28 +308,14 @@ __device__ __forceinline__ long long fixed_contrib(double x, int bits) {
   return round_to_ll(ldexp(x, bits));
 }
 
-// Largest block a kernel of each precision is compiled for.
-template <typename T> struct EvalBlockLimit;
-template <> struct EvalBlockLimit<float> {
+// Largest block a kernel is compiled for: 16 wavefronts leave 128 registers to a lane, and the
+// clash-damped force evaluations in double precision (HEAVY) need 150.
+template <typename T, bool HEAVY> struct EvalBlockLimit {
   static constexpr int value = kMaxEvalBlock;
 };
-template <> struct EvalBlockLimit<double> {
-  static constexpr int value = kMaxEvalBlockDouble;
+template <> struct EvalBlockLimit<double, true> {
+  static constexpr int value = kMaxEvalBlockDoubleClash;
 };
-
-// Threads of an evaluation block.  With no more units than compute units each block has its
-// compute unit to itself, and 16 wavefronts hide the latencies that 8 leave open (24 systems of
-// 487 atoms 196 -> 161 us); with more units two blocks of 8 share it, whose barriers do not
-// coincide (1024 systems 110 us against 125).
-template <typename T> inline int eval_block(const MMKit &k, int blocks) {
-  if (k.block > 0) {
-    return (k.block < EvalBlockLimit<T>::value) ? k.block : EvalBlockLimit<T>::value;
-  }
-  if (sizeof(T) == 8) {
-    return kMaxEvalBlockDouble;
-  }
-  return (blocks <= k.cus) ? kEvalBlockSparse : kEvalBlock;
-}
 
 // ------------------------------------------------------------------------------------------
 // Work-unit LDS layout.  Everything the pair loops read or add to of one atom lies in one record,
@@ -420,6 +406,27 @@ template <typename T> struct WuLds {
                                               sizeof(unsigned)));
   }
 };
+
+// Threads of an evaluation block.  With no more units than compute units each block has its
+// compute unit to itself, and 16 wavefronts hide the latencies that 8 leave open (24 systems of
+// 487 atoms 196 -> 161 us); with more units two blocks of 8 share it, whose barriers do not
+// coincide (1024 systems 110 us against 125).  In double precision two such blocks need units of
+// at most 336 atoms to fit the LDS (600 systems of 20-200 atoms 77 us against 96); beyond that
+// one block takes the whole compute unit (1024 systems of 24-256 atoms 157 us against 178 at
+// half the size), and a unit alone that is too small for 16 wavefronts takes 8 (200 systems of
+// 100 atoms 37 us against 40).  A HEAVY kernel's registers hold 12 wavefronts instead of 16.
+template <typename T, bool HEAVY> inline int eval_block(const MMKit &k, int blocks) {
+  constexpr int limit = EvalBlockLimit<T, HEAVY>::value;
+  if (k.block > 0) {
+    return (k.block < limit) ? k.block : limit;
+  }
+  if (sizeof(T) == 4) {
+    return (blocks <= k.cus) ? kEvalBlockSparse : kEvalBlock;
+  }
+  const bool half = (blocks <= k.cus) ? (k.maxa <= kSmallUnitDouble) :
+                                        (2 * WuLds<T>::bytes(k.maxa, limit / 128) <= kLdsPerCu);
+  return half ? (limit / 2) : limit;
+}
 
 // Inverse Born radius of LDS atom a.
 __device__ __forceinline__ float &inv_radius(const WuLds<float> &L, int a) { return L.irad[a]; }

@@ -9,7 +9,7 @@ namespace stormm_amd {
 // CLASH instantiations carry the clash-damped Coulomb / Lennard-Jones / 1:4 potentials used in
 // the first cycles of a minimization; the others never pay for them.
 template <typename T, bool FORCES, bool CLASH>
-__global__ void __launch_bounds__(EvalBlockLimit<T>::value)
+__global__ void __launch_bounds__((EvalBlockLimit<T, FORCES && CLASH>::value))
     k_mm_eval(MMKit k, int terms, int eval_energy) {
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
@@ -20,7 +20,7 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
 
 template <typename T, bool FORCES, bool CLASH>
 static hipError_t launch_eval_t(const MMKit &k, int terms, int eval_energy, hipStream_t stream) {
-  const int block = eval_block<T>(k, k.nwu);
+  const int block = eval_block<T, FORCES && CLASH>(k, k.nwu);
   const size_t lds = WuLds<T>::bytes(k.maxa, block / 64);
   auto fn = k_mm_eval<T, FORCES, CLASH>;
   hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),

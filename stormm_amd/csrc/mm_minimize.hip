@@ -490,7 +490,7 @@ namespace stormm_amd {
 // too).  A unit whose systems have all stopped returns at once: its coordinates, forces and
 // ScoreCard rows already hold what an evaluation would write.
 template <typename T, bool FORCES, bool CLASH>
-__global__ void __launch_bounds__(EvalBlockLimit<T>::value)
+__global__ void __launch_bounds__((EvalBlockLimit<T, FORCES && CLASH>::value))
     k_min_cycle(MMKit k, CycleKit ck, int pending_move) {
   extern __shared__ __align__(16) unsigned char smem[];
   const WuDesc &wu = k.wu[blockIdx.x];
@@ -533,7 +533,7 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
 template <typename T, bool FORCES, bool CLASH>
 static hipError_t launch_cycle_t(const MMKit &k, const CycleKit &ck, int pending_move,
                                  hipStream_t stream) {
-  const int block = eval_block<T>(k, k.nwu);
+  const int block = eval_block<T, FORCES && CLASH>(k, k.nwu);
   const size_t lds = WuLds<T>::bytes(k.maxa, block / 64);
   auto fn = k_min_cycle<T, FORCES, CLASH>;
   hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),

@@ -50,7 +50,7 @@ __device__ __forceinline__ void part_store(StageCtx<T> &c, const MMKit &k, bool 
 // first part also clears what the later phases add to: dE/dR, and, when the launch overwrites,
 // the forces and energies (this phase adds to neither).
 template <typename T, bool FORCES>
-__global__ void __launch_bounds__(EvalBlockLimit<T>::value)
+__global__ void __launch_bounds__((EvalBlockLimit<T, false>::value))
     k_part_psi(MMKit k, int terms, int eval_energy) {
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
 // Phase 1: radii from the summed integrals (every part; the first adds the self terms and keeps
 // dR/dpsi), this part's share of the valence terms and pairs; the first part takes the restraints.
 template <typename T, bool FORCES, bool CLASH>
-__global__ void __launch_bounds__(EvalBlockLimit<T>::value)
+__global__ void __launch_bounds__((EvalBlockLimit<T, FORCES && CLASH>::value))
     k_part_pairs(MMKit k, int terms, int eval_energy) {
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
@@ -143,7 +143,8 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value)
 // Phase 2: this part's share of the derivative forces.  The first part returns the Born-radius
 // integrals, which no phase reads any more, to zero for the next evaluation.
 template <typename T>
-__global__ void __launch_bounds__(EvalBlockLimit<T>::value) k_part_deriv(MMKit k, int terms) {
+__global__ void __launch_bounds__((EvalBlockLimit<T, false>::value))
+    k_part_deriv(MMKit k, int terms) {
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
   const WuPart wp = k.parts[blockIdx.x];
@@ -163,9 +164,10 @@ __global__ void __launch_bounds__(EvalBlockLimit<T>::value) k_part_deriv(MMKit k
   part_store<T, true>(c, k, false);
 }
 
-template <typename F, typename... Args>
-static hipError_t launch_parts(F fn, const MMKit &k, size_t lds, int block, hipStream_t stream,
-                               Args... args) {
+template <typename T, bool HEAVY = false, typename F, typename... Args>
+static hipError_t launch_parts(F fn, const MMKit &k, hipStream_t stream, Args... args) {
+  const int block = eval_block<T, HEAVY>(k, k.nparts);
+  const size_t lds = WuLds<T>::bytes(k.maxa, block / 64);
   const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
                                              static_cast<int>(lds));
@@ -179,22 +181,23 @@ static hipError_t launch_parts(F fn, const MMKit &k, size_t lds, int block, hipS
 template <typename T>
 static hipError_t launch_mm_parts_t(const MMKit &k, int terms, bool force, int eval_energy,
                                     hipStream_t stream) {
-  const int block = eval_block<T>(k, k.nparts);
-  const size_t lds = WuLds<T>::bytes(k.maxa, block / 64);
   const bool gb = (k.igb != 0) && (terms & kTermNonbonded) != 0;
   const bool clash = (k.clash_variant != 0);
   hipError_t err = hipSuccess;
   if (gb || k.store_overwrite) {
-    err = launch_parts(force ? k_part_psi<T, true> : k_part_psi<T, false>, k, lds, block, stream,
-                       terms, eval_energy);
+    err = launch_parts<T>(force ? k_part_psi<T, true> : k_part_psi<T, false>, k, stream, terms,
+                          eval_energy);
   }
   if (err == hipSuccess) {
-    auto fn = force ? (clash ? k_part_pairs<T, true, true> : k_part_pairs<T, true, false>)
-                    : (clash ? k_part_pairs<T, false, true> : k_part_pairs<T, false, false>);
-    err = launch_parts(fn, k, lds, block, stream, terms, eval_energy);
+    err = (force && clash)
+              ? launch_parts<T, true>(k_part_pairs<T, true, true>, k, stream, terms, eval_energy)
+              : launch_parts<T>(force ? k_part_pairs<T, true, false>
+                                      : clash ? k_part_pairs<T, false, true>
+                                              : k_part_pairs<T, false, false>,
+                                k, stream, terms, eval_energy);
   }
   if (err == hipSuccess && gb && force) {
-    err = launch_parts(k_part_deriv<T>, k, lds, block, stream, terms);
+    err = launch_parts<T>(k_part_deriv<T>, k, stream, terms);
   }
   return err;
 }

@@ -30,3 +30,26 @@ def test_default_block_equals_explicit_blocks(count, lo, hi, prec):
     for threads in (256, 512, 1024):
         f, e = evaluate(topos, coords, prec, {"block_threads": threads})
         assert np.array_equal(f, forces) and np.array_equal(e, energies), threads
+
+
+# Units at the sizes where the double-precision block changes, alone on a compute unit (112 and
+# 144 atoms) and in greater number (336 and 352 atoms), plain and clash-damped.
+@pytest.mark.parametrize("count,natom", [(3, 112), (3, 129), (260, 336), (260, 337)])
+@pytest.mark.parametrize("clash", [0.0, 1.5])
+def test_double_block_by_unit_size(count, natom, clash):
+    topos, coords = synthetic.uniform_batch(count, natom, natom, seed=78, gb=True)
+
+    def run(shape):
+        ag = S.AtomGraphSynthesis(topos, shape)
+        ps = S.PhaseSpaceSynthesis(ag, 32, 40)
+        sc = S.ScoreCard(ag.system_count, 32)
+        ps.upload(coords)
+        ps.initialize_forces()
+        sc.initialize()
+        S.launch_nonbonded("double", ag, None, ps, sc, True, True, clash_distance=clash,
+                           clash_ratio=0.7 if clash else 0.0)
+        return np.concatenate(ps.fixed()[1]), sc.accumulators()
+
+    forces, energies = run(None)
+    f, e = run({"block_threads": 256})
+    assert np.array_equal(f, forces) and np.array_equal(e, energies)
