@@ -134,7 +134,8 @@ int fill_atom_parameters(const stormm_topology_batch *b, const SystemTerms &t, i
                          const TopoTemplate &tp, const SolventModel &sm, int start,
                          AtomParams &ap, int s);
 
-// Longest-processing-time assignment of systems onto about `groups` x `per_group` work units.
+// Longest-processing-time assignment of systems onto about `groups` x `per_group` work units, or
+// a larger multiple of `groups` where these cannot hold them.
 // With `grouped`, and when every unit fits on the device at once, the systems are balanced over
 // `groups` groups (one per compute unit) emitted so that units g, g + G, g + 2G, ... form group
 // g; otherwise the units are balanced individually and emitted by decreasing cost.
