@@ -52,6 +52,8 @@ constexpr int kMaxEvalBlock = 1024;
 constexpr int kMaxEvalBlockDoubleClash = 768;
 constexpr int kSmallUnitDouble = 128;  // atoms
 constexpr size_t kLdsPerCu = 160 * 1024;
+// Atoms of the largest unit two of which fit a compute unit in double precision.
+constexpr int kTwoBlockAtomsDouble = 336;
 // Entries of each wavefront's LDS queue of near-field Born-integral pairs.  A wave drains 64
 // entries at a time whenever the queue holds at least 64 after a group of four rotation steps,
 // each of which adds at most 64 (and stores its lanes without an entry just past the new

@@ -369,7 +369,7 @@ template <typename T> struct WuLds {
   int *clash_on;            // per-system flag: damped potentials apply
   unsigned *nearq;          // kNearQueueStride entries per wavefront: its near-pair queue
 
-  static __host__ __device__ size_t bytes(int maxa, int waves) {
+  static constexpr __host__ __device__ size_t bytes(int maxa, int waves) {
     const size_t m = static_cast<size_t>(maxa);
     return (kMaxWuTasks * sizeof(int4)) +
            (m * sizeof(AtomRec<T>)) + (kMaxWuSystems * sizeof(WuSys)) +
@@ -406,6 +406,11 @@ template <typename T> struct WuLds {
                                               sizeof(unsigned)));
   }
 };
+
+static_assert(2 * WuLds<double>::bytes(kTwoBlockAtomsDouble, kEvalBlock / 64) <= kLdsPerCu &&
+                  2 * WuLds<double>::bytes(kTwoBlockAtomsDouble + kTile, kEvalBlock / 64) >
+                      kLdsPerCu,
+              "two units of kTwoBlockAtomsDouble atoms, and no larger ones, share a compute unit");
 
 // Threads of an evaluation block.  With no more units than compute units each block has its
 // compute unit to itself, and 16 wavefronts hide the latencies that 8 leave open (24 systems of

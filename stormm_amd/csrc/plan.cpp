@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <set>
 #include <string>
 
 namespace stormm_amd {
@@ -493,14 +494,20 @@ static void pack_lpt(const std::vector<double> &cost, const std::vector<int> &na
     const int target = std::max(1, static_cast<int>(std::lround(target_total * mode_cost /
                                                                 std::max(total_cost, 1.0))));
     const size_t first_bin = bins.size();
+    // The units that take more systems by their room (in tiles, as far as a system can need),
+    // cost and number: the cheapest with enough room is the first of one of the sets.
+    constexpr int kMostTiles = kMaxWuAtoms / kTile;
+    std::set<std::pair<double, int>> open[kMostTiles + 1];
+    auto room_set = [&](int bin) -> std::set<std::pair<double, int>> & {
+      return open[std::min(std::max(cap - bins[bin].atoms, 0) / kTile, kMostTiles)];
+    };
     for (int s : order) {
       const int need = round_up(natom[s], kTile);
       int best = -1;
-      for (size_t k = first_bin; k < bins.size(); k++) {
-        if (bins[k].atoms + need <= cap &&
-            static_cast<int>(bins[k].systems.size()) < kMaxWuSystems &&
-            (best < 0 || bins[k].cost < bins[best].cost)) {
-          best = static_cast<int>(k);
+      for (int room = need / kTile; room <= kMostTiles; room++) {
+        if (!open[room].empty() &&
+            (best < 0 || *open[room].begin() < std::make_pair(bins[best].cost, best))) {
+          best = open[room].begin()->second;
         }
       }
       const bool open_new = (best < 0) ||
@@ -512,9 +519,15 @@ static void pack_lpt(const std::vector<double> &cost, const std::vector<int> &na
         bins.push_back(nb);
         best = static_cast<int>(bins.size()) - 1;
       }
+      else {
+        room_set(best).erase({bins[best].cost, best});
+      }
       bins[best].systems.push_back(s);
       bins[best].atoms += need;
       bins[best].cost += cost[s];
+      if (static_cast<int>(bins[best].systems.size()) < kMaxWuSystems) {
+        room_set(best).insert({bins[best].cost, best});
+      }
     }
   }
   std::stable_sort(bins.begin(), bins.end(), [](const Bin &a, const Bin &c) {
@@ -585,16 +598,11 @@ static bool pack_parts(const std::vector<double> &cost, const std::vector<int> &
   return false;
 }
 
-void pack_systems(const std::vector<double> &cost, const std::vector<int> &natom,
-                  const std::vector<char> &table_mode, int cap, int groups, int per_group,
-                  bool grouped, std::vector<std::vector<int>> &bins_out,
-                  std::vector<int> &mode_out, std::vector<WuPart> &parts) {
-  groups = std::max(1, groups);
-  per_group = std::max(1, per_group);
-  parts.clear();
-  if (pack_parts(cost, natom, table_mode, cap, groups, bins_out, mode_out, parts)) {
-    return;
-  }
+// Units without parts: see pack_systems.
+static void pack_units(const std::vector<double> &cost, const std::vector<int> &natom,
+                       const std::vector<char> &table_mode, int cap, int groups, int per_group,
+                       bool grouped, std::vector<std::vector<int>> &bins_out,
+                       std::vector<int> &mode_out) {
   if (grouped &&
       pack_grouped(cost, natom, table_mode, cap, groups, per_group, bins_out, mode_out)) {
     return;
@@ -622,6 +630,18 @@ void pack_systems(const std::vector<double> &cost, const std::vector<int> &natom
     }
   }
   pack_lpt(cost, natom, table_mode, cap, groups * per_group, bins_out, mode_out);
+}
+
+void pack_systems(const std::vector<double> &cost, const std::vector<int> &natom,
+                  const std::vector<char> &table_mode, int cap, int groups, int per_group,
+                  bool grouped, std::vector<std::vector<int>> &bins_out,
+                  std::vector<int> &mode_out, std::vector<WuPart> &parts) {
+  groups = std::max(1, groups);
+  per_group = std::max(1, per_group);
+  parts.clear();
+  if (!pack_parts(cost, natom, table_mode, cap, groups, bins_out, mode_out, parts)) {
+    pack_units(cost, natom, table_mode, cap, groups, per_group, grouped, bins_out, mode_out);
+  }
 }
 
 int solvent_model(const stormm_topology_batch *b, SolventModel &sm) {
@@ -1071,17 +1091,36 @@ int build_plan(const stormm_topology_batch *b, const stormm_launch_shape *shape_
   std::vector<int> bin_mode;
   pack_systems(cost, P.atom_counts, P.lj_table_mode, cap, cus, wu_per_cu, true, bins, bin_mode,
                P.parts);
-  P.maxa = 0;
-  for (size_t u = 0; u < bins.size(); u++) {
-    P.maxa = std::max(P.maxa, append_work_unit(bins[u], bin_mode[u], sys_index, P.atom_starts,
-                                               P.atom_counts, P.sys_template, P.ts, P.wu,
-                                               P.wu_sys, &P.rst_first, &P.rst_count));
-    if (P.wu.back().task_count > kMaxWuTasks) {
-      return fail(STORMM_ERR_CAPACITY, "a work unit holds more than " +
-                                           std::to_string(kMaxWuTasks) + " tile tasks");
+  auto append = [&](std::vector<WuDesc> &wu, std::vector<WuSys> &wu_sys, int &maxa) {
+    maxa = 0;
+    for (size_t u = 0; u < bins.size(); u++) {
+      maxa = std::max(maxa, append_work_unit(bins[u], bin_mode[u], sys_index, P.atom_starts,
+                                             P.atom_counts, P.sys_template, P.ts, wu, wu_sys,
+                                             &P.rst_first, &P.rst_count));
+      if (wu.back().task_count > kMaxWuTasks) {
+        return fail(STORMM_ERR_CAPACITY, "a work unit holds more than " +
+                                             std::to_string(kMaxWuTasks) + " tile tasks");
+      }
     }
+    return static_cast<int>(STORMM_OK);
+  };
+  rc = append(P.wu, P.wu_sys, P.maxa);
+  // Larger units than two of which fit a compute unit's LDS in double precision: smaller ones
+  // for that precision, if the systems allow and the caller did not choose the shape.  Two blocks
+  // whose barriers do not coincide then share the compute unit (1024 systems of 24-256 atoms
+  // 171 us in units of up to 384 atoms, 154 in units of 336).
+  int largest = 0;
+  for (int n : P.atom_counts) {
+    largest = std::max(largest, round_up(n, kTile));
   }
-  return STORMM_OK;
+  if (rc == STORMM_OK && shape.wu_atom_capacity <= 0 && P.block == 0 && P.parts.empty() &&
+      P.maxa > kTwoBlockAtomsDouble && largest <= kTwoBlockAtomsDouble &&
+      static_cast<int>(P.wu.size()) > cus) {
+    pack_units(cost, P.atom_counts, P.lj_table_mode, kTwoBlockAtomsDouble, cus, wu_per_cu, true,
+               bins, bin_mode);
+    rc = append(P.wu_double, P.wu_sys_double, P.maxa_double);
+  }
+  return rc;
 }
 
 }  // namespace stormm_amd

@@ -108,6 +108,10 @@ struct SynthesisPlan {
   std::vector<int> sys_template;
   std::vector<WuDesc> wu;
   std::vector<WuSys> wu_sys;
+  // Units of the double-precision launches, where they take others (empty: the same).
+  std::vector<WuDesc> wu_double;
+  std::vector<WuSys> wu_sys_double;
+  int maxa_double = 0;
   std::vector<WuPart> parts;  // blocks of an evaluation in parts (empty: one block per unit)
   long long pairs = 0;
   long long task_count = 0;

@@ -45,7 +45,7 @@ extern "C" const char *stormm_last_error(void) { return g_last_error.c_str(); }
 struct stormm_synthesis {
   SynthesisPlan plan;
   DevMem atom_starts, atom_counts, q, ljp1, ljp2, lj_type, ljab, ljab14, rho, scr,
-      wu, wu_sys, tasks, masks, vterms, bond_par, angl_par, dihe_par,
+      wu, wu_sys, wu_double, wu_sys_double, tasks, masks, vterms, bond_par, angl_par, dihe_par,
       dihe14, status, cycles_run, rms_force, stop_flags, rst, parts;
   MMKit kit;
 };
@@ -154,6 +154,8 @@ extern "C" int stormm_synthesis_create(const stormm_topology_batch *batch,
   HIP_TRY(ag->scr.upload(P.ap.scr));
   HIP_TRY(ag->wu.upload(P.wu));
   HIP_TRY(ag->wu_sys.upload(P.wu_sys));
+  HIP_TRY(ag->wu_double.upload(P.wu_double));
+  HIP_TRY(ag->wu_sys_double.upload(P.wu_sys_double));
   HIP_TRY(ag->tasks.upload(P.ts.tasks));
   HIP_TRY(ag->masks.upload(P.ts.masks));
   HIP_TRY(ag->vterms.upload(P.ts.vterms));
@@ -1216,8 +1218,15 @@ static int check_writer(const stormm_synthesis *ag, const stormm_ps_writer *w, i
   return STORMM_OK;
 }
 
-static MMKit make_kit(const stormm_synthesis *ag, const stormm_ps_writer &w, const ScView *sc) {
+static MMKit make_kit(const stormm_synthesis *ag, const stormm_ps_writer &w, const ScView *sc,
+                      int precision) {
   MMKit k = ag->kit;
+  if (precision == STORMM_PREC_DOUBLE && !ag->plan.wu_double.empty()) {
+    k.wu = ag->wu_double.as<WuDesc>();
+    k.wu_sys = ag->wu_sys_double.as<WuSys>();
+    k.nwu = static_cast<int>(ag->plan.wu_double.size());
+    k.maxa = ag->plan.maxa_double;
+  }
   k.gpos_bits = w.gpos_bits;
   // Forces above 40 bits are accumulated at 40 bits inside a work unit and shifted on store.
   k.frc_bits = std::min(w.frc_bits, kMaxPlainFrcBits);
@@ -1360,7 +1369,7 @@ static int launch_terms(int32_t precision, const stormm_synthesis *ag,
   if (!(clash_d >= 0.0) || !(clash_r >= 0.0)) {
     return fail(STORMM_ERR_INVALID_ARGUMENT, "clash parameters must be non-negative");
   }
-  MMKit k = make_kit(ag, w, &sc);
+  MMKit k = make_kit(ag, w, &sc, precision);
   set_clash(k, precision, clash_d, clash_r);
   k.rst_step = step;
   HIP_TRY(launch_eval_on(ps, ag, precision == STORMM_PREC_DOUBLE ? 0 : 1, k, terms,
@@ -1637,7 +1646,7 @@ static int minimize_stepwise(int32_t precision, const stormm_synthesis *ag,
     return rc;
   }
   const int prec = (precision == STORMM_PREC_DOUBLE) ? 0 : 1;
-  MMKit k = make_kit(ag, w, &sc);
+  MMKit k = make_kit(ag, w, &sc, precision);
   k.store_overwrite = 1;
   LineKit lk = make_line_kit(ag, w, sc, lm, precision);
   if (use_parts(k, ag, ps)) {
@@ -1727,7 +1736,7 @@ static int minimize_graph(int32_t precision, const stormm_synthesis *ag_c,
   HIP_TRY(hipMemsetAsync(ag->stop_flags.ptr, 0, ns * sizeof(int), stream));
   HIP_TRY(hipMemsetAsync(ag->rms_force.ptr, 0, ns * sizeof(double), stream));
   const int prec = (precision == STORMM_PREC_DOUBLE) ? 0 : 1;
-  MMKit k = make_kit(ag, w, &sc);
+  MMKit k = make_kit(ag, w, &sc, precision);
   k.store_overwrite = 1;
   set_clash(k, precision, 0.0, 0.0);
   CgKit cg = make_cg_kit(ag, w, precision);
@@ -1906,7 +1915,7 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
   }
   const int ns = ag->plan.nsys;
   const int prec = (precision == STORMM_PREC_DOUBLE) ? 0 : 1;
-  MMKit k = make_kit(ag, w, &sc);
+  MMKit k = make_kit(ag, w, &sc, precision);
   k.store_overwrite = 1;
   set_clash(k, precision, 0.0, 0.0);
   CycleKit ck;
@@ -2256,7 +2265,7 @@ extern "C" int stormm_time_launch(int32_t precision, const stormm_synthesis *ag,
   if ((rc = check_writer(ag, &w, precision, &scv, false)) != STORMM_OK) {
     return rc;
   }
-  const MMKit k = make_kit(ag, w, &scv);
+  const MMKit k = make_kit(ag, w, &scv, precision);
   const int prec = (precision == STORMM_PREC_DOUBLE) ? 0 : 1;
   HIP_TRY(hipEventRecord(e0, st));
   for (int r = 0; r < repeats; r++) {

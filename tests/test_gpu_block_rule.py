@@ -53,3 +53,31 @@ def test_double_block_by_unit_size(count, natom, clash):
     forces, energies = run(None)
     f, e = run({"block_threads": 256})
     assert np.array_equal(f, forces) and np.array_equal(e, energies)
+
+
+# Units of more than 336 atoms are packed anew for double precision: as evaluated in them and as
+# evaluated in the units of an explicit capacity, in and out of a minimization.
+@pytest.mark.parametrize("cycles", [0, 3])
+def test_double_units(cycles):
+    topos, coords = synthetic.uniform_batch(1300, 17, 240, seed=79, gb=True)
+    shape = {"wu_atom_capacity": 512}
+    assert S.plan_synthesis(topos, shape).max_wu_atoms > 336
+    if cycles == 0:
+        forces, energies = evaluate(topos, coords, "double", None)
+        f, e = evaluate(topos, coords, "double", shape)
+        assert np.array_equal(f, forces) and np.array_equal(e, energies)
+        return
+
+    def minimize(shape):
+        ag = S.AtomGraphSynthesis(topos, shape)
+        ps = S.PhaseSpaceSynthesis(ag, 32, 40)
+        sc = S.ScoreCard(ag.system_count, 32)
+        ps.upload(coords)
+        controls = S.minimize_controls(cycles, sd_cycles=1)
+        line = S.LineMinimization(ag.system_count, 0.01)
+        S.launch_minimization("double", ag, ps, controls, sc, line)
+        return np.concatenate(ps.fixed()[0]), sc.accumulators()
+
+    xyz, energies = minimize(None)
+    x, e = minimize(shape)
+    assert np.array_equal(x, xyz) and np.array_equal(e, energies)
