@@ -113,4 +113,9 @@ struct SlotInitKit {
 };
 hipError_t launch_pool_init_slots(const SlotInitKit &k, hipStream_t stream);
 
+// Coordinates of one resident system into `out` (3 * natom words the device can write: pinned
+// host memory), axis after axis.
+hipError_t launch_pool_coordinates(const long long *x, const long long *y, const long long *z,
+                                   int natom, long long *out, hipStream_t stream);
+
 }  // namespace stormm_amd

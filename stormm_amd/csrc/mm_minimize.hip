@@ -629,4 +629,28 @@ hipError_t launch_pool_init_slots(const SlotInitKit &k, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// A resident system's coordinates straight into host memory, axis after axis.  Three blocking
+// copies of a few kB cost 47 us a system, nearly all of it their set-up and waits; one launch and
+// one wait cost 15 (a lane's eight bytes go out in 512-byte rows).
+__global__ void __launch_bounds__(256)
+    k_pool_coordinates(const long long *x, const long long *y, const long long *z, int natom,
+                       long long *out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < natom) {
+    out[i] = x[i];
+    out[natom + i] = y[i];
+    out[(2 * natom) + i] = z[i];
+  }
+}
+
+hipError_t launch_pool_coordinates(const long long *x, const long long *y, const long long *z,
+                                   int natom, long long *out, hipStream_t stream) {
+  if (natom == 0) {
+    return hipSuccess;
+  }
+  hipLaunchKernelGGL(k_pool_coordinates, dim3((natom + 255) / 256), dim3(256), 0, stream, x, y, z,
+                     natom, out);
+  return hipGetLastError();
+}
+
 }  // namespace stormm_amd

@@ -13,6 +13,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -98,6 +99,15 @@ struct stormm_pool {
   size_t up_tasks = 0, up_masks = 0, up_vterms = 0, up_bond = 0, up_angl = 0, up_dihe = 0,
          up_d14 = 0, up_ljab = 0, up_ljab14 = 0;
   DevMem wu, wu_sys, active, init_buf;
+  // Pinned host memory for one system's coordinates, and who is reading it.
+  long long *out_xyz = nullptr;
+  mutable std::mutex out_mutex;
+
+  ~stormm_pool() {
+    if (out_xyz != nullptr) {
+      (void)hipHostFree(out_xyz);
+    }
+  }
 };
 
 static int check_config(const stormm_pool_config *c) {
@@ -167,6 +177,8 @@ extern "C" int stormm_pool_create(const stormm_pool_config *cfg, stormm_pool **o
   if (p->cap_atoms < kGlobalPad) {
     return fail(STORMM_ERR_CAPACITY, "budget holds no atoms");
   }
+  HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&p->out_xyz),
+                        3 * kMaxWuAtoms * sizeof(long long), hipHostMallocDefault));
   const size_t na = static_cast<size_t>(p->cap_atoms), ns = static_cast<size_t>(p->cap_slots);
   for (DevMem *d : {&p->xcrd, &p->ycrd, &p->zcrd, &p->xfrc, &p->yfrc, &p->zfrc, &p->xprv,
                     &p->yprv, &p->zprv, &p->xcg, &p->ycg, &p->zcg}) {
@@ -993,14 +1005,12 @@ extern "C" int stormm_pool_coordinates(const stormm_pool *pool, int32_t slot, do
   }
   const int n = pool->slot_natom[slot];
   const int s0 = pool->slot_start[slot];
-  std::vector<long long> x(n), y(n), z(n);
+  std::lock_guard<std::mutex> lock(pool->out_mutex);
   HIP_TRY(hipDeviceSynchronize());
-  HIP_TRY(hipMemcpy(x.data(), pool->xcrd.as<long long>() + s0, n * sizeof(long long),
-                    hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(y.data(), pool->ycrd.as<long long>() + s0, n * sizeof(long long),
-                    hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(z.data(), pool->zcrd.as<long long>() + s0, n * sizeof(long long),
-                    hipMemcpyDeviceToHost));
+  HIP_TRY(launch_pool_coordinates(pool->xcrd.as<long long>() + s0, pool->ycrd.as<long long>() + s0,
+                                  pool->zcrd.as<long long>() + s0, n, pool->out_xyz, nullptr));
+  HIP_TRY(hipStreamSynchronize(nullptr));
+  const long long *x = pool->out_xyz, *y = x + n, *z = y + n;
   const double inv = std::ldexp(1.0, -pool->cfg.gpos_bits);
   for (int i = 0; i < n; i++) {
     if (xyz) {
