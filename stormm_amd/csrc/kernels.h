@@ -113,6 +113,17 @@ struct SlotInitKit {
 };
 hipError_t launch_pool_init_slots(const SlotInitKit &k, hipStream_t stream);
 
+// Values of admitted atoms from their staging buffer (eight rows of `count` words: coordinates and
+// parameters) to the pool's arrays, whose other values of these atoms become zero.
+struct AdmitKit {
+  int count;
+  const long long *words;
+  const int *types;
+  long long *word_out[8], *zero_out[9];
+  int *type_out;
+};
+hipError_t launch_pool_admit(const AdmitKit &k, hipStream_t stream);
+
 // Coordinates of one resident system into `out` (3 * natom words the device can write: pinned
 // host memory), axis after axis.
 hipError_t launch_pool_coordinates(const long long *x, const long long *y, const long long *z,

@@ -629,6 +629,33 @@ hipError_t launch_pool_init_slots(const SlotInitKit &k, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Admitted atoms' values to their places in the pool, from one staged copy.  Twelve copies and
+// nine fills of a few kB each cost 245 us an admission more, nearly all of it set-up and waits
+// (20 conformers of one molecule 405 us, now 160).
+__global__ void __launch_bounds__(256) k_pool_admit(AdmitKit k) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= k.count) {
+    return;
+  }
+#pragma unroll
+  for (int v = 0; v < 8; v++) {
+    k.word_out[v][i] = k.words[(static_cast<size_t>(v) * k.count) + i];
+  }
+#pragma unroll
+  for (int v = 0; v < 9; v++) {
+    k.zero_out[v][i] = 0;
+  }
+  k.type_out[i] = k.types[i];
+}
+
+hipError_t launch_pool_admit(const AdmitKit &k, hipStream_t stream) {
+  if (k.count == 0) {
+    return hipSuccess;
+  }
+  hipLaunchKernelGGL(k_pool_admit, dim3((k.count + 255) / 256), dim3(256), 0, stream, k);
+  return hipGetLastError();
+}
+
 // A resident system's coordinates straight into host memory, axis after axis.  Three blocking
 // copies of a few kB cost 47 us a system, nearly all of it their set-up and waits; one launch and
 // one wait cost 15 (a lane's eight bytes go out in 512-byte rows).

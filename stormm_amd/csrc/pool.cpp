@@ -34,6 +34,10 @@ constexpr size_t kPoolBytesPerAtom = (12 * 8) + (9 * 8) + 4;
 // Device bytes per system slot: layout (2 ints), step / stop flag (2 ints), RMS force, nine
 // line-search doubles and a ScoreCard row.
 constexpr size_t kPoolBytesPerSlot = (4 * 4) + 8 + (9 * 8) + (kScoreStride * 8);
+// Atoms of an admission staged at once, and the bytes of each: three coordinates, five parameters
+// and the LJ type.
+constexpr int kAdmitChunk = 32768;
+constexpr size_t kAdmitBytesPerAtom = (8 * 8) + 4;
 // Share of the budget kept for work templates (tile tasks, masks, valence terms, parameters).
 constexpr double kTemplateShare = 0.2;
 
@@ -380,6 +384,90 @@ static int admit_templates(stormm_pool *p, const stormm_topology_batch *batch,
   return fail(STORMM_ERR_CAPACITY, "work templates exceed the pool's template budget");
 }
 
+// Brings an admission's entries to the device: one staged copy and a kernel per kAdmitChunk atoms.
+static hipError_t upload_entries(stormm_pool *p, int start, int total,
+                                 const std::vector<long long> &cx,
+                                 const std::vector<long long> &cy,
+                                 const std::vector<long long> &cz, const AtomParams &ap,
+                                 const std::vector<int> &e_slot, const std::vector<int> &e_start,
+                                 const std::vector<int> &e_natom) {
+  const int ns = static_cast<int>(e_slot.size());
+  const size_t entry_bytes = 3 * static_cast<size_t>(ns) * sizeof(int);
+  const size_t most = static_cast<size_t>(std::min(total, kAdmitChunk));
+  const size_t need = entry_bytes + (most * kAdmitBytesPerAtom) + 8;
+  if (p->init_buf.bytes < need) {
+    const hipError_t e = p->init_buf.alloc(need + (need / 2));
+    if (e != hipSuccess) {
+      return e;
+    }
+  }
+  std::vector<char> stage(need);
+  AdmitKit k;
+  long long *crd[3] = {p->xcrd.as<long long>(), p->ycrd.as<long long>(), p->zcrd.as<long long>()};
+  DevMem *zero[9] = {&p->xfrc, &p->yfrc, &p->zfrc, &p->xprv, &p->yprv, &p->zprv, &p->xcg, &p->ycg,
+                     &p->zcg};
+  DevMem *par[5] = {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr};
+  const void *src[8] = {cx.data(), cy.data(), cz.data(), ap.q.data(), ap.ljp1.data(),
+                        ap.ljp2.data(), ap.rho.data(), ap.scr.data()};
+  for (int first = 0; first < total; first += kAdmitChunk) {
+    const int count = std::min(total - first, kAdmitChunk);
+    const size_t row = static_cast<size_t>(count) * sizeof(long long);
+    for (int v = 0; v < 8; v++) {
+      std::memcpy(stage.data() + v * row,
+                  static_cast<const char *>(src[v]) + static_cast<size_t>(first) * 8, row);
+    }
+    size_t at = 8 * row;
+    std::memcpy(stage.data() + at, ap.lj_type.data() + first, count * sizeof(int));
+    at += count * sizeof(int);
+    const bool last = (first + count == total);
+    const size_t entries = at;
+    if (last) {
+      for (const std::vector<int> *v : {&e_slot, &e_start, &e_natom}) {
+        std::memcpy(stage.data() + at, v->data(), ns * sizeof(int));
+        at += ns * sizeof(int);
+      }
+    }
+    char *dev = p->init_buf.as<char>();
+    hipError_t err = hipMemcpy(dev, stage.data(), at, hipMemcpyHostToDevice);
+    if (err != hipSuccess) {
+      return err;
+    }
+    k.count = count;
+    k.words = reinterpret_cast<const long long *>(dev);
+    k.types = reinterpret_cast<const int *>(dev + 8 * row);
+    const size_t to = static_cast<size_t>(start) + first;
+    for (int v = 0; v < 8; v++) {
+      k.word_out[v] = ((v < 3) ? crd[v] : par[v - 3]->as<long long>()) + to;
+    }
+    for (int v = 0; v < 9; v++) {
+      k.zero_out[v] = zero[v]->as<long long>() + to;
+    }
+    k.type_out = p->lj_type.as<int>() + to;
+    err = launch_pool_admit(k, nullptr);
+    if (err == hipSuccess && last) {
+      SlotInitKit ik;
+      ik.count = ns;
+      ik.cap_slots = p->cap_slots;
+      ik.slots = reinterpret_cast<const int *>(dev + entries);
+      ik.starts = ik.slots + ns;
+      ik.natoms = ik.starts + ns;
+      ik.slot_start = p->starts.as<int>();
+      ik.slot_natom = p->natoms.as<int>();
+      ik.steps = p->steps.as<int>();
+      ik.done = p->done.as<int>();
+      ik.rms = p->rms.as<double>();
+      ik.line = p->line.as<double>();
+      ik.scorecard = p->scorecard.as<long long>();
+      ik.dx0 = p->cfg.minimize.initial_step;
+      err = launch_pool_init_slots(ik, nullptr);
+    }
+    if (err != hipSuccess) {
+      return err;
+    }
+  }
+  return hipDeviceSynchronize();
+}
+
 // Admits `count` systems; entry e is system sys_of[e] of the batch with coordinates at
 // xyz + 3 * (first atom of entry e), entries laid out one after another.
 static int admit_entries(stormm_pool *pool, const stormm_topology_batch *batch,
@@ -465,28 +553,25 @@ static int admit_entries(stormm_pool *pool, const stormm_topology_batch *batch,
       return fail(STORMM_ERR_HIP, std::string("template upload: ") + hipGetErrorString(e));
     }
   }
-  auto put = [&](DevMem &d, const void *src, size_t elt) {
-    return hipMemcpy(static_cast<char *>(d.ptr) + static_cast<size_t>(start) * elt, src,
-                     static_cast<size_t>(total) * elt, hipMemcpyHostToDevice);
-  };
-  auto zero = [&](DevMem &d) {
-    return hipMemset(static_cast<char *>(d.ptr) + static_cast<size_t>(start) * sizeof(long long),
-                     0, static_cast<size_t>(total) * sizeof(long long));
-  };
-  HIP_TRY(put(p->xcrd, cx.data(), sizeof(long long)));
-  HIP_TRY(put(p->ycrd, cy.data(), sizeof(long long)));
-  HIP_TRY(put(p->zcrd, cz.data(), sizeof(long long)));
-  for (DevMem *d : {&p->xfrc, &p->yfrc, &p->zfrc, &p->xprv, &p->yprv, &p->zprv, &p->xcg,
-                    &p->ycg, &p->zcg}) {
-    HIP_TRY(zero(*d));
-  }
-  HIP_TRY(put(p->q, ap.q.data(), sizeof(double)));
-  HIP_TRY(put(p->ljp1, ap.ljp1.data(), sizeof(double)));
-  HIP_TRY(put(p->ljp2, ap.ljp2.data(), sizeof(double)));
-  HIP_TRY(put(p->rho, ap.rho.data(), sizeof(double)));
-  HIP_TRY(put(p->scr, ap.scr.data(), sizeof(double)));
-  HIP_TRY(put(p->lj_type, ap.lj_type.data(), sizeof(int)));
+  // The new systems' slots, and fresh per-system state (LineMinimization::primeMoveLengths:
+  // l_move = dx0, the rest zero).
+  std::vector<int> e_slot(ns), e_start(ns), e_natom(ns);
   off = 0;
+  for (int e = 0; e < ns; e++) {
+    e_slot[e] = p->free_slots[p->free_slots.size() - 1 - static_cast<size_t>(e)];
+    e_start[e] = start + off;
+    e_natom[e] = batch->atom_counts[sys_of[e]];
+    off += round_up(e_natom[e], kGlobalPad);
+  }
+  {
+    const hipError_t e = upload_entries(p, start, total, cx, cy, cz, ap, e_slot, e_start, e_natom);
+    if (e != hipSuccess) {
+      give_atoms(p, start, total);
+      rollback_templates(p->ts, mark);
+      invalidate_template_upload(p);
+      return fail(STORMM_ERR_HIP, std::string("admission upload: ") + hipGetErrorString(e));
+    }
+  }
   int rid;
   if (!p->free_range_ids.empty()) {
     rid = p->free_range_ids.back();
@@ -499,48 +584,18 @@ static int admit_entries(stormm_pool *pool, const stormm_topology_batch *batch,
   p->ranges[rid].start = start;
   p->ranges[rid].len = total;
   p->ranges[rid].refs = ns;
-  std::vector<int> e_slot(ns), e_start(ns), e_natom(ns);
   for (int e = 0; e < ns; e++) {
-    const int s = sys_of[e];
-    const int slot = p->free_slots.back();
+    const int slot = e_slot[e];
     p->free_slots.pop_back();
-    p->slot_start[slot] = start + off;
-    p->slot_natom[slot] = batch->atom_counts[s];
+    p->slot_start[slot] = e_start[e];
+    p->slot_natom[slot] = e_natom[e];
     p->slot_template[slot] = tids[e];
     p->slot_live[slot] = 1;
     p->slot_table[slot] = p->ts.templates[tids[e]].lb ? 0 : 1;
     p->slot_range[slot] = rid;
     p->template_refs[tids[e]]++;
-    off += round_up(batch->atom_counts[s], kGlobalPad);
-    e_slot[e] = slot;
-    e_start[e] = p->slot_start[slot];
-    e_natom[e] = p->slot_natom[slot];
     slots[e] = slot;
   }
-  // Fresh per-system state (LineMinimization::primeMoveLengths: l_move = dx0, the rest zero).
-  if (p->init_buf.bytes < 3 * static_cast<size_t>(ns) * sizeof(int)) {
-    HIP_TRY(p->init_buf.alloc(6 * static_cast<size_t>(ns) * sizeof(int)));
-  }
-  int *ib = p->init_buf.as<int>();
-  HIP_TRY(hipMemcpy(ib, e_slot.data(), ns * sizeof(int), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(ib + ns, e_start.data(), ns * sizeof(int), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(ib + 2 * ns, e_natom.data(), ns * sizeof(int), hipMemcpyHostToDevice));
-  SlotInitKit ik;
-  ik.count = ns;
-  ik.cap_slots = p->cap_slots;
-  ik.slots = ib;
-  ik.starts = ib + ns;
-  ik.natoms = ib + 2 * ns;
-  ik.slot_start = p->starts.as<int>();
-  ik.slot_natom = p->natoms.as<int>();
-  ik.steps = p->steps.as<int>();
-  ik.done = p->done.as<int>();
-  ik.rms = p->rms.as<double>();
-  ik.line = p->line.as<double>();
-  ik.scorecard = p->scorecard.as<long long>();
-  ik.dx0 = p->cfg.minimize.initial_step;
-  HIP_TRY(launch_pool_init_slots(ik, nullptr));
-  HIP_TRY(hipDeviceSynchronize());
   return STORMM_OK;
 }
 
