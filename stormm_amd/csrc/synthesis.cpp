@@ -2291,7 +2291,9 @@ extern "C" int stormm_autotune_launch_shape(const stormm_topology_batch *batch,
   for (int s = 0; s < batch->system_count; s++) {
     maxn = std::max(maxn, batch->atom_counts[s]);
   }
-  const int caps[4] = {128, 256, 384, 512};
+  // In double precision two units of 384 atoms do not share a compute unit, two of 336 do.
+  const int caps[4] = {128, 256, (precision == STORMM_PREC_DOUBLE) ? kTwoBlockAtomsDouble : 384,
+                       512};
   const int per_cu[4] = {1, 2, 3, 4};
   const int blocks[3] = {256, 512, 1024};
   double best_t = 1.0e30;
