@@ -19,7 +19,7 @@ Further workloads ride on the same line (skip them with --no-extra):
     takes: kernel time next to the combining-rule path's, and FP32 errors on 16 systems.
   "minimization": 4096 systems, N ~ U[16, 128], starts perturbed by N(0, 0.3 A), 500 cycles
     (50 steepest descent, then conjugate gradient, the first 25 clash-damped) in FP32: the fused
-    cycle kernels captured whole in one HIP graph (whole batch, and once per size class), the
+    cycle kernels issued mostly from a graph of eight cycles (whole batch, and once per size class), the
     reference's per-step launch sequence, and that sequence captured per cycle and replayed,
     with the oracle's minimizer on host threads as the CPU rate.
   "large_batch": 16384 systems, N ~ U[32, 96]: FP32 and FP64 evaluation throughput and the

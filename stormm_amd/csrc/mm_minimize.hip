@@ -1,6 +1,6 @@
 // Line-minimization kernels: the conjugate-gradient direction update and the four line moves of
-// the reference's launch-per-step minimizer, plus the persistent minimizer that runs every cycle
-// of a work unit's systems inside one block.
+// the reference's launch-per-step minimizer, the evaluation kernels that make the pending line
+// move themselves, and the serving pool's transfer kernels.
 #include <algorithm>
 #include <mutex>
 

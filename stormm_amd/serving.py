@@ -339,8 +339,8 @@ def serve_batched(requests: Sequence[Request], precision: str = "single",
                   total_cycles: int = 300, sd_cycles: int = 50, dx0: float = 0.01,
                   conv_rms: float = 0.1, shape=None) -> Dict[str, float]:
     """The batch minimizer on the same conformers: every conformer of every request in one
-    AtomGraphSynthesis / PhaseSpaceSynthesis, minimized by one call (the fused cycle kernels
-    captured whole in a graph) with the same RMS-force stop and cycle limit.  The synthesis
+    AtomGraphSynthesis / PhaseSpaceSynthesis, minimized by one call (the fused cycle kernels,
+    mostly replayed from a graph of eight cycles) with the same RMS-force stop and cycle limit.  The synthesis
     build and upload are timed too, as the serving pool's admissions are."""
     from . import synthesis as S
     bits = (32, 23, 26) if precision == "single" else (32, 40, 32)
