@@ -517,7 +517,9 @@ typedef struct {
   double salt_concentration;
   double coulomb_constant;
   stormm_minimize_controls minimize; /* cycle limit, steepest-descent cycles, dx0, RMS stop    */
-  stormm_launch_shape shape;       /* work-unit shaping (zero = defaults)                       */
+  stormm_launch_shape shape;       /* work-unit shaping (zero = defaults); capacities above 512
+                                      count as 512, block sizes become whole wavefronts, at
+                                      least 256 threads                                         */
 } stormm_pool_config;
 
 int stormm_pool_create(const stormm_pool_config *config, stormm_pool **out);

@@ -32,10 +32,11 @@ def _compile(src: str) -> str:
 ROOT = os.path.dirname(HERE)
 CAPI_DIR = os.path.join(ROOT, "tests", "capi")
 CAPI_BIN = os.path.join(CAPI_DIR, "bin")
-# Test programs written against the C-ABI (tests/capi/*.cpp): the host check of the 95-bit
-# helpers, and a C++ caller that owns its device arrays.
-CAPI_PROGRAMS = {"int95_host": [], "kit_boundary": ["-L", HERE, "-lstormm_amd",
-                                                    "-Wl,-rpath,$ORIGIN/../../../stormm_amd"]}
+# Test programs (tests/capi/*.cpp): host checks of the 95-bit helpers and of the launch rules, and
+# a C++ caller of the C-ABI that owns its device arrays.
+CAPI_PROGRAMS = {"int95_host": [], "launch_host": [],
+                 "kit_boundary": ["-L", HERE, "-lstormm_amd",
+                                  "-Wl,-rpath,$ORIGIN/../../../stormm_amd"]}
 
 
 def build_capi_programs(verbose: bool = False) -> None:

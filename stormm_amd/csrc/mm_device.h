@@ -420,10 +420,14 @@ static_assert(2 * WuLds<double>::bytes(kTwoBlockAtomsDouble, kEvalBlock / 64) <=
 // one block takes the whole compute unit (1024 systems of 24-256 atoms 157 us against 178 at
 // half the size), and a unit alone that is too small for 16 wavefronts takes 8 (200 systems of
 // 100 atoms 37 us against 40).  A HEAVY kernel's registers hold 12 wavefronts instead of 16.
+// A size that was asked for (the pool takes any) becomes whole wavefronts, no fewer than cover a
+// unit's atoms at stage_load's two to a thread.  Results do not depend on the size.
 template <typename T, bool HEAVY> inline int eval_block(const MMKit &k, int blocks) {
   constexpr int limit = EvalBlockLimit<T, HEAVY>::value;
+  static_assert(limit >= kMinEvalBlock && limit % 64 == 0, "a block is whole wavefronts");
   if (k.block > 0) {
-    return (k.block < limit) ? k.block : limit;
+    const int asked = (k.block < limit) ? k.block : limit;
+    return (asked < kMinEvalBlock) ? kMinEvalBlock : (asked + 63) / 64 * 64;
   }
   if (sizeof(T) == 4) {
     return (blocks <= k.cus) ? kEvalBlockSparse : kEvalBlock;

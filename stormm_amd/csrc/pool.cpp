@@ -757,7 +757,9 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
     index[i] = s;
   }
   const stormm_launch_shape &sh = p->cfg.shape;
-  const int cap = (sh.wu_atom_capacity > 0) ? sh.wu_atom_capacity : kMaxWuAtoms;
+  // A unit holds kMaxWuAtoms at most, whatever capacity was asked for.
+  const int cap = (sh.wu_atom_capacity > 0) ? std::min<int>(sh.wu_atom_capacity, kMaxWuAtoms)
+                                            : kMaxWuAtoms;
   const int per_cu = (sh.target_wu_per_cu > 0) ? sh.target_wu_per_cu : 2;
   const int block = std::max(sh.block_threads, 0);
   std::vector<std::vector<int>> bins;
