@@ -32,9 +32,10 @@ def _compile(src: str) -> str:
 ROOT = os.path.dirname(HERE)
 CAPI_DIR = os.path.join(ROOT, "tests", "capi")
 CAPI_BIN = os.path.join(CAPI_DIR, "bin")
-# Test programs (tests/capi/*.cpp): host checks of the 95-bit helpers and of the launch rules, and
-# a C++ caller of the C-ABI that owns its device arrays.
-CAPI_PROGRAMS = {"int95_host": [], "launch_host": [],
+# Test programs (tests/capi/*.cpp): host checks of the 95-bit helpers and of the launch rules, a
+# device check of the double-precision functions, and a C++ caller of the C-ABI that owns its
+# device arrays.
+CAPI_PROGRAMS = {"int95_host": [], "launch_host": [], "math_device": DEVICE_FLAGS,
                  "kit_boundary": ["-L", HERE, "-lstormm_amd",
                                   "-Wl,-rpath,$ORIGIN/../../../stormm_amd"]}
 

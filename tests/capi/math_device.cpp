@@ -1,0 +1,125 @@
+// Errors of the double-precision functions of the evaluation kernels (stormm_amd/csrc/mm_device.h)
+// on the device, in units of the last place against 80-bit arithmetic on the host, over the
+// arguments that the kernels give them.  Arguments: the names of the functions to check.
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <functional>
+#include <random>
+#include <vector>
+
+#include <hip/hip_runtime.h>
+
+#include "../../stormm_amd/csrc/mm_device.h"
+
+using namespace stormm_amd;
+using D = Prec<double>;
+
+struct Exp {
+  static __device__ double eval(double x, double) { return D::exp(x); }
+};
+
+template <typename F> __global__ void k_eval(const double *x, const double *y, double *out, int n) {
+  const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < n) {
+    out[i] = F::eval(x[i], y[i]);
+  }
+}
+
+#define TRY(call)                                                     \
+  do {                                                                \
+    const hipError_t e_ = (call);                                     \
+    if (e_ != hipSuccess) {                                           \
+      std::printf("%s: %s\n", #call, hipGetErrorString(e_));          \
+      return false;                                                   \
+    }                                                                 \
+  } while (0)
+
+template <typename F>
+static bool evaluate(const std::vector<double> &x, const std::vector<double> &y,
+                     std::vector<double> &out) {
+  const int n = static_cast<int>(x.size());
+  const size_t bytes = x.size() * sizeof(double);
+  double *d = nullptr;
+  TRY(hipMalloc(&d, 3 * bytes));
+  TRY(hipMemcpy(d, x.data(), bytes, hipMemcpyHostToDevice));
+  TRY(hipMemcpy(d + n, y.data(), bytes, hipMemcpyHostToDevice));
+  hipLaunchKernelGGL((k_eval<F>), dim3((n + 255) / 256), dim3(256), 0, 0, d, d + n, d + 2 * n, n);
+  TRY(hipGetLastError());
+  out.resize(x.size());
+  TRY(hipMemcpy(out.data(), d + 2 * n, bytes, hipMemcpyDeviceToHost));
+  TRY(hipFree(d));
+  return true;
+}
+
+struct Range {
+  double lo, hi;
+};
+
+// The largest error over 2^18 arguments of each range; `real` is the exact function.
+template <typename F>
+static bool check(const char *name, double most, const std::vector<Range> &ranges,
+                  const std::function<long double(long double, long double)> &real) {
+  bool ok = true;
+  for (size_t r = 0; r < ranges.size(); r++) {
+    std::mt19937_64 rng(7000 + r);
+    std::uniform_real_distribution<double> u(0.0, 1.0);
+    std::vector<double> x(1 << 18), y(1 << 18), out;
+    for (size_t i = 0; i < x.size(); i++) {
+      // Every other argument spread over the logarithm where the range does not cross zero.
+      const double lo = ranges[r].lo, hi = ranges[r].hi;
+      x[i] = (lo > 0.0 && (i & 1)) ? lo * std::pow(hi / lo, u(rng)) : lo + ((hi - lo) * u(rng));
+      y[i] = 0.1 + (3.0 * u(rng));
+    }
+    if (!evaluate<F>(x, y, out)) {
+      return false;
+    }
+    long double worst = 0.0L;
+    double at = 0.0;
+    for (size_t i = 0; i < x.size(); i++) {
+      const long double want = real(x[i], y[i]);
+      int e = 0;
+      (void)std::frexp(want, &e);
+      const long double err = std::fabs((out[i] - want) / std::ldexp(1.0L, e - 53));
+      if (!(err <= worst)) {
+        worst = err;
+        at = x[i];
+      }
+    }
+    std::printf("%s [%g, %g]: %.4Lf ulp at %.17g (at most %g)\n", name, ranges[r].lo, ranges[r].hi,
+                worst, at, most);
+    ok = ok && worst <= most;
+  }
+  return ok;
+}
+
+// A value that is not a number stays one.
+template <typename F> static bool keeps_nan(const char *name) {
+  std::vector<double> out;
+  const bool ok = evaluate<F>({std::nan(""), -std::nan("")}, {1.0, 1.0}, out) &&
+                  std::isnan(out[0]) && std::isnan(out[1]);
+  std::printf("%s of a NaN: %s\n", name, ok ? "NaN" : "a number");
+  return ok;
+}
+
+static bool check_named(const char *name) {
+  const std::string f(name);
+  if (f == "exp") {
+    // The device library's bound is one unit.
+    return check<Exp>(name, 1.0, {{-1.0, 0.0}, {-5.0, -1.0}, {-20.0, -5.0}, {-40.0, -20.0},
+                                  {-700.0, -40.0}},
+                      [](long double x, long double) { return std::exp(x); }) &&
+           keeps_nan<Exp>(name);
+  }
+  std::printf("no function %s\n", name);
+  return false;
+}
+
+int main(int argc, char **argv) {
+  bool ok = argc > 1;
+  for (int i = 1; i < argc; i++) {
+    ok = check_named(argv[i]) && ok;
+  }
+  std::printf(ok ? "math ok\n" : "math FAILED\n");
+  return ok ? 0 : 1;
+}
