@@ -18,6 +18,9 @@ using D = Prec<double>;
 struct Exp {
   static __device__ double eval(double x, double) { return D::exp(x); }
 };
+struct Log {
+  static __device__ double eval(double x, double) { return D::log(x); }
+};
 
 template <typename F> __global__ void k_eval(const double *x, const double *y, double *out, int n) {
   const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
@@ -110,6 +113,12 @@ static bool check_named(const char *name) {
                                   {-700.0, -40.0}},
                       [](long double x, long double) { return std::exp(x); }) &&
            keeps_nan<Exp>(name);
+  }
+  if (f == "log") {
+    // Half a unit from the last sum and less than a tenth from the terms below it.
+    return check<Log>(name, 0.6, {{0.02, 0.5}, {0.5, 0.9}, {0.9, 1.0}, {1.0, 1.1}, {1.1, 50.0}},
+                      [](long double x, long double) { return std::log(x); }) &&
+           keeps_nan<Log>(name);
   }
   std::printf("no function %s\n", name);
   return false;
