@@ -60,13 +60,16 @@ template <> struct Prec<double> {
   // ln 2 in two parts, the first of 36 bits.
   static constexpr double kLn2High = 0x1.62e42fefap-1, kLn2Low = 0x1.cf79abc9e3b39p-40;
   // The hardware estimates leave residuals e = 1 - x y (reciprocal) and 1 - x y^2 (reciprocal
-  // square root) of at most 2^-24 and 2^-23 (measured over a full octave); the binomial series
-  // y (1 + e + e^2) and y (1 + e / 2 + 3 e^2 / 8) leave about e^3, below the last bit.  Three and
-  // five instructions after the estimate, where two Newton-Raphson steps took four and eight.  For
-  // positive, finite, normal arguments (distances and radii here).
+  // square root) of at most 2^-24 and 2^-22 (measured over a full octave); the binomial series
+  // y (1 + e + e^2) and y (1 + e / 2 + 3 e^2 / 8) leave about e^3, below the last bit.  The root's
+  // estimate is cut to 26 bits first, so that y^2 and with it the residual are exact: 0.5005 units
+  // in the last place at most, where the rounding of x y left 0.99.  Three and six instructions
+  // after the estimate, where two Newton-Raphson steps took four and eight.  For positive, finite,
+  // normal arguments (distances and radii here).
   static __device__ __forceinline__ double rsqrt(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * y, y, 1.0);
+    const double y = __longlong_as_double(__double_as_longlong(__builtin_amdgcn_rsq(x)) &
+                                          ~0x7ffffffLL);
+    const double e = fma(-x, y * y, 1.0);
     return fma(y * e, fma(0.375, e, 0.5), y);
   }
   static __device__ __forceinline__ double rcp(double x) {

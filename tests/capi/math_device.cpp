@@ -21,6 +21,9 @@ struct Exp {
 struct Log {
   static __device__ double eval(double x, double) { return D::log(x); }
 };
+struct Rsqrt {
+  static __device__ double eval(double x, double) { return D::rsqrt(x); }
+};
 
 template <typename F> __global__ void k_eval(const double *x, const double *y, double *out, int n) {
   const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
@@ -119,6 +122,11 @@ static bool check_named(const char *name) {
     return check<Log>(name, 0.6, {{0.02, 0.5}, {0.5, 0.9}, {0.9, 1.0}, {1.0, 1.1}, {1.1, 50.0}},
                       [](long double x, long double) { return std::log(x); }) &&
            keeps_nan<Log>(name);
+  }
+  if (f == "rsqrt") {
+    // Half a unit from the last sum; the residual is exact and e^3 a thousandth of a unit.
+    return check<Rsqrt>(name, 0.51, {{0.25, 1.0}, {1.0, 4.0}, {1.0, 1.0e5}, {1.0e-6, 1.0}},
+                        [](long double x, long double) { return 1.0L / std::sqrt(x); });
   }
   std::printf("no function %s\n", name);
   return false;

@@ -11,7 +11,7 @@ from stormm_amd import build
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("function", ["exp", "log"])
+@pytest.mark.parametrize("function", ["exp", "log", "rsqrt"])
 def test_error(function):
     exe = os.path.join(build.CAPI_BIN, "math_device")
     if not os.path.exists(exe):
