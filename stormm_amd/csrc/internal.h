@@ -170,6 +170,7 @@ struct MMKit {
   const double2 *ljab14;     // 1:4 A, B per system table
   const double *rho;         // intrinsic radius - offset
   const double *scr;         // screening factor * rho
+  const double *pbr;         // intrinsic radius
   double gb_alpha, gb_beta, gb_gamma;  // OBC constants of the solvent model
   long long *xcrd, *ycrd, *zcrd;
   long long *xfrc, *yfrc, *zfrc;

@@ -113,13 +113,14 @@ struct SlotInitKit {
 };
 hipError_t launch_pool_init_slots(const SlotInitKit &k, hipStream_t stream);
 
-// Values of admitted atoms from their staging buffer (eight rows of `count` words: coordinates and
-// parameters) to the pool's arrays, whose other values of these atoms become zero.
+// Values of admitted atoms from their staging buffer (rows of `count` words: three coordinates and
+// six parameters) to the pool's arrays, whose other values of these atoms become zero.
+constexpr int kAdmitRows = 9;
 struct AdmitKit {
   int count;
   const long long *words;
   const int *types;
-  long long *word_out[8], *zero_out[9];
+  long long *word_out[kAdmitRows], *zero_out[9];
   int *type_out;
 };
 hipError_t launch_pool_admit(const AdmitKit &k, hipStream_t stream);

@@ -749,38 +749,23 @@ __device__ __forceinline__ void stage_radii(StageCtx<T> &c, const MMKit &k, doub
       continue;
     }
     const double psi = static_cast<double>(L.atom[a].psi) * ldexp(1.0, -kPsiBits);
-    const double rho = k.rho[g];
-    using D = Prec<double>;
-    double R, invR;
-    if (k.igb == 1) {
-      invR = D::rcp(rho) + psi;
-      R = (invR < 0.0) ? 30.0 : 1.0 / invR;
-      invR = 1.0 / R;
-    }
-    else {
-      const double fipsi = psi * (-rho);
-      const double al = k.gb_alpha, be = k.gb_beta, ga = k.gb_gamma;
-      const double inv_pbr = D::rcp(rho + kGbOffset);  // of the intrinsic radius
-      const double thi = D::tanh((al - (be * fipsi) + (ga * fipsi * fipsi)) * fipsi);
-      invR = D::rcp(rho) - (thi * inv_pbr);
-      R = D::rcp(invR);
-      if (FORCES) {
-        // dR/dpsi of the OBC model (nonbonded_potential.tpp:985-1017), kept for the chain rule
-        // in the accumulator slot whose psi is no longer needed.
-        const double dr_dpsi = (al - ((2.0 * be) - (3.0 * ga * fipsi)) * fipsi) *
-                               (1.0 - thi * thi) * rho * inv_pbr;
-        L.atom[a].psi = __double_as_longlong(dr_dpsi);
-      }
+    const BornRadius b = born_radius(k.igb, k.gb_alpha, k.gb_beta, k.gb_gamma, k.rho[g],
+                                     k.pbr[g], psi);
+    const double R = b.R;
+    if (FORCES && k.igb != 1) {
+      // Kept for the chain rule in the accumulator slot whose psi is no longer needed.
+      L.atom[a].psi = __double_as_longlong(b.dr_dpsi);
     }
     L.atom[a].nb.rad = static_cast<T>(R);
-    inv_radius(L, a) = static_cast<T>(invR);
+    inv_radius(L, a) = static_cast<T>(b.inv_R);
     // q holds charge * sqrt(Coulomb), so q^2 = Coulomb * charge^2.
     const double qg = k.q[g];
-    const double expmkf = ((k.kappa != 0.0) ? D::exp(-kGbKscale * k.kappa * R) : 1.0) * inv_diel;
+    const double expmkf = ((k.kappa != 0.0) ? Prec<double>::exp(-kGbKscale * k.kappa * R) : 1.0) *
+                          inv_diel;
     const double dielfac = 1.0 - expmkf;
     const double atmq2h = 0.5 * qg * qg;
     const double atmqd2h = atmq2h * dielfac;
-    const double contrib = -atmqd2h * invR;
+    const double contrib = -atmqd2h / R;
     if (c.part != 0) {
       continue;  // the unit's first part adds the self terms
     }

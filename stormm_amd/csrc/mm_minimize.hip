@@ -638,7 +638,7 @@ __global__ void __launch_bounds__(256) k_pool_admit(AdmitKit k) {
     return;
   }
 #pragma unroll
-  for (int v = 0; v < 8; v++) {
+  for (int v = 0; v < kAdmitRows; v++) {
     k.word_out[v][i] = k.words[(static_cast<size_t>(v) * k.count) + i];
   }
 #pragma unroll

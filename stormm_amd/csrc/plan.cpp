@@ -876,6 +876,7 @@ int fill_atom_parameters(const stormm_topology_batch *b, const SystemTerms &t, i
     }
     const double pr = (b->pb_radii != nullptr) ? b->pb_radii[src] : 0.0;
     const double sc = (b->gb_screen != nullptr) ? b->gb_screen[src] : 0.0;
+    ap.pbr[g] = pr;
     ap.rho[g] = pr - 0.09;
     ap.scr[g] = sc * (pr - 0.09);
     if (sm.igb != 0 && ap.rho[g] <= 0.0) {

@@ -81,7 +81,7 @@ struct SolventModel {
 
 // Per-atom parameter arrays (one entry per padded global atom).
 struct AtomParams {
-  std::vector<double> q, ljp1, ljp2, rho, scr;
+  std::vector<double> q, ljp1, ljp2, rho, scr, pbr;
   std::vector<int> lj_type;
   void assign(size_t n) {
     q.assign(n, 0.0);
@@ -89,6 +89,7 @@ struct AtomParams {
     ljp2.assign(n, 0.0);
     rho.assign(n, 0.0);
     scr.assign(n, 0.0);
+    pbr.assign(n, 0.0);
     lj_type.assign(n, 0);
   }
 };

@@ -27,17 +27,16 @@ using namespace stormm_amd;
 
 namespace {
 
-// Device bytes counted per resident atom: int64 coordinates, forces, previous forces and CG
-// direction (12 x 8), nine 8-byte values (five parameters, the three sums of evaluations in parts
-// and room for one) and the LJ type.
+// Device bytes per resident atom: int64 coordinates, forces, previous forces and CG direction
+// (12 x 8), six double parameters, the three sums of evaluations in parts and the LJ type.
 constexpr size_t kPoolBytesPerAtom = (12 * 8) + (9 * 8) + 4;
 // Device bytes per system slot: layout (2 ints), step / stop flag (2 ints), RMS force, nine
 // line-search doubles and a ScoreCard row.
 constexpr size_t kPoolBytesPerSlot = (4 * 4) + 8 + (9 * 8) + (kScoreStride * 8);
-// Atoms of an admission staged at once, and the bytes of each: three coordinates, five parameters
+// Atoms of an admission staged at once, and the bytes of each: three coordinates, six parameters
 // and the LJ type.
 constexpr int kAdmitChunk = 32768;
-constexpr size_t kAdmitBytesPerAtom = (8 * 8) + 4;
+constexpr size_t kAdmitBytesPerAtom = (kAdmitRows * 8) + 4;
 // Share of the budget kept for work templates (tile tasks, masks, valence terms, parameters).
 constexpr double kTemplateShare = 0.2;
 
@@ -90,7 +89,7 @@ struct stormm_pool {
   std::vector<int> slot_range;          // range of each resident slot
   // Device state.
   DevMem xcrd, ycrd, zcrd, xfrc, yfrc, zfrc, xprv, yprv, zprv, xcg, ycg, zcg;
-  DevMem q, ljp1, ljp2, rho, scr, lj_type;
+  DevMem q, ljp1, ljp2, rho, scr, pbr, lj_type;
   // Per-atom sums of evaluations in parts (the integrals zero at rest unless part_dirty).
   DevMem part_psi, part_dedr, part_drdpsi, parts;
   bool part_dirty = false;
@@ -189,7 +188,7 @@ extern "C" int stormm_pool_create(const stormm_pool_config *cfg, stormm_pool **o
     HIP_TRY(d->alloc(na * sizeof(long long)));
     HIP_TRY(hipMemset(d->ptr, 0, na * sizeof(long long)));
   }
-  for (DevMem *d : {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr}) {
+  for (DevMem *d : {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr, &p->pbr}) {
     HIP_TRY(d->alloc(na * sizeof(double)));
   }
   for (DevMem *d : {&p->part_psi, &p->part_dedr, &p->part_drdpsi}) {
@@ -406,17 +405,17 @@ static hipError_t upload_entries(stormm_pool *p, int start, int total,
   long long *crd[3] = {p->xcrd.as<long long>(), p->ycrd.as<long long>(), p->zcrd.as<long long>()};
   DevMem *zero[9] = {&p->xfrc, &p->yfrc, &p->zfrc, &p->xprv, &p->yprv, &p->zprv, &p->xcg, &p->ycg,
                      &p->zcg};
-  DevMem *par[5] = {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr};
-  const void *src[8] = {cx.data(), cy.data(), cz.data(), ap.q.data(), ap.ljp1.data(),
-                        ap.ljp2.data(), ap.rho.data(), ap.scr.data()};
+  DevMem *par[kAdmitRows - 3] = {&p->q, &p->ljp1, &p->ljp2, &p->rho, &p->scr, &p->pbr};
+  const void *src[kAdmitRows] = {cx.data(), cy.data(), cz.data(), ap.q.data(), ap.ljp1.data(),
+                                 ap.ljp2.data(), ap.rho.data(), ap.scr.data(), ap.pbr.data()};
   for (int first = 0; first < total; first += kAdmitChunk) {
     const int count = std::min(total - first, kAdmitChunk);
     const size_t row = static_cast<size_t>(count) * sizeof(long long);
-    for (int v = 0; v < 8; v++) {
+    for (int v = 0; v < kAdmitRows; v++) {
       std::memcpy(stage.data() + v * row,
                   static_cast<const char *>(src[v]) + static_cast<size_t>(first) * 8, row);
     }
-    size_t at = 8 * row;
+    size_t at = kAdmitRows * row;
     std::memcpy(stage.data() + at, ap.lj_type.data() + first, count * sizeof(int));
     at += count * sizeof(int);
     const bool last = (first + count == total);
@@ -434,9 +433,9 @@ static hipError_t upload_entries(stormm_pool *p, int start, int total,
     }
     k.count = count;
     k.words = reinterpret_cast<const long long *>(dev);
-    k.types = reinterpret_cast<const int *>(dev + 8 * row);
+    k.types = reinterpret_cast<const int *>(dev + kAdmitRows * row);
     const size_t to = static_cast<size_t>(start) + first;
-    for (int v = 0; v < 8; v++) {
+    for (int v = 0; v < kAdmitRows; v++) {
       k.word_out[v] = ((v < 3) ? crd[v] : par[v - 3]->as<long long>()) + to;
     }
     for (int v = 0; v < 9; v++) {
@@ -687,6 +686,7 @@ static MMKit pool_mm_kit(stormm_pool *p, int nwu, int maxa, int block, const WuD
   k.ljab14 = p->ljab14.as<double2>();
   k.rho = p->rho.as<double>();
   k.scr = p->scr.as<double>();
+  k.pbr = p->pbr.as<double>();
   k.gb_alpha = p->sm.alpha;
   k.gb_beta = p->sm.beta;
   k.gb_gamma = p->sm.gamma;

@@ -44,7 +44,7 @@ extern "C" const char *stormm_last_error(void) { return g_last_error.c_str(); }
 // ------------------------------------------------------------------------------------------
 struct stormm_synthesis {
   SynthesisPlan plan;
-  DevMem atom_starts, atom_counts, q, ljp1, ljp2, lj_type, ljab, ljab14, rho, scr,
+  DevMem atom_starts, atom_counts, q, ljp1, ljp2, lj_type, ljab, ljab14, rho, scr, pbr,
       wu, wu_sys, wu_double, wu_sys_double, tasks, masks, vterms, bond_par, angl_par, dihe_par,
       dihe14, status, cycles_run, rms_force, stop_flags, rst, parts;
   MMKit kit;
@@ -152,6 +152,7 @@ extern "C" int stormm_synthesis_create(const stormm_topology_batch *batch,
   HIP_TRY(ag->ljab14.upload(P.ts.ljab14));
   HIP_TRY(ag->rho.upload(P.ap.rho));
   HIP_TRY(ag->scr.upload(P.ap.scr));
+  HIP_TRY(ag->pbr.upload(P.ap.pbr));
   HIP_TRY(ag->wu.upload(P.wu));
   HIP_TRY(ag->wu_sys.upload(P.wu_sys));
   HIP_TRY(ag->wu_double.upload(P.wu_double));
@@ -201,6 +202,7 @@ extern "C" int stormm_synthesis_create(const stormm_topology_batch *batch,
   k.ljab14 = ag->ljab14.as<double2>();
   k.rho = ag->rho.as<double>();
   k.scr = ag->scr.as<double>();
+  k.pbr = ag->pbr.as<double>();
   k.gb_alpha = P.sm.alpha;
   k.gb_beta = P.sm.beta;
   k.gb_gamma = P.sm.gamma;

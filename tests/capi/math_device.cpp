@@ -21,6 +21,9 @@ struct Exp {
 struct Log {
   static __device__ double eval(double x, double) { return D::log(x); }
 };
+struct Tanh {
+  static __device__ double eval(double x, double) { return D::tanh(x); }
+};
 struct Rsqrt {
   static __device__ double eval(double x, double) { return D::rsqrt(x); }
 };
@@ -108,6 +111,49 @@ template <typename F> static bool keeps_nan(const char *name) {
   return ok;
 }
 
+// Born radii against the same formulas in the IEEE operations, bit for bit.  x: the share of
+// 1 / rho that the integral takes away; y: the intrinsic radius; out: 0 for equal.
+template <int MODEL> struct Radii {
+  static __device__ double eval(double x, double pbr) {
+    const int igb = (MODEL == 0) ? 1 : 5;
+    // Variables, so that the products below are contracted as the ones of born_radius.
+    double al = (MODEL == 1) ? 0.8 : 1.0, be = (MODEL == 1) ? 0.0 : 0.8,
+           ga = (MODEL == 1) ? 2.909125 : 4.85;
+    const double rho = pbr - 0.09, psi = -x / rho;
+    const BornRadius got = born_radius(igb, al, be, ga, rho, pbr, psi);
+    double R, dr_dpsi = 0.0;
+    if (igb == 1) {
+      R = 1.0 / ((1.0 / rho) + psi);
+      R = (R < 0.0) ? 30.0 : R;
+    }
+    else {
+      const double fipsi = psi * (-rho);
+      const double thi = D::tanh((al - (be * fipsi) + (ga * fipsi * fipsi)) * fipsi);
+      R = 1.0 / ((1.0 / rho) - thi / pbr);
+      dr_dpsi = (al - ((2.0 * be) - (3.0 * ga * fipsi)) * fipsi) * (1.0 - thi * thi) * rho / pbr;
+    }
+    return (got.R == R && got.inv_R == 1.0 / R && got.dr_dpsi == dr_dpsi) ? 0.0 : 1.0;
+  }
+};
+static bool check_radii(int model) {
+  std::mt19937_64 rng(8000 + model);
+  std::uniform_real_distribution<double> u(0.0, 1.0);
+  std::vector<double> x(1 << 18), pbr(1 << 18), out;
+  for (size_t i = 0; i < x.size(); i++) {
+    x[i] = (i == 0) ? 0.0 : 1.5 * u(rng);
+    pbr[i] = 1.0 + (2.0 * u(rng));
+  }
+  const bool ran = (model == 0) ? evaluate<Radii<0>>(x, pbr, out) :
+                   (model == 1) ? evaluate<Radii<1>>(x, pbr, out) :
+                                  evaluate<Radii<2>>(x, pbr, out);
+  size_t differ = 0;
+  for (double o : out) {
+    differ += (o != 0.0) ? 1 : 0;
+  }
+  std::printf("born_radius, model %d: %zu of %zu differ\n", model, differ, x.size());
+  return ran && differ == 0;
+}
+
 static bool check_named(const char *name) {
   const std::string f(name);
   if (f == "exp") {
@@ -127,6 +173,21 @@ static bool check_named(const char *name) {
     // Half a unit from the last sum; the residual is exact and e^3 a thousandth of a unit.
     return check<Rsqrt>(name, 0.51, {{0.25, 1.0}, {1.0, 4.0}, {1.0, 1.0e5}, {1.0e-6, 1.0}},
                         [](long double x, long double) { return 1.0L / std::sqrt(x); });
+  }
+  if (f == "tanh") {
+    // The device library's error over the same arguments.
+    return check<Tanh>(name, 0.859, {{1.0e-8, 1.0e-4}, {1.0e-4, 0.01}, {0.01, 0.5}, {0.5, 3.0},
+                                     {3.0, 40.0}, {-1.0, 0.0}},
+                       [](long double x, long double) { return std::tanh(x); }) &&
+           keeps_nan<Tanh>(name);
+  }
+  if (f == "born_radius") {
+    // Integrals from none to a buried atom's, radii of 1 to 3 A, the three models' constants.
+    bool ok = true;
+    for (int model = 0; model < 3; model++) {
+      ok = check_radii(model) && ok;
+    }
+    return ok;
   }
   std::printf("no function %s\n", name);
   return false;
