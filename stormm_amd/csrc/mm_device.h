@@ -158,6 +158,10 @@ template <> struct Prec<double> {
     const double q = a * inv_b;
     return fma(fma(-q, b, a), inv_b, q);
   }
+  static __device__ __forceinline__ double root(double x, double y) {
+    const double s = x * y;
+    return fma(fma(-s, s, x), 0.5 * y, s);
+  }
   static __device__ __forceinline__ long long fixed(double x) { return round_to_ll(x); }
 };
 

@@ -1321,12 +1321,13 @@ template <bool FORCES, typename V>
 __device__ __forceinline__ double eval_bond(const V &v, int i, int j, double kb,
                                             double r0, double fscale) {
   const Vec3 d = v.disp(i, j);
+  using D = Prec<double>;
   const double d2 = dot(d, d);
-  const double inv = Prec<double>::rsqrt(d2);
-  const double dr = (d2 > 0.0) ? d2 * inv : 0.0;
+  const double inv = D::rsqrt(d2);
+  const double dr = (d2 > 0.0) ? D::root(d2, inv) : 0.0;
   const double dl = dr - r0;
   if (FORCES) {
-    const double fmag = 2.0 * kb * dl * inv;
+    const double fmag = D::quotient(2.0 * kb * dl, dr, inv);
     const long long ix = fix64(fmag * d.x * fscale);
     const long long iy = fix64(fmag * d.y * fscale);
     const long long iz = fix64(fmag * d.z * fscale);
@@ -1342,18 +1343,22 @@ __device__ __forceinline__ double eval_angle(const V &v, int i, int j, int kk,
                                              double ka, double th0, double fscale) {
   const Vec3 ba = v.disp(j, i);
   const Vec3 bc = v.disp(j, kk);
-  const double invba = Prec<double>::rsqrt(dot(ba, ba));
-  const double invbc = Prec<double>::rsqrt(dot(bc, bc));
-  const double invbabc = invba * invbc;
+  using D = Prec<double>;
+  const double mgba = dot(ba, ba);
+  const double mgbc = dot(bc, bc);
+  const double mg2 = mgba * mgbc;
+  const double invmg = D::rsqrt(mg2);
+  const double invbabc = D::quotient(1.0, D::root(mg2, invmg), invmg);
   double costheta = dot(ba, bc) * invbabc;
   costheta = (costheta < -1.0) ? -1.0 : ((costheta > 1.0) ? 1.0 : costheta);
   const double theta = acos(costheta);
   const double dtheta = theta - th0;
   if (FORCES) {
-    const double dA = -2.0 * ka * dtheta *
-                      Prec<double>::rsqrt(1.0 - (costheta * costheta));
-    const double sqba = dA * invba * invba;
-    const double sqbc = dA * invbc * invbc;
+    const double sin2 = 1.0 - (costheta * costheta);
+    const double invsin = D::rsqrt(sin2);
+    const double dA = D::quotient(-2.0 * ka * dtheta, D::root(sin2, invsin), invsin);
+    const double sqba = D::quotient(dA, mgba, D::rcp(mgba));
+    const double sqbc = D::quotient(dA, mgbc, D::rcp(mgbc));
     const double mbabc = dA * invbabc;
     const long long iax = fix64(((bc.x * mbabc) - (costheta * ba.x * sqba)) * fscale);
     const long long iay = fix64(((bc.y * mbabc) - (costheta * ba.y * sqba)) * fscale);

@@ -1,6 +1,7 @@
 // Errors of the double-precision functions of the evaluation kernels (stormm_amd/csrc/mm_device.h)
 // on the device, in units of the last place against 80-bit arithmetic on the host, over the
-// arguments that the kernels give them.  Arguments: the names of the functions to check.
+// arguments that the kernels give them; Born radii, bonds and angles against the same formulas in
+// the IEEE operations.  Arguments: the names of the functions to check.
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -10,7 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
-#include "../../stormm_amd/csrc/mm_device.h"
+#include "../../stormm_amd/csrc/mm_eval.h"
 
 using namespace stormm_amd;
 using D = Prec<double>;
@@ -135,6 +136,85 @@ template <int MODEL> struct Radii {
     return (got.R == R && got.inv_R == 1.0 / R && got.dr_dpsi == dr_dpsi) ? 0.0 : 1.0;
   }
 };
+
+// Atoms of a valence term and the forces it adds, for the terms of the evaluation kernels.
+struct Atoms {
+  Vec3 p[3];
+  long long *f;
+  __device__ Vec3 disp(int from, int to) const {
+    return {p[to].x - p[from].x, p[to].y - p[from].y, p[to].z - p[from].z};
+  }
+  __device__ void add(int a, long long x, long long y, long long z) const {
+    f[3 * a] += x;
+    f[3 * a + 1] += y;
+    f[3 * a + 2] += z;
+  }
+};
+constexpr double kForceScale = 1099511627776.0;  // 2^40
+
+// A bond of 0.1 to 3 A along x and y, and an angle between bonds of 1 to 2 A that is y, against
+// the same terms in the IEEE operations, bit for bit.
+struct Bond {
+  static __device__ double eval(double x, double y) {
+    long long got[6] = {0, 0, 0, 0, 0, 0};
+    const Atoms v = {{{0.0, 0.0, 0.0}, {x, 0.3 * y, 0.1}, {}}, got};
+    const double kb = 310.0, r0 = 1.09;
+    const double e = eval_bond<true>(v, 0, 1, kb, r0, kForceScale);
+    const Vec3 d = v.disp(0, 1);
+    const double dr = sqrt(dot(d, d));
+    const double dl = dr - r0;
+    const double fmag = 2.0 * kb * dl / dr;
+    return (e == kb * dl * dl && got[0] == fix64(fmag * d.x * kForceScale) &&
+            got[1] == fix64(fmag * d.y * kForceScale) &&
+            got[2] == fix64(fmag * d.z * kForceScale)) ? 0.0 : 1.0;
+  }
+};
+struct Angle {
+  static __device__ double eval(double x, double y) {
+    long long got[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const double l = 1.0 + (0.5 * fabs(x));
+    const Atoms v = {{{1.2, 0.0, 0.1 * x}, {0.0, 0.0, 0.0}, {l * cos(y), l * sin(y), 0.0}}, got};
+    const double ka = 63.0, th0 = 1.91;
+    const double e = eval_angle<true>(v, 0, 1, 2, ka, th0, kForceScale);
+    const Vec3 ba = v.disp(1, 0);
+    const Vec3 bc = v.disp(1, 2);
+    const double mgba = dot(ba, ba);
+    const double mgbc = dot(bc, bc);
+    const double invbabc = 1.0 / sqrt(mgba * mgbc);
+    double costheta = dot(ba, bc) * invbabc;
+    costheta = (costheta < -1.0) ? -1.0 : ((costheta > 1.0) ? 1.0 : costheta);
+    const double dtheta = acos(costheta) - th0;
+    const double dA = -2.0 * ka * dtheta / sqrt(1.0 - (costheta * costheta));
+    const double sqba = dA / mgba;
+    const double sqbc = dA / mgbc;
+    const double mbabc = dA * invbabc;
+    return (e == ka * dtheta * dtheta &&
+            got[0] == -fix64(((bc.x * mbabc) - (costheta * ba.x * sqba)) * kForceScale) &&
+            got[1] == -fix64(((bc.y * mbabc) - (costheta * ba.y * sqba)) * kForceScale) &&
+            got[2] == -fix64(((bc.z * mbabc) - (costheta * ba.z * sqba)) * kForceScale) &&
+            got[6] == -fix64(((ba.x * mbabc) - (costheta * bc.x * sqbc)) * kForceScale) &&
+            got[7] == -fix64(((ba.y * mbabc) - (costheta * bc.y * sqbc)) * kForceScale) &&
+            got[8] == -fix64(((ba.z * mbabc) - (costheta * bc.z * sqbc)) * kForceScale)) ? 0.0
+                                                                                         : 1.0;
+  }
+};
+template <typename F> static bool check_term(const char *name) {
+  std::mt19937_64 rng(9000);
+  std::uniform_real_distribution<double> u(0.0, 1.0);
+  std::vector<double> x(1 << 18), y(1 << 18), out;
+  for (size_t i = 0; i < x.size(); i++) {
+    x[i] = 4.0 * (u(rng) - 0.5);
+    y[i] = 0.05 + (3.05 * u(rng));
+  }
+  const bool ran = evaluate<F>(x, y, out);
+  size_t differ = 0;
+  for (double o : out) {
+    differ += (o != 0.0) ? 1 : 0;
+  }
+  std::printf("%s: %zu of %zu differ\n", name, differ, x.size());
+  return ran && differ == 0;
+}
+
 static bool check_radii(int model) {
   std::mt19937_64 rng(8000 + model);
   std::uniform_real_distribution<double> u(0.0, 1.0);
@@ -188,6 +268,12 @@ static bool check_named(const char *name) {
       ok = check_radii(model) && ok;
     }
     return ok;
+  }
+  if (f == "bond") {
+    return check_term<Bond>(name);
+  }
+  if (f == "angle") {
+    return check_term<Angle>(name);
   }
   std::printf("no function %s\n", name);
   return false;

@@ -11,7 +11,8 @@ from stormm_amd import build
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("function", ["exp", "log", "rsqrt", "tanh", "born_radius"])
+@pytest.mark.parametrize("function", ["exp", "log", "rsqrt", "tanh", "born_radius", "bond",
+                                      "angle"])
 def test_error(function):
     exe = os.path.join(build.CAPI_BIN, "math_device")
     if not os.path.exists(exe):
