@@ -394,11 +394,12 @@ int stormm_launch_line_advance(int32_t precision, const stormm_synthesis *ag,
 /* Whole minimization.  persistent == 0 issues the reference's per-step launch sequence (per
  * cycle: force evaluation, conjugate gradient, four line moves with three energy evaluations);
  * persistent == 2 captures that sequence for one cycle in a HIP graph and replays it for every
- * cycle.  persistent == 1, 3 and 4 run fused cycle kernels: each evaluation block also updates
- * the conjugate-gradient direction and makes the line move of the whole systems it holds, so a
- * cycle is four launches; mode 1 issues the damped and first cycles one by one and a longer run's
- * rest as replays of a HIP graph of eight cycles captured meanwhile, mode 3 captures one cycle and
- * replays it, mode 4 issues the kernels one by one.  All modes
+ * cycle.  persistent == 1, 3 and 4 run fused cycle kernels: each evaluation block also makes the
+ * line move of the whole systems it holds, so a cycle is five launches with the
+ * conjugate-gradient update (14 where few large systems are evaluated by several blocks each, whose
+ * line moves are launches of their own); mode 1 issues the damped and first cycles one by one and
+ * a longer run's rest as replays of a HIP graph of eight cycles captured meanwhile, mode 3
+ * captures one cycle and replays it, mode 4 issues the kernels one by one.  All modes
  * give bit-identical results.  Modes 1-4 stop a system once its RMS force reaches
  * convergence_rms_force (if > 0) and record per-system cycle counts and RMS forces
  * (stormm_minimization_status).  Final energies land in the ScoreCard.  Modes 1, 3 and 4 take

@@ -198,6 +198,7 @@ struct MMKit {
   const WuPart *parts;
   long long *part_psi, *part_dedr;
   double *part_drdpsi;
+  const int *done;           // per system, nonzero once stopped (parts only; null: none stops)
   // Restraints (src/Potential/valence_potential.tpp:2090-2160) and the step number their
   // parameters are mixed at: rst_step, or, when rst_step_sys holds each system's cycle count,
   // minimizer_step(rst_step_sys[system] + rst_cycle_offset, rst_move, rst_clash_cycles).

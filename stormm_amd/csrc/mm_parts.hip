@@ -22,6 +22,19 @@ __device__ __forceinline__ void global_add(long long *addr, long long v) {
   }
 }
 
+// True in every thread when all systems of the unit have stopped (k.done).  Its coordinates no
+// longer change, so its forces and ScoreCard rows already hold what the evaluation would write
+// and its integrals are zero: the block returns, as k_min_cycle's does.
+__device__ __forceinline__ bool unit_stopped(const MMKit &k, int unit) {
+  if (k.done == nullptr) {
+    return false;
+  }
+  const WuDesc &wu = k.wu[unit];
+  const int tid = static_cast<int>(threadIdx.x);
+  const bool runs = tid < wu.sys_count && k.done[k.wu_sys[wu.sys_first + tid].sys_index] == 0;
+  return __syncthreads_or(runs ? 1 : 0) == 0;
+}
+
 // This part's force and energy sums added to the global arrays.
 template <typename T, bool FORCES>
 __device__ __forceinline__ void part_store(StageCtx<T> &c, const MMKit &k, bool eval_energy) {
@@ -55,6 +68,9 @@ __global__ void __launch_bounds__((EvalBlockLimit<T, false>::value))
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
   const WuPart wp = k.parts[blockIdx.x];
+  if (unit_stopped(k, wp.unit)) {
+    return;
+  }
   init_ctx<T>(c, k, wp.unit, terms);
   c.part = wp.part;
   c.parts = wp.parts;
@@ -101,6 +117,9 @@ __global__ void __launch_bounds__((EvalBlockLimit<T, FORCES && CLASH>::value))
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
   const WuPart wp = k.parts[blockIdx.x];
+  if (unit_stopped(k, wp.unit)) {
+    return;
+  }
   init_ctx<T>(c, k, wp.unit, terms);
   c.part = wp.part;
   c.parts = wp.parts;
@@ -148,6 +167,9 @@ __global__ void __launch_bounds__((EvalBlockLimit<T, false>::value))
   extern __shared__ __align__(16) unsigned char smem[];
   StageCtx<T> c(smem, k.maxa, static_cast<int>(blockDim.x >> 6));
   const WuPart wp = k.parts[blockIdx.x];
+  if (unit_stopped(k, wp.unit)) {
+    return;
+  }
   init_ctx<T>(c, k, wp.unit, terms);
   c.part = wp.part;
   c.parts = wp.parts;

@@ -1933,6 +1933,7 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
   const bool in_parts = use_parts(k, ag, ps);
   if (in_parts) {
     ck.line.clear = k.part_psi;
+    k.done = cs.done;
   }
   const int sd = mc->steepest_descent_cycles;
   const int cdcyc = std::min(mc->clash_damping_cycles, mc->total_cycles);
