@@ -81,6 +81,8 @@ hipError_t launch_conjugate_gradient(const CgKit &k, int step, int sd_cycles,
 hipError_t launch_history_fill(const HistKit &h, const int *steps, int nsys, int count,
                                hipStream_t stream);
 hipError_t launch_line_advance(const LineKit &k, int move_number, hipStream_t stream);
+// Sets k.clear to zero for the kit's systems, stopped or not, as their line moves do.
+hipError_t launch_clear_systems(const LineKit &k, hipStream_t stream);
 
 // Fused minimization cycle (mm_minimize.hip): evaluations that make the pending line move of
 // the systems they hold while loading the coordinates.  cg.done is required; line holds the

@@ -421,6 +421,13 @@ __device__ __forceinline__ void line_apply(const LineKit &k, int start, int n, d
   }
 }
 
+// k.clear of one system's atoms, by one wavefront.
+__device__ __forceinline__ void clear_system(const LineKit &k, int s, int lane) {
+  for (int i = lane; i < k.sys_natom[s]; i += 64) {
+    k.clear[k.sys_start[s] + i] = 0;
+  }
+}
+
 // One line move per system, src/MolecularMechanics/line_movement.cui:4-415, one wavefront per
 // system and four systems per block.  Stopped systems (serving) keep their coordinates and line
 // state.
@@ -434,9 +441,7 @@ __global__ void __launch_bounds__(64 * kLineWaves) k_line_advance(LineKit k, int
   }
   const int s = (k.slots != nullptr) ? k.slots[e] : e;
   if (k.clear != nullptr) {
-    for (int i = lane; i < k.sys_natom[s]; i += 64) {
-      k.clear[k.sys_start[s] + i] = 0;
-    }
+    clear_system(k, s, lane);
   }
   if (k.done != nullptr && k.done[s] != 0) {
     return;
@@ -464,6 +469,22 @@ hipError_t launch_line_advance(const LineKit &k, int move_number, hipStream_t st
   }
   hipLaunchKernelGGL(k_line_advance, dim3((k.nsys + kLineWaves - 1) / kLineWaves),
                      dim3(64 * kLineWaves), 0, stream, k, move_number);
+  return hipGetLastError();
+}
+
+__global__ void __launch_bounds__(64 * kLineWaves) k_clear_systems(LineKit k) {
+  const int e = (blockIdx.x * kLineWaves) + static_cast<int>(threadIdx.x >> 6);
+  if (e < k.nsys) {
+    clear_system(k, (k.slots != nullptr) ? k.slots[e] : e, threadIdx.x & 63);
+  }
+}
+
+hipError_t launch_clear_systems(const LineKit &k, hipStream_t stream) {
+  if (k.nsys == 0 || k.clear == nullptr) {
+    return hipSuccess;
+  }
+  hipLaunchKernelGGL(k_clear_systems, dim3((k.nsys + kLineWaves - 1) / kLineWaves),
+                     dim3(64 * kLineWaves), 0, stream, k);
   return hipGetLastError();
 }
 

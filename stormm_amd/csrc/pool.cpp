@@ -924,13 +924,10 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
     return (k.nparts > 0) ? launch_mm_parts(prec, k, terms, force, 1, st)
                           : launch_mm_eval(prec, k, terms, force, 1, st);
   };
-  auto clear_sums = [&]() {
-    return launch_fill(p->part_psi.as<long long>(), nullptr, nullptr,
-                       static_cast<size_t>(p->cap_atoms), st);
-  };
   if (mm.nparts > 0) {
     if (p->part_dirty) {
-      HIP_TRY(clear_sums());
+      HIP_TRY(launch_fill(p->part_psi.as<long long>(), nullptr, nullptr,
+                          static_cast<size_t>(p->cap_atoms), st));
     }
     p->part_dirty = true;
   }
@@ -948,7 +945,9 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
   // Energies at the coordinates the call leaves.
   HIP_TRY(evaluate(mm, 0));
   if (mm.nparts > 0) {
-    HIP_TRY(clear_sums());
+    // Only this call's systems can have left integrals: the whole array would cost with the
+    // pool's budget, not its work (48 GB: 0.4 ms a call).
+    HIP_TRY(launch_clear_systems(lk, st));
     p->part_dirty = false;
   }
   if (staging.base != nullptr) {
