@@ -139,7 +139,9 @@ typedef struct {
 /* Work-unit shaping, chosen by the autotuner (or fixed by the caller).  Zero = default. */
 typedef struct {
   int32_t wu_atom_capacity;        /* atoms staged in LDS per work unit (<= 512)                */
-  int32_t target_wu_per_cu;        /* work units per compute unit to aim for when packing       */
+  int32_t target_wu_per_cu;        /* work units per compute unit to aim for when packing, each
+                                      evaluated by one block (default: 2, or several blocks to a
+                                      unit where few large systems leave compute units idle)    */
   int32_t block_threads;           /* threads per work-unit block: 256, 512 or 1024 (default: by
                                       precision and number of units)                            */
 } stormm_launch_shape;
@@ -251,6 +253,9 @@ int stormm_synthesis_atom_layout(const stormm_synthesis *ag, int32_t *atom_start
 /* Build the host-side plan (layout, work units, tile tasks) without touching the device. */
 int stormm_synthesis_plan(const stormm_topology_batch *batch, const stormm_launch_shape *shape,
                           stormm_synthesis_info *info);
+/* Blocks of an evaluation whose work units are shared by several blocks each (0: one block to a
+ * unit).  Few large systems are evaluated so where the caller names no units per compute unit. */
+int stormm_synthesis_part_count(const stormm_synthesis *ag, int32_t *blocks);
 /* Kernel status bits (1 = coordinates beyond the LDS coordinate range); clear != 0 resets. */
 int stormm_synthesis_status(const stormm_synthesis *ag, int32_t *status, int32_t clear);
 /* Autotuner: time force + energy evaluations of the batch under candidate launch shapes (work-unit

@@ -127,6 +127,7 @@ _SIGS = {
     "stormm_synthesis_destroy": (c_int32, [vp]),
     "stormm_synthesis_get_info": (c_int32, [vp, P(SynthesisInfo)]),
     "stormm_synthesis_atom_layout": (c_int32, [vp, vp, vp]),
+    "stormm_synthesis_part_count": (c_int32, [vp, P(c_int32)]),
     "stormm_synthesis_plan": (c_int32, [P(TopologyBatch), P(LaunchShape), P(SynthesisInfo)]),
     "stormm_synthesis_status": (c_int32, [vp, P(c_int32), c_int32]),
     "stormm_autotune_launch_shape": (c_int32, [P(TopologyBatch), c_int32, vp, P(LaunchShape),

@@ -18,6 +18,9 @@ constexpr double kMinPartCost = 300.0;
 constexpr double kPartsFactor = 2.4;
 constexpr double kPartsOverhead = 1800.0;
 
+// Units to aim for at each compute unit where the caller names no number.
+constexpr int kDefaultPerGroup = 2;
+
 // Units a compute unit tried beyond the fewest that could hold a batch, and the share of their
 // atoms that may be taken.
 constexpr int kMoreUnits = 2;
@@ -637,9 +640,10 @@ void pack_systems(const std::vector<double> &cost, const std::vector<int> &natom
                   bool grouped, std::vector<std::vector<int>> &bins_out,
                   std::vector<int> &mode_out, std::vector<WuPart> &parts) {
   groups = std::max(1, groups);
-  per_group = std::max(1, per_group);
+  const bool chosen = (per_group > 0);
+  per_group = chosen ? per_group : kDefaultPerGroup;
   parts.clear();
-  if (!pack_parts(cost, natom, table_mode, cap, groups, bins_out, mode_out, parts)) {
+  if (chosen || !pack_parts(cost, natom, table_mode, cap, groups, bins_out, mode_out, parts)) {
     pack_units(cost, natom, table_mode, cap, groups, per_group, grouped, bins_out, mode_out);
   }
 }
@@ -1023,7 +1027,7 @@ int build_plan(const stormm_topology_batch *b, const stormm_launch_shape *shape_
     return fail(STORMM_ERR_INVALID_ARGUMENT, "work-unit capacity must be a multiple of 16 in "
                                              "[16, 512]");
   }
-  const int wu_per_cu = (shape.target_wu_per_cu > 0) ? shape.target_wu_per_cu : 2;
+  const int wu_per_cu = std::max(shape.target_wu_per_cu, 0);
   P.block = std::max(shape.block_threads, 0);
   if (P.block != 0 && P.block != 256 && P.block != 512 && P.block != 1024) {
     return fail(STORMM_ERR_INVALID_ARGUMENT, "block_threads must be 256, 512 or 1024");
@@ -1117,8 +1121,8 @@ int build_plan(const stormm_topology_batch *b, const stormm_launch_shape *shape_
   if (rc == STORMM_OK && shape.wu_atom_capacity <= 0 && P.block == 0 && P.parts.empty() &&
       P.maxa > kTwoBlockAtomsDouble && largest <= kTwoBlockAtomsDouble &&
       static_cast<int>(P.wu.size()) > cus) {
-    pack_units(cost, P.atom_counts, P.lj_table_mode, kTwoBlockAtomsDouble, cus, wu_per_cu, true,
-               bins, bin_mode);
+    pack_units(cost, P.atom_counts, P.lj_table_mode, kTwoBlockAtomsDouble, cus,
+               (wu_per_cu > 0) ? wu_per_cu : kDefaultPerGroup, true, bins, bin_mode);
     rc = append(P.wu_double, P.wu_sys_double, P.maxa_double);
   }
   return rc;

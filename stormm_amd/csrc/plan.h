@@ -140,7 +140,9 @@ int fill_atom_parameters(const stormm_topology_batch *b, const SystemTerms &t, i
                          AtomParams &ap, int s);
 
 // Longest-processing-time assignment of systems onto about `groups` x `per_group` work units, or
-// a larger multiple of `groups` where these cannot hold them.
+// a larger multiple of `groups` where these cannot hold them.  per_group 0 (the caller names no
+// number): two, or, where a few large systems would leave compute units idle, units evaluated by
+// several blocks each (`parts`).
 // With `grouped`, and when every unit fits on the device at once, the systems are balanced over
 // `groups` groups (one per compute unit) emitted so that units g, g + G, g + 2G, ... form group
 // g; otherwise the units are balanced individually and emitted by decreasing cost.

@@ -760,7 +760,7 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
   // A unit holds kMaxWuAtoms at most, whatever capacity was asked for.
   const int cap = (sh.wu_atom_capacity > 0) ? std::min<int>(sh.wu_atom_capacity, kMaxWuAtoms)
                                             : kMaxWuAtoms;
-  const int per_cu = (sh.target_wu_per_cu > 0) ? sh.target_wu_per_cu : 2;
+  const int per_cu = std::max(sh.target_wu_per_cu, 0);
   const int block = std::max(sh.block_threads, 0);
   std::vector<std::vector<int>> bins;
   std::vector<int> modes;

@@ -2223,6 +2223,14 @@ extern "C" int stormm_minimization_status(const stormm_synthesis *ag, int32_t *c
   return STORMM_OK;
 }
 
+extern "C" int stormm_synthesis_part_count(const stormm_synthesis *ag, int32_t *blocks) {
+  if (ag == nullptr || blocks == nullptr) {
+    return fail(STORMM_ERR_INVALID_ARGUMENT, "null argument");
+  }
+  *blocks = static_cast<int32_t>(ag->plan.parts.size());
+  return STORMM_OK;
+}
+
 extern "C" int stormm_synthesis_status(const stormm_synthesis *ag, int32_t *status,
                                        int32_t clear) {
   if (ag == nullptr || status == nullptr) {
@@ -2297,7 +2305,8 @@ extern "C" int stormm_autotune_launch_shape(const stormm_topology_batch *batch,
   // In double precision two units of 384 atoms do not share a compute unit, two of 336 do.
   const int caps[4] = {128, 256, (precision == STORMM_PREC_DOUBLE) ? kTwoBlockAtomsDouble : 384,
                        512};
-  const int per_cu[4] = {1, 2, 3, 4};
+  // 0, the default, where it stands for units evaluated by several blocks each.
+  const int per_cu[5] = {0, 1, 2, 3, 4};
   const int blocks[3] = {256, 512, 1024};
   double best_t = 1.0e30;
   stormm_launch_shape best_shape = {512, 2, kEvalBlock};
@@ -2324,6 +2333,10 @@ extern "C" int stormm_autotune_launch_shape(const stormm_topology_batch *batch,
       int rc = stormm_synthesis_create(batch, &shape, &ag);
       if (rc != STORMM_OK) {
         return rc;
+      }
+      if (pc == 0 && ag->plan.parts.empty()) {
+        stormm_synthesis_destroy(ag);
+        break;
       }
       stormm_phasespace *ps = nullptr;
       stormm_scorecard *sc = nullptr;

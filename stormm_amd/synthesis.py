@@ -224,6 +224,13 @@ class AtomGraphSynthesis:
     def total_atoms(self) -> int:
         return int(self.atom_counts.sum())
 
+    @property
+    def part_count(self) -> int:
+        """Blocks of an evaluation in which several share a work unit (0: one to a unit)."""
+        n = ctypes.c_int32(0)
+        check(self._L.stormm_synthesis_part_count(self.handle, ctypes.byref(n)))
+        return n.value
+
     def status(self, clear: bool = True) -> int:
         st = ctypes.c_int32(0)
         check(self._L.stormm_synthesis_status(self.handle, ctypes.byref(st), int(clear)))
