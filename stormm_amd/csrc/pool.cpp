@@ -702,17 +702,8 @@ static MMKit pool_mm_kit(stormm_pool *p, int nwu, int maxa, int block, const WuD
   return k;
 }
 
-// Where one call's work units, their system entries and the list of running slots go: the
-// pool's own (growing) buffers, or a caller-provided region of fixed size.
-struct PoolStaging {
-  void *base = nullptr;   // null: the pool's buffers
-  size_t bytes = 0;
-};
-
-static size_t align256(size_t n) { return (n + 255) & ~static_cast<size_t>(255); }
-
-static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, void *stream,
-                         const PoolStaging &staging) {
+extern "C" int stormm_pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running,
+                                    void *stream) {
   if (pool == nullptr || cycles < 0) {
     return fail(STORMM_ERR_INVALID_ARGUMENT, "invalid minimization request");
   }
@@ -783,42 +774,19 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
   const size_t wu_bytes = wu.size() * sizeof(WuDesc);
   const size_t wu_sys_bytes = wu_sys.size() * sizeof(WuSys);
   const size_t act_bytes = act.size() * sizeof(int);
-  WuDesc *d_wu;
-  WuSys *d_wu_sys;
-  int *d_active;
-  WuPart *d_parts;
-  if (staging.base == nullptr) {
-    if (p->parts.bytes < part_bytes) {
-      HIP_TRY(p->parts.alloc(2 * part_bytes));
-    }
-    d_parts = p->parts.as<WuPart>();
-    if (p->wu.bytes < wu_bytes) {
-      HIP_TRY(p->wu.alloc(2 * wu_bytes));
-    }
-    if (p->wu_sys.bytes < wu_sys_bytes) {
-      HIP_TRY(p->wu_sys.alloc(2 * wu_sys_bytes));
-    }
-    d_wu = p->wu.as<WuDesc>();
-    d_wu_sys = p->wu_sys.as<WuSys>();
-    d_active = p->active.as<int>();
+  if (p->parts.bytes < part_bytes) {
+    HIP_TRY(p->parts.alloc(2 * part_bytes));
   }
-  else {
-    const size_t need = align256(wu_bytes) + align256(wu_sys_bytes) + align256(act_bytes) +
-                        align256(part_bytes);
-    if (need > staging.bytes) {
-      return fail(STORMM_ERR_CAPACITY,
-                  "the call's work units need " + std::to_string(need) + " bytes of staging (" +
-                      std::to_string(wu.size()) + " units, " + std::to_string(na) +
-                      " systems); the allocation-free entry point holds " +
-                      std::to_string(staging.bytes));
-    }
-    char *b = static_cast<char *>(staging.base);
-    d_wu = reinterpret_cast<WuDesc *>(b);
-    d_wu_sys = reinterpret_cast<WuSys *>(b + align256(wu_bytes));
-    d_active = reinterpret_cast<int *>(b + align256(wu_bytes) + align256(wu_sys_bytes));
-    d_parts = reinterpret_cast<WuPart *>(b + align256(wu_bytes) + align256(wu_sys_bytes) +
-                                         align256(act_bytes));
+  if (p->wu.bytes < wu_bytes) {
+    HIP_TRY(p->wu.alloc(2 * wu_bytes));
   }
+  if (p->wu_sys.bytes < wu_sys_bytes) {
+    HIP_TRY(p->wu_sys.alloc(2 * wu_sys_bytes));
+  }
+  WuPart *d_parts = p->parts.as<WuPart>();
+  WuDesc *d_wu = p->wu.as<WuDesc>();
+  WuSys *d_wu_sys = p->wu_sys.as<WuSys>();
+  int *d_active = p->active.as<int>();
   HIP_TRY(hipMemcpy(d_wu, wu.data(), wu_bytes, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_wu_sys, wu_sys.data(), wu_sys_bytes, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_active, act.data(), act_bytes, hipMemcpyHostToDevice));
@@ -950,17 +918,7 @@ static int pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running, vo
     HIP_TRY(launch_clear_systems(lk, st));
     p->part_dirty = false;
   }
-  if (staging.base != nullptr) {
-    // The staging region is shared by every call on the device: it must not be rewritten
-    // before this call's kernels have read it.
-    HIP_TRY(hipStreamSynchronize(st));
-  }
   return STORMM_OK;
-}
-
-extern "C" int stormm_pool_minimize(stormm_pool *pool, int32_t cycles, int32_t *running,
-                                    void *stream) {
-  return pool_minimize(pool, cycles, running, stream, PoolStaging());
 }
 
 extern "C" int stormm_pool_status(const stormm_pool *pool, const int32_t *slots, int32_t count,
