@@ -56,8 +56,7 @@ constexpr size_t kLdsPerCu = 160 * 1024;
 constexpr int kTwoBlockAtomsDouble = 336;
 // Entries of each wavefront's LDS queue of near-field Born-integral pairs.  A wave drains 64
 // entries at a time whenever the queue holds at least 64 after a group of four rotation steps,
-// each of which adds at most 64 (and stores its lanes without an entry just past the new
-// ones).
+// each of which adds at most 64.
 constexpr int kNearQueue = 320;
 constexpr int kNearQueueStride = kNearQueue;
 constexpr int kStageCounters = 3;  // work-item counters of the psi, derivative and valence stages

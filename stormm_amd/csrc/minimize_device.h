@@ -1,5 +1,5 @@
 // Line-search state machine of the minimizer, shared by the per-step line-advance kernel and
-// the persistent minimizer.  All arithmetic is double precision, as in the reference
+// the fused cycle kernels.  All arithmetic is double precision, as in the reference
 // (src/MolecularMechanics/hpc_minimization.cu:59-61).
 #pragma once
 

@@ -1,5 +1,5 @@
-// Device-side arithmetic shared by the fused evaluation kernel and the persistent minimizer:
-// precision traits, DPP row rotation, the Born-radius integral and its radial derivative, the
+// Device-side arithmetic shared by the evaluation and the fused minimization kernels: precision
+// traits, DPP row rotation, the Born-radius integral and its radial derivative, the
 // work-unit LDS layout and the valence term evaluators.
 #pragma once
 
@@ -18,8 +18,8 @@ constexpr double kGbKscale = 0.73;      // src/Constants/generalized_born.h:120
 
 // ------------------------------------------------------------------------------------------
 // Precision traits.  Single precision uses the hardware transcendental units (v_rsq, v_rcp,
-// v_log, v_exp); double precision refines the hardware estimates and has its own exponential and
-// logarithm for the arguments that occur.
+// v_log, v_exp); double precision refines the hardware estimates and has its own logarithm and
+// hyperbolic tangent for the arguments that occur.
 // ------------------------------------------------------------------------------------------
 // Nearest integer (ties to even, as rint) of a double as int64.  For |x| < 2^51, adding
 // 1.5 * 2^52 rounds x to an integer held in the low bits of the sum's bit pattern; subtracting
@@ -372,7 +372,7 @@ __device__ __forceinline__ long long fixed_contrib(double x, int bits) {
 }
 
 // Largest block a kernel is compiled for: 16 wavefronts leave 128 registers to a lane, and the
-// clash-damped force evaluations in double precision (HEAVY) need 150.
+// clash-damped force evaluations in double precision (HEAVY) need 152.
 template <typename T, bool HEAVY> struct EvalBlockLimit {
   static constexpr int value = kMaxEvalBlock;
 };

@@ -20,12 +20,12 @@ __device__ __forceinline__ double wave_sum64(double v) {
 // Polak-Ribiere direction and normalization, one 64-lane wave per system:
 // src/Math/hpc_reduction.cu:39-244 (gather / scatter cores) and
 // src/Math/conjugate_gradient.cui:259-370 (all-reduce kernel).  The per-lane accumulation order
-// and the butterfly reductions match the persistent minimizer, so both paths produce the same
-// directions bit for bit.
+// and the butterfly reductions are the same in every minimization mode, so that all of them
+// produce the same directions bit for bit.
 //
 // With per-system step counters (serving), each system advances its own counter and stops (its
 // `done` flag is set, the direction left untouched and no line move follows) once its RMS force
-// reaches `conv_rms` or its counter reaches `max_steps`: the persistent minimizer's stopping rule.
+// reaches `conv_rms` or its counter reaches `max_steps`.
 // Systems of up to kCgCached x 64 atoms keep their forces and directions in registers from the
 // first pass to the last, so the three passes cost one round trip to memory; larger systems read
 // them again in each pass.  Both forms accumulate in the same order.

@@ -1690,7 +1690,7 @@ static int minimize_stepwise(int32_t precision, const stormm_synthesis *ag,
 
 // The per-cycle launch sequence captured once in a HIP graph and replayed for every cycle.  The
 // conjugate-gradient kernel reads each system's cycle count from device memory (so one captured
-// cycle serves them all) and applies the RMS-force stop of the persistent minimizer; evaluations
+// cycle serves them all) and applies the RMS-force stop of the fused modes; evaluations
 // overwrite, so the graph holds kernels only.  With clash damping a second graph, whose
 // evaluations take each system's damping schedule from the same cycle counts, serves the first
 // clash_damping_cycles cycles.
