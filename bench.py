@@ -153,7 +153,7 @@ def minimization_workload(S, synthetic, oracle, nsys, cycles, with_cpu, shape=No
         timings[name] = run(whole, mode)
         energies[name] = whole[0][2].potential_energies()
         del whole
-    # The fused whole-run graph once per size class (atom-count quartiles of the range).
+    # The fused cycles (mode 1) once per size class (atom-count quartiles of the range).
     edges = [16, 44, 72, 100, 129]
     classes = [[i for i, t in enumerate(topos) if lo <= t.natom < hi]
                for lo, hi in zip(edges[:-1], edges[1:])]

@@ -477,12 +477,12 @@ static_assert(2 * WuLds<double>::bytes(kTwoBlockAtomsDouble, kEvalBlock / 64) <=
 
 // Threads of an evaluation block.  With no more units than compute units each block has its
 // compute unit to itself, and 16 wavefronts hide the latencies that 8 leave open (24 systems of
-// 487 atoms 196 -> 161 us); with more units two blocks of 8 share it, whose barriers do not
-// coincide (1024 systems 110 us against 125).  In double precision two such blocks need units of
-// at most 336 atoms to fit the LDS (600 systems of 20-200 atoms 77 us against 96); beyond that
-// one block takes the whole compute unit (1024 systems of 24-256 atoms 157 us against 178 at
+// 487 atoms 180 -> 144 us); with more units two blocks of 8 share it, whose barriers do not
+// coincide (1024 systems 87 us against 100).  In double precision two such blocks need units of
+// at most 336 atoms to fit the LDS (600 systems of 20-200 atoms 77 us against 101); beyond that
+// one block takes the whole compute unit (1024 systems of 24-256 atoms 158 us against 179 at
 // half the size), and a unit alone that is too small for 16 wavefronts takes 8 (200 systems of
-// 100 atoms 37 us against 40).  A HEAVY kernel's registers hold 12 wavefronts instead of 16.
+// 100 atoms 37 us against 41).  A HEAVY kernel's registers hold 12 wavefronts instead of 16.
 // A size that was asked for (the pool takes any) becomes whole wavefronts, no fewer than cover a
 // unit's atoms at stage_load's two to a thread.  Results do not depend on the size.
 template <typename T, bool HEAVY> inline int eval_block(const MMKit &k, int blocks) {

@@ -6,7 +6,8 @@
 // valence, radii and pairs; derivative forces) that pass those sums through per-atom arrays in
 // device memory.  All sums are fixed-precision integers, so results equal one block's bit for bit.
 // Measured against one block of 1024 threads per unit: an evaluation of 24 systems of 487 atoms
-// 161 -> 60 us (15, 27 and 17 us for the three launches), 20 served cycles of 160 systems of
+// 161 -> 60 us with its fills (15, 27 and 17 us for the three launches; in double precision and
+// without the fills 234 -> 58 us), 20 served cycles of 160 systems of
 // 16-416 atoms 21.1 -> 17.1 ms.  Below about 250 atoms the two extra launches and set-ups cost
 // more than the idle compute units (33 systems of 149 atoms: 61 us against 50).
 #include <algorithm>

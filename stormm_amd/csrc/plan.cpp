@@ -1113,7 +1113,7 @@ int build_plan(const stormm_topology_batch *b, const stormm_launch_shape *shape_
   // Larger units than two of which fit a compute unit's LDS in double precision: smaller ones
   // for that precision, if the systems allow and the caller did not choose the shape.  Two blocks
   // whose barriers do not coincide then share the compute unit (1024 systems of 24-256 atoms
-  // 171 us in units of up to 384 atoms, 154 in units of 336).
+  // 158 us in units of up to 352 atoms, 139 in units of 336).
   int largest = 0;
   for (int n : P.atom_counts) {
     largest = std::max(largest, round_up(n, kTile));
