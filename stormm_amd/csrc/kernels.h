@@ -84,6 +84,9 @@ hipError_t launch_line_advance(const LineKit &k, int move_number, hipStream_t st
 // Sets k.clear to zero for the kit's systems, stopped or not, as their line moves do.
 hipError_t launch_clear_systems(const LineKit &k, hipStream_t stream);
 
+// Writes to *running (memory the host reads) whether any of the systems has not stopped.
+hipError_t launch_any_running(const int *done, int nsys, int *running, hipStream_t stream);
+
 // Fused minimization cycle (mm_minimize.hip): evaluations that make the pending line move of
 // the systems they hold while loading the coordinates.  cg.done is required; line holds the
 // line-search state and scales.

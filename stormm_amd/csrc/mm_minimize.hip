@@ -472,6 +472,22 @@ hipError_t launch_line_advance(const LineKit &k, int move_number, hipStream_t st
   return hipGetLastError();
 }
 
+__global__ void __launch_bounds__(256) k_any_running(const int *done, int nsys, int *running) {
+  int any = 0;
+  for (int s = threadIdx.x; s < nsys; s += blockDim.x) {
+    any |= (done[s] == 0) ? 1 : 0;
+  }
+  any = __syncthreads_or(any);
+  if (threadIdx.x == 0) {
+    *running = any;
+  }
+}
+
+hipError_t launch_any_running(const int *done, int nsys, int *running, hipStream_t stream) {
+  hipLaunchKernelGGL(k_any_running, dim3(1), dim3(256), 0, stream, done, nsys, running);
+  return hipGetLastError();
+}
+
 __global__ void __launch_bounds__(64 * kLineWaves) k_clear_systems(LineKit k) {
   const int e = (blockIdx.x * kLineWaves) + static_cast<int>(threadIdx.x >> 6);
   if (e < k.nsys) {

@@ -65,6 +65,13 @@ struct stormm_phasespace {
   DevMem part_psi, part_dedr, part_drdpsi;
   // The integrals may not be zero: a launch sequence that should have cleared them failed.
   bool part_dirty = false;
+  // Pinned words in which minimizations in parts report whether systems still run (StopWatch).
+  int *running = nullptr;
+  ~stormm_phasespace() {
+    if (running != nullptr) {
+      (void)hipHostFree(running);
+    }
+  }
 };
 
 struct stormm_scorecard {
@@ -298,6 +305,10 @@ extern "C" int stormm_phasespace_create(const stormm_synthesis *ag, int32_t gpos
   for (DevMem *d : ovrf) {
     HIP_TRY(d->alloc(na * sizeof(int)));
     HIP_TRY(hipMemset(d->ptr, 0, na * sizeof(int)));
+  }
+  if (!ag->plan.parts.empty()) {
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&ps->running), 2 * sizeof(int),
+                          hipHostMallocDefault));
   }
   if (!ag->plan.parts.empty() && ag->plan.sm.igb != 0) {
     for (DevMem *d : {&ps->part_psi, &ps->part_dedr, &ps->part_drdpsi}) {
@@ -1876,6 +1887,57 @@ static hipError_t launch_fused_cycle(int prec, const MMKit &kf, const MMKit &ke,
   return err;
 }
 
+// Looks at the stop flags behind the launches of a minimization in parts, one group of cycles late:
+// the device runs the group last issued while the host waits for the one before, and the cycles of
+// a batch whose systems have all stopped are not issued.  A stopped cycle in parts is 14 launches
+// that return at once, 30 us (one block to a unit: 5 launches, 12 us): 24 systems of 400 atoms that
+// stop after 11-20 of 200 cycles take 3.7 ms, with all cycles issued 8.3, with one block 7.4.
+class StopWatch {
+ public:
+  ~StopWatch() {
+    for (hipEvent_t e : event) {
+      if (e != nullptr) {
+        (void)hipEventDestroy(e);
+      }
+    }
+  }
+  // Watches the flags of ps's synthesis; without a call nothing is watched.
+  hipError_t start(stormm_phasespace *ps, const int *flags, int systems) {
+    hipError_t err = hipSuccess;
+    for (int i = 0; i < 2 && err == hipSuccess; i++) {
+      err = hipEventCreateWithFlags(&event[i], hipEventDisableTiming);
+    }
+    running = ps->running;
+    done = flags;
+    nsys = systems;
+    return err;
+  }
+  // After a group was issued: sets *stopped when all systems had stopped by the end of the group
+  // before it.
+  hipError_t look(hipStream_t stream, bool *stopped) {
+    if (done == nullptr) {
+      return hipSuccess;
+    }
+    const int now = groups++ & 1;
+    hipError_t err = launch_any_running(done, nsys, running + now, stream);
+    if (err == hipSuccess) {
+      err = hipEventRecord(event[now], stream);
+    }
+    if (err == hipSuccess && groups > 1) {
+      err = hipEventSynchronize(event[1 - now]);
+      *stopped = (err == hipSuccess) &&
+                 *static_cast<volatile const int *>(running + (1 - now)) == 0;
+    }
+    return err;
+  }
+
+ private:
+  hipEvent_t event[2] = {nullptr, nullptr};
+  int *running = nullptr;
+  const int *done = nullptr;
+  int nsys = 0, groups = 0;
+};
+
 // Captures `cycles` fused cycles into an executable graph.
 static hipError_t capture_fused_cycle(int prec, const MMKit &kf, const MMKit &ke,
                                       const CycleKit &ck, int sd_cycles, int cycles,
@@ -1974,6 +2036,15 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
   if (err == hipSuccess && in_parts) {
     err = clear_part_sums(k, ag, stream);
   }
+  StopWatch watch;
+  bool stopped = false;
+  if (err == hipSuccess && in_parts && mc->convergence_rms_force > 0.0) {
+    err = watch.start(ps, cs.done, ns);
+  }
+  // After cycle c (and the ones before it) was issued.
+  auto look = [&](int c) {
+    return (c % kChunkCycles == kChunkCycles - 1) ? watch.look(stream, &stopped) : hipSuccess;
+  };
   if (how == FusedIssue::kCycleGraph) {
     if (err == hipSuccess) {
       err = capture_fused_cycle(prec, k, k, ck, sd, 1, cap, &graph[0], &exec[0]);
@@ -1981,16 +2052,22 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
     if (err == hipSuccess && cdcyc > 0) {
       err = capture_fused_cycle(prec, kf_clash, ke_clash, ck, sd, 1, cap, &graph[1], &exec[1]);
     }
-    for (int c = 0; c < mc->total_cycles && err == hipSuccess; c++) {
+    for (int c = 0; c < mc->total_cycles && !stopped && err == hipSuccess; c++) {
       err = hipGraphLaunch(exec[(c < cdcyc) ? 1 : 0], stream);
+      if (err == hipSuccess) {
+        err = look(c);
+      }
     }
   }
   else {
-    for (int c = 0; c < mc->total_cycles && err == hipSuccess; c++) {
+    for (int c = 0; c < mc->total_cycles && !stopped && err == hipSuccess; c++) {
       if (chunks > 0 && c == lead) {
         err = capture_fused_cycle(prec, k, k, ck, sd, kChunkCycles, cap, &graph[0], &exec[0]);
-        for (int g = 0; g < chunks && err == hipSuccess; g++) {
+        for (int g = 0; g < chunks && !stopped && err == hipSuccess; g++) {
           err = hipGraphLaunch(exec[0], stream);
+          if (err == hipSuccess) {
+            err = watch.look(stream, &stopped);
+          }
         }
         c += (chunks * kChunkCycles) - 1;
         continue;
@@ -1998,6 +2075,9 @@ static int minimize_fused(int32_t precision, const stormm_synthesis *ag,
       const bool damped = (c < cdcyc);
       err = launch_fused_cycle(prec, damped ? kf_clash : k, damped ? ke_clash : k, ck, sd,
                                stream);
+      if (err == hipSuccess) {
+        err = look(c);
+      }
     }
   }
   if (err == hipSuccess) {

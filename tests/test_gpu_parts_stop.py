@@ -84,3 +84,39 @@ def test_stopped_units_cost_next_to_nothing():
     assert cycles.max() == 0
     # Empty launches in place of evaluations of some ten microseconds each.
     assert stopped < 0.5 * running
+
+
+# Runs that stop early against the same units with one block each, which the caller gets by naming
+# their number: in every fused mode the cycles after the stop cost less than they do there.
+@pytest.mark.parametrize("mode", [1, 3, 4])
+def test_early_stop_is_no_slower_than_one_block(mode):
+    topos, coords = synthetic.generate([400] * 24, list(range(800, 824)), gb=True, perturb=0.05,
+                                       workers=1)
+
+    def run(shape):
+        ag = S.AtomGraphSynthesis(topos, shape)
+        ps = S.PhaseSpaceSynthesis(ag, 32, 23)
+        sc = S.ScoreCard(ag.system_count, 26)
+        lm = S.LineMinimization(ag.system_count, 0.01)
+        mc = S.minimize_controls(400, 50, 0.01, 6.0, clash_cycles=0, ntpr=7)
+        best = 1.0e9
+        for _ in range(3):
+            ps.upload(coords)
+            S.synchronize()
+            t0 = time.perf_counter()
+            S.launch_minimization("single", ag, ps, mc, sc, lm, persistent=mode)
+            S.synchronize()
+            best = min(best, time.perf_counter() - t0)
+        state = [sc.accumulators()] + [np.asarray(h) for h in sc.history()] + list(sc.series())
+        return ag.part_count, best, ps.fixed(), state, ag.minimization_status()
+
+    parts, t_parts, x, e, status = run(None)
+    none, t_one, x1, e1, status1 = run({"target_wu_per_cu": 2})
+    print(f"mode {mode}: {t_parts * 1e3:.2f} ms in parts, {t_one * 1e3:.2f} ms in one block")
+    assert parts > 0 and none == 0
+    assert status[0].max() < 100 and np.array_equal(status[0], status1[0])
+    assert np.array_equal(np.concatenate(x[0]), np.concatenate(x1[0]))
+    assert np.array_equal(np.concatenate(x[1]), np.concatenate(x1[1]))
+    for a, b in zip(e, e1):
+        assert np.array_equal(a, b)
+    assert t_parts < t_one
